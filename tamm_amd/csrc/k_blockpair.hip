@@ -10,9 +10,9 @@
 // multop.hpp:690-839).
 //
 // k_assign replaces kernels::assign / librett (assign.hpp:466-485, multiply.hpp:108-157):
-// dst(dl) (+)= scale * src(sl) for a label permutation, tiled 32x32 through LDS so both the
-// source read (along the source's contiguous mode) and the destination write (along the
-// destination's contiguous mode) are coalesced.
+// dst(dl) (+)= scale * src(sl) for a label permutation, in boxes of up to 2304 elements that
+// pass through LDS so both the source read (along the source's contiguous mode) and the
+// destination write (along the destination's contiguous mode) are coalesced.
 #include "tmx_device.hpp"
 #include "tmx_kernels.hpp"
 
@@ -244,72 +244,155 @@ void launch_bp_f64(const BPTask* tasks, int ntasks, const BPPair* pairs, const B
 }
 
 // ---------------------------------------------------------------------------
-// Block assign / transpose-accumulate.
+// Block assign / transpose-accumulate: HBM-bound (16 B per element, 24 when accumulating).
 //
-// Job j covers one (dst block, src block) pair and sh.tiles_o * sh.tiles_d * sh.tiles_s tiles.
-// d = dst's contiguous label, s = src's contiguous label, outer = the remaining labels.
-//   transpose case (d != s): a tile is 32 (along s) x 32 (along d); the source is read along s
-//     and the destination written along d, the 32x32 block passing through LDS.
-//   same case (d == s): both are contiguous along d; a tile is 1024 consecutive elements.
-__global__ __launch_bounds__(256) void k_assign(const AssignJob* __restrict__ jobs, int njobs,
-                                                const int64_t* __restrict__ tile_prefix,
+// A workgroup iteration takes one box of a (dst block, src block) pair (AssignShape).  The
+// offsets of the box's X, Y and Z indices go to LDS tables once; elements are read with X
+// fastest, then Y, then Z (the source's contiguous mode along the lanes), pass through an LDS
+// tile and are written with Y fastest, then X, then Z.  Without X modes both orders are the same
+// and the tile is skipped.  Each thread has its PER source loads and, accumulating, its PER
+// destination loads in flight together: 9 for whole boxes, 1 for the 256-element boxes of small
+// ops.  Boxes span as many modes as it takes to hold about 2304
+// elements: with one workgroup per 32x32 tile or per run of the contiguous mode, amplitude blocks
+// of 48x48x16x16 gave each workgroup 256 or 16 elements: over 3.5e7 elements, R(a,b,i,j) -=
+// T(b,a,i,j) went from 9.49 to 0.17 ms (5.0 TB/s) and R(a,b,i,j) -= T(a,b,j,i) from 0.93 to 0.17.
+struct AssignTable {
+  int s, d;
+};
+__device__ __forceinline__ uint32_t div_magic(uint32_t d) { return d > 1 ? 0xffffffffu / d + 1 : 0; }
+// e / d for e, d <= 4096 and m = div_magic(d).
+__device__ __forceinline__ uint32_t div_by(uint32_t e, uint32_t d, uint32_t m) {
+  return d > 1 ? __umulhi(e, m) : e;
+}
+
+template <int PER>
+__global__ __launch_bounds__(256) void k_assign(const AssignJob* __restrict__ jobs,
+                                                const AssignUnit* __restrict__ units, int64_t nunits,
                                                 const AssignShape* __restrict__ shapes,
                                                 const double* __restrict__ src,
                                                 double* __restrict__ dst, double scale,
                                                 int is_assign) {
-  __shared__ double tile[32][33];
-  const int64_t total = tile_prefix[njobs];
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-  for (int64_t t = blockIdx.x; t < total; t += gridDim.x) {
-    int lo = 0, hi = njobs - 1;
-    while (lo < hi) {
-      int mid = (lo + hi + 1) >> 1;
-      if (tile_prefix[mid] <= t) lo = mid; else hi = mid - 1;
-    }
-    const AssignJob jb = jobs[lo];
+  __shared__ double tile[kAssignLds];
+  __shared__ AssignTable tx[kAssignSide], ty[kAssignTable], tz[kAssignTable];
+  __shared__ int act[MAXR];
+  __shared__ int64_t first_s[MAXR], first_d[MAXR];
+  const int tid = threadIdx.x;
+  for (int64_t u = blockIdx.x; u < nunits; u += gridDim.x) {
+    const AssignUnit un = units[u];
+    const AssignJob jb = jobs[un.job];
     const AssignShape& sh = shapes[jb.shape];
-    int64_t local = t - tile_prefix[lo];
-    const int ts = (int)(local % sh.tiles_s);
-    local /= sh.tiles_s;
-    const int td = (int)(local % sh.tiles_d);
-    const int outer = (int)(local / sh.tiles_d);
-    const double* sp = src + jb.src_off + radix_off(sh.src_outer, outer);
-    double* dp = dst + jb.dst_off + radix_off(sh.dst_outer, outer);
-    if (sh.same) {
-      for (int e = threadIdx.x; e < 1024; e += 256) {
-        int d = td * 1024 + e;
-        if (d < sh.ed) {
-          double v = scale * sp[d];
-          dp[d] = is_assign ? v : dp[d] + v;
+    // the box's start and its extents (short at the end of a mode), a lane per mode
+    const int n_modes = sh.n, by = sh.nx, bz = sh.nx + sh.ny;
+    if (tid < MAXR) {
+      int a = 1, start = 0;
+      if (tid < n_modes) {
+        const uint32_t q = (uint32_t)un.tile / (uint32_t)sh.tdiv[tid], nt = (uint32_t)sh.nt[tid];
+        start = (int)(q % nt) * sh.box[tid];
+        a = min(sh.box[tid], sh.ext[tid] - start);
+      }
+      act[tid] = a;
+      first_s[tid] = tid < n_modes ? start * sh.sstr[tid] : 0;
+      first_d[tid] = tid < n_modes ? start * sh.dstr[tid] : 0;
+    }
+    __syncthreads();
+    int64_t sb = jb.src_off, db = jb.dst_off;
+    int X = 1, Y = 1, Z = 1;
+#pragma unroll
+    for (int k = 0; k < MAXR; ++k) {
+      sb += first_s[k];
+      db += first_d[k];
+      X *= k < by ? act[k] : 1;
+      Y *= k >= by && k < bz ? act[k] : 1;
+      Z *= k >= bz ? act[k] : 1;
+    }
+    // offsets of index i of the role with modes [b, e)
+    auto entry = [&](int b, int e, int i) {
+      AssignTable t{0, 0};
+      for (int k = e - 1; k >= b; --k) {
+        int dig = i;
+        if (k > b) {  // the slowest mode's digit is what is left
+          const uint32_t q = (uint32_t)i / (uint32_t)act[k];
+          dig = i - (int)q * act[k];
+          i = (int)q;
+        }
+        t.s += dig * (int)sh.sstr[k];
+        t.d += dig * (int)sh.dstr[k];
+      }
+      return t;
+    };
+    const int XY = X * Y, n = XY * Z;
+    for (int i = tid; i < X; i += 256) tx[i] = entry(0, by, i);
+    for (int i = tid; i < Y; i += 256) ty[i] = entry(by, bz, i);
+    for (int i = tid; i < Z; i += 256) tz[i] = entry(bz, n_modes, i);
+    const uint32_t mx = div_magic(X), my = div_magic(Y), mxy = div_magic(XY);
+    __syncthreads();
+    const double* sp = src + sb;
+    double* dp = dst + db;
+    double v[PER], old[PER];
+    int dof[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = tid + 256 * k;
+      v[k] = 0.0;
+      if (e < n) {
+        const int z = div_by(e, XY, mxy), r = e - z * XY, y = div_by(r, X, mx), x = r - y * X;
+        v[k] = sp[tx[x].s + ty[y].s + tz[z].s];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = tid + 256 * k;
+      old[k] = 0.0;
+      dof[k] = 0;
+      if (e < n) {
+        const int z = div_by(e, XY, mxy), r = e - z * XY, x = div_by(r, Y, my), y = r - x * Y;
+        dof[k] = tx[x].d + ty[y].d + tz[z].d;
+        if (!is_assign) old[k] = dp[dof[k]];
+      }
+    }
+    if (X > 1) {
+      const int ld = Y | 1;
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int e = tid + 256 * k;
+        if (e < n) {
+          const int z = div_by(e, XY, mxy), r = e - z * XY, y = div_by(r, X, mx), x = r - y * X;
+          tile[(z * X + x) * ld + y] = v[k];
         }
       }
-      continue;
-    }
-    __syncthreads();
-    for (int r = ty; r < 32; r += 8) {
-      int s_i = ts * 32 + tx, d_i = td * 32 + r;
-      tile[r][tx] = (s_i < sh.es && d_i < sh.ed)
-                        ? sp[(int64_t)s_i + (int64_t)d_i * sh.src_stride_d] : 0.0;
-    }
-    __syncthreads();
-    for (int r = ty; r < 32; r += 8) {
-      int d_i = td * 32 + tx, s_i = ts * 32 + r;
-      if (s_i < sh.es && d_i < sh.ed) {
-        double* q = dp + (int64_t)d_i + (int64_t)s_i * sh.dst_stride_s;
-        double v = scale * tile[tx][r];
-        *q = is_assign ? v : *q + v;
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        const int e = tid + 256 * k;
+        if (e < n) {
+          const int q = div_by(e, Y, my);  // z * X + x
+          v[k] = tile[q * ld + (e - q * Y)];
+        }
       }
     }
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = tid + 256 * k;
+      if (e < n) {
+        const double t = scale * v[k];
+        dp[dof[k]] = is_assign ? t : old[k] + t;
+      }
+    }
+    __syncthreads();  // the next box rewrites the tables and the tile
   }
 }
 
-void launch_assign(const AssignJob* jobs, int njobs, const int64_t* tile_prefix, int64_t ntiles,
+void launch_assign(const AssignJob* jobs, const AssignUnit* units, int64_t nunits, int box,
                    const AssignShape* shapes, const double* src, double* dst, double scale,
                    int is_assign, hipStream_t s) {
-  if (njobs <= 0 || ntiles <= 0) return;
-  int grid = (int)std::min<int64_t>(ntiles, 65536);
-  hipLaunchKernelGGL(k_assign, dim3(grid), dim3(256), 0, s, jobs, njobs, tile_prefix, shapes, src,
-                     dst, scale, is_assign);
+  if (nunits <= 0) return;
+  const int grid = (int)std::min<int64_t>(nunits, 65536);
+  if (box <= 256)
+    hipLaunchKernelGGL(k_assign<1>, dim3(grid), dim3(256), 0, s, jobs, units, nunits, shapes, src, dst,
+                       scale, is_assign);
+  else
+    hipLaunchKernelGGL(k_assign<kAssignElems / 256>, dim3(grid), dim3(256), 0, s, jobs, units, nunits,
+                       shapes, src, dst, scale, is_assign);
   TMX_HIP(hipGetLastError());
 }
 

@@ -1041,9 +1041,17 @@ struct BlockMulPlan {
   BPPlan bp;
 };
 struct AssignPlan {
-  DevBuf jobs, prefix, shapes;
-  int njobs = 0;
-  int64_t ntiles = 0;
+  DevBuf tables;  // shapes, jobs, units, zero_off and zero_prefix, in one upload
+  const AssignShape* shapes = nullptr;
+  const AssignJob* jobs = nullptr;
+  const AssignUnit* units = nullptr;
+  int64_t nunits = 0;
+  int box = 0;  // most elements of a unit
+  // Destination blocks whose source block is zero (element ranges; zero_prefix holds running
+  // lengths), zeroed when the op assigns.
+  const int64_t *zero_off = nullptr, *zero_prefix = nullptr;
+  int nzero = 0;
+  int64_t zero_elems = 0;
 };
 // Heap singletons, never destroyed (their device buffers must not be freed during static
 // destruction, see runtime.cpp).
@@ -1083,16 +1091,110 @@ LOperand single_block_operand(int n, const int64_t* dims, const int* labels) {
 
 namespace tmx {
 
-// Assign plan between two operands whose labels are a permutation of each other.
-std::unique_ptr<AssignPlan> build_assign_plan(const LOperand& D, const LOperand& S,
-                                              std::vector<std::pair<int64_t, int64_t>>* zero_blocks,
-                                              bool is_assign) {
+// Tile shape of a block permutation: dims of the destination block and the source stride of
+// each of its modes (see AssignShape).  Boxes hold up to `elems` elements.  X starts as the
+// source's contiguous mode and Y as the destination's; each side of fewer than 32 indices takes
+// in the next mode of its own block's order unless that mode is already on the other side (the
+// two sides together are then one contiguous piece of that block), so reads and writes come in
+// runs of at least 256 bytes wherever the blocks allow it.  Z then fills the box with the
+// remaining modes, the destination's fastest first.  A mode is cut into boxes of equal size.
+static AssignShape make_assign_shape(const std::vector<int64_t>& dd, const std::vector<int64_t>& src_stride,
+                                     int64_t elems) {
+  const int64_t side = elems >= kAssignElems ? kAssignSide : 16;
+  AssignShape sh;
+  std::memset(&sh, 0, sizeof(sh));
+  std::vector<int64_t> ext, ss;
+  for (size_t i = 0; i < dd.size(); ++i) {
+    TMX_REQUIRE(dd[i] < (1ll << 31), "block too large");
+    if (dd[i] == 1) continue;
+    if (!ext.empty() && ss.back() == src_stride[i] * dd[i] && ext.back() * dd[i] < (1ll << 31)) {
+      ext.back() *= dd[i];
+      ss.back() = src_stride[i];
+    } else {
+      ext.push_back(dd[i]);
+      ss.push_back(src_stride[i]);
+    }
+  }
+  const std::vector<int64_t> ds = strides_of(ext);
+  const int n = (int)ext.size();
+  TMX_REQUIRE(n <= MAXR, "too many modes in a block permutation");
+  sh.n = n;
+  if (n == 0) return sh;
+  std::vector<int64_t> box(n, 1);
+  std::vector<int> role(n, -1), X, Y, Z;  // fastest first
+  // Takes mode m into a side: in full when that keeps the side at `cap` (and offsets inside the
+  // box in 32 bits), else cut evenly.
+  int64_t span = (1ll << 31) - 1;  // largest offset the box may still add
+  auto take = [&](std::vector<int>& side, int r, int m, int64_t have, int64_t cap) {
+    const int64_t stride = std::max(ss[m], ds[m]);
+    const int64_t most = std::max<int64_t>(1, std::min(cap / have, 1 + span / stride));
+    const int64_t cuts = (ext[m] + most - 1) / most;
+    box[m] = (ext[m] + cuts - 1) / cuts;
+    span -= (box[m] - 1) * stride;
+    role[m] = r;
+    side.push_back(m);
+    return have * box[m];
+  };
+  std::vector<int> by_src(n);  // modes by source stride, fastest first
+  std::iota(by_src.begin(), by_src.end(), 0);
+  std::sort(by_src.begin(), by_src.end(), [&](int a, int b) { return ss[a] < ss[b]; });
+  const bool same = by_src[0] == n - 1;
+  int64_t nx = 1, ny = 1, nz = 1;
+  if (same) {
+    const int64_t run = std::min<int64_t>(kAssignTable, elems);
+    ny = take(Y, 1, n - 1, 1, run);
+    for (int m = n - 2; m >= 0 && ny < 64 && box[Y.back()] == ext[Y.back()]; --m) ny = take(Y, 1, m, ny, run);
+  } else {
+    nx = take(X, 0, by_src[0], 1, side);
+    ny = take(Y, 1, n - 1, 1, side);
+    for (int k = 1; k < n && nx < std::min<int64_t>(side, 32) && box[X.back()] == ext[X.back()] && role[by_src[k]] < 0; ++k)
+      nx = take(X, 0, by_src[k], nx, side);
+    for (int m = n - 2; m >= 0 && ny < std::min<int64_t>(side, 32) && box[Y.back()] == ext[Y.back()] && role[m] < 0; --m)
+      ny = take(Y, 1, m, ny, side);
+  }
+  const int64_t room = std::min<int64_t>(std::min<int64_t>(elems / (nx * ny), kAssignTable),
+                                         same ? kAssignTable : kAssignLds / (nx * (ny | 1)));
+  for (int m = n - 1; m >= 0; --m) {
+    if (role[m] >= 0) continue;
+    // a side's cut mode, or Z's own, ends the run: later modes stay outside the box
+    if (nz < room) nz = take(Z, 2, m, nz, room);
+    else {
+      Z.push_back(m);
+    }
+  }
+  sh.nx = (int)X.size();
+  sh.ny = (int)Y.size();
+  std::vector<int64_t> nt(n);
+  for (int i = 0; i < n; ++i) nt[i] = (ext[i] + box[i] - 1) / box[i];
+  const std::vector<int64_t> tdiv = strides_of(nt);
+  int k = 0;
+  for (const std::vector<int>* side : {&X, &Y, &Z})
+    for (size_t i = side->size(); i-- > 0; ++k) {
+      const int m = (*side)[i];
+      sh.ext[k] = (int)ext[m];
+      sh.box[k] = (int)box[m];
+      sh.nt[k] = (int)nt[m];
+      sh.tdiv[k] = (int)tdiv[m];
+      sh.sstr[k] = ss[m];
+      sh.dstr[k] = ds[m];
+    }
+  return sh;
+}
+
+// Assign plan between two operands whose labels are a permutation of each other; zeroing: lists
+// the destination blocks that have no source block.
+std::unique_ptr<AssignPlan> build_assign_plan(const LOperand& D, const LOperand& S, bool zeroing) {
   TMX_REQUIRE(D.labels.size() == S.labels.size(), "assign: label sets differ");
   for (int l : D.labels) TMX_REQUIRE(pos_of(S.labels, l) >= 0, "assign: labels are not a permutation");
+  // Box size: whole boxes once the destination makes 1024 of them (four workgroups per CU),
+  // else boxes of a workgroup's 256 threads, so that small ops spread over the chip (one
+  // 36x36x16x16 block: 7.9 us in 256-element boxes, 9.0 in whole ones).
+  const int64_t elems = D.t->total >= 1024 * kAssignElems ? kAssignElems : 256;
   std::vector<AssignJob> jobs;
+  std::vector<AssignUnit> units;
   std::vector<AssignShape> shapes;
   std::map<std::vector<int64_t>, int> sidx;
-  std::vector<int64_t> prefix{0};
+  std::vector<int64_t> zoff, zpre{0};
   const size_t r = D.labels.size();
   std::vector<int64_t> ext(r);
   for (size_t i = 0; i < r; ++i) ext[i] = D.ntl[i];
@@ -1106,53 +1208,35 @@ std::unique_ptr<AssignPlan> build_assign_plan(const LOperand& D, const LOperand&
       int64_t doff = D.t->find(db.data());
       int64_t soff = S.t->is_non_zero(sb.data()) ? S.t->find(sb.data()) : -1;
       std::vector<int64_t> dd(r), sd(r);
-      for (size_t i = 0; i < r; ++i) dd[i] = D.t->modes[i]->tsize(db[i]);
+      int64_t size = 1;
+      for (size_t i = 0; i < r; ++i) size *= dd[i] = D.t->modes[i]->tsize(db[i]);
       for (size_t i = 0; i < r; ++i) sd[i] = S.t->modes[i]->tsize(sb[i]);
       if (soff < 0) {
-        if (is_assign && zero_blocks) {
-          int64_t sz = 1;
-          for (auto x : dd) sz *= x;
-          zero_blocks->push_back({doff, sz});
+        if (zeroing && size > 0) {
+          zoff.push_back(doff);
+          zpre.push_back(zpre.back() + size);
         }
-      } else {
-        std::vector<int64_t> ds = strides_of(dd), ss = strides_of(sd);
-        AssignShape sh;
-        std::memset(&sh, 0, sizeof(sh));
-        int ld = r ? D.labels.back() : 0, ls = r ? S.labels.back() : 0;
-        std::vector<int64_t> oe, os, od;
-        int64_t ed = r ? dd.back() : 1, es = r ? sd.back() : 1;
-        sh.same = (r == 0 || ld == ls) ? 1 : 0;
-        for (size_t i = 0; i < r; ++i) {
-          int l = D.labels[i];
-          if (l == ld) continue;
-          if (!sh.same && l == ls) continue;
-          oe.push_back(dd[i]);
-          od.push_back(ds[i]);
-          os.push_back(ss[pos_of(S.labels, l)]);
+      } else if (size > 0) {
+        const std::vector<int64_t> ss = strides_of(sd);
+        std::vector<int64_t> key(dd), st(r);
+        for (size_t i = 0; i < r; ++i) st[i] = ss[pos_of(S.labels, D.labels[i])];
+        key.insert(key.end(), st.begin(), st.end());
+        auto f = sidx.find(key);
+        if (f == sidx.end()) {
+          f = sidx.emplace(key, (int)shapes.size()).first;
+          shapes.push_back(make_assign_shape(dd, st, elems));
         }
-        sh.ed = (int)ed;
-        sh.es = (int)es;
-        int64_t to = 1;
-        for (auto x : oe) to *= x;
-        sh.tiles_o = (int)to;
-        if (sh.same) {
-          sh.tiles_d = (int)((ed + 1023) / 1024);
-          sh.tiles_s = 1;
-        } else {
-          sh.tiles_d = (int)((ed + 31) / 32);
-          sh.tiles_s = (int)((es + 31) / 32);
-          sh.src_stride_d = ss[pos_of(S.labels, ld)];
-          sh.dst_stride_s = ds[pos_of(D.labels, ls)];
-        }
-        sh.src_outer = make_radix(oe, os);
-        sh.dst_outer = make_radix(oe, od);
+        const AssignShape& sh = shapes[f->second];
+        int64_t tiles = 1;
+        for (int i = 0; i < sh.n; ++i) tiles *= sh.nt[i];
+        TMX_REQUIRE(tiles < (1ll << 31), "block too large");
+        for (int64_t t = 0; t < tiles; ++t) units.push_back({(int32_t)jobs.size(), (int32_t)t});
         AssignJob jb;
         jb.src_off = soff;
         jb.dst_off = doff;
-        jb.shape = intern(shapes, sidx, sh);
+        jb.shape = f->second;
         jb.pad = 0;
         jobs.push_back(jb);
-        prefix.push_back(prefix.back() + (int64_t)sh.tiles_o * sh.tiles_d * sh.tiles_s);
       }
     }
     int d = (int)r - 1;
@@ -1163,11 +1247,25 @@ std::unique_ptr<AssignPlan> build_assign_plan(const LOperand& D, const LOperand&
     if (d < 0) break;
   }
   auto p = std::make_unique<AssignPlan>();
-  p->njobs = (int)jobs.size();
-  p->ntiles = prefix.back();
-  p->jobs = upload(jobs);
-  p->prefix = upload(prefix);
-  p->shapes = upload(shapes);
+  p->nunits = (int64_t)units.size();
+  p->box = (int)elems;
+  p->nzero = (int)zoff.size();
+  p->zero_elems = zpre.back();
+  std::vector<char> bytes;
+  auto put = [&](const auto& v) {  // offset of v's bytes, 8-byte aligned
+    const size_t at = (bytes.size() + 7) / 8 * 8, n = v.size() * sizeof(v[0]);
+    bytes.resize(at + n);
+    if (n) std::memcpy(bytes.data() + at, v.data(), n);
+    return at;
+  };
+  const size_t o_shapes = put(shapes), o_jobs = put(jobs), o_units = put(units), o_zoff = put(zoff), o_zpre = put(zpre);
+  p->tables = upload(bytes);
+  const char* base = p->tables.as<char>();
+  p->shapes = reinterpret_cast<const AssignShape*>(base + o_shapes);
+  p->jobs = reinterpret_cast<const AssignJob*>(base + o_jobs);
+  p->units = reinterpret_cast<const AssignUnit*>(base + o_units);
+  p->zero_off = reinterpret_cast<const int64_t*>(base + o_zoff);
+  p->zero_prefix = reinterpret_cast<const int64_t*>(base + o_zpre);
   return p;
 }
 
@@ -1178,7 +1276,6 @@ struct tmx_addop_s {
   double alpha = 1;
   int is_assign = 0;
   std::unique_ptr<AssignPlan> plan;
-  std::vector<std::pair<int64_t, int64_t>> zero_blocks;
   bool whole = false;  // identical labels and layouts over whole tensors: one streaming pass
 };
 
@@ -1254,12 +1351,11 @@ int tmx_block_assign(double* dst, int ndim, const int64_t* ddims, const int* dla
           int p = pos_of(S.labels, D.labels[i]);
           TMX_REQUIRE(p >= 0 && sdims[p] == ddims[i], "assign: dims do not match the permutation");
         }
-        it = g_as_cache.emplace(key, build_assign_plan(D, S, nullptr, false)).first;
+        it = g_as_cache.emplace(key, build_assign_plan(D, S, false)).first;
       }
       plan = it->second.get();
     }
-    launch_assign(plan->jobs.as<AssignJob>(), plan->njobs, plan->prefix.as<int64_t>(), plan->ntiles,
-                  plan->shapes.as<AssignShape>(), src, dst, scale, is_assign, s);
+    launch_assign(plan->jobs, plan->units, plan->nunits, plan->box, plan->shapes, src, dst, scale, is_assign, s);
   });
 }
 
@@ -1280,7 +1376,7 @@ int tmx_addop_create(const tmx_operand* C, double alpha, const tmx_operand* A, i
     LabelInfo li = analyse_labels(op->C, op->A, op->A);  // validates tilings of shared labels
     (void)li;
     op->whole = same_layout_whole(op->C, op->A);
-    if (!op->whole) op->plan = build_assign_plan(op->C, op->A, &op->zero_blocks, is_assign != 0);
+    if (!op->whole) op->plan = build_assign_plan(op->C, op->A, is_assign != 0);
     *out = addops().add(std::move(op));
   });
 }
@@ -1295,10 +1391,9 @@ int tmx_addop_execute(tmx_addop op, const double* A, double* C, void* stream) {
       else launch_axpy(op->C.t->total, op->alpha, A, C, s);
       return;
     }
-    for (auto& z : op->zero_blocks) launch_fill(C + z.first, z.second, 0.0, s);
-    launch_assign(op->plan->jobs.as<AssignJob>(), op->plan->njobs, op->plan->prefix.as<int64_t>(),
-                  op->plan->ntiles, op->plan->shapes.as<AssignShape>(), A, C, op->alpha,
-                  op->is_assign, s);
+    const AssignPlan& p = *op->plan;
+    launch_zero_ranges(p.zero_off, p.zero_prefix, p.nzero, p.zero_elems, C, s);
+    launch_assign(p.jobs, p.units, p.nunits, p.box, p.shapes, A, C, op->alpha, op->is_assign, s);
   });
 }
 

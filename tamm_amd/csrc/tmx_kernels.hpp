@@ -5,19 +5,27 @@
 
 namespace tmx {
 
-// Block assign (permutation) descriptors.
+// Block assign (permutation) descriptors.  Unit modes are dropped and modes that are neighbours
+// in both blocks merged; a tile is a box of box[k] indices of every mode.  The modes have three
+// roles and are listed by role, X's nx first, then Y's ny, then Z's, each slowest first: X holds
+// the source's contiguous mode, Y the destination's, Z the rest.  When both blocks share their
+// contiguous mode X is empty.  Offsets inside a box fit 32 bits.
 struct AssignShape {
-  int32_t same;       // 1 when dst and src share their contiguous label
-  int32_t ed, es;     // extents of the dst-contiguous (d) and src-contiguous (s) labels
-  int32_t tiles_o, tiles_d, tiles_s;
-  int64_t src_stride_d;  // src stride of label d (transpose case)
-  int64_t dst_stride_s;  // dst stride of label s (transpose case)
-  Radix src_outer, dst_outer;  // remaining labels -> src / dst offsets
+  int32_t n, nx, ny;
+  int32_t ext[MAXR], box[MAXR], nt[MAXR];  // extent, box extent and boxes of each mode
+  int32_t tdiv[MAXR];              // tile / tdiv % nt: the mode's box (tiles in destination order)
+  int64_t sstr[MAXR], dstr[MAXR];  // source and destination strides
 };
 struct AssignJob {
   int64_t src_off, dst_off;
   int32_t shape, pad;
 };
+struct AssignUnit {
+  int32_t job, tile;
+};
+// Limits of a tile: elements, LDS doubles of a staged tile (X * Z rows of Y | 1), entries of the
+// Y and Z offset tables, and of X and of Y when both are present.
+constexpr int kAssignElems = 2304, kAssignLds = 2560, kAssignTable = 512, kAssignSide = 48;
 
 // xr: XCD task ranges (null: the tasks split into 8 equal contiguous ranges).
 // C-tile shapes of the fused block-pair kernel (rows x columns of one task).
@@ -28,7 +36,8 @@ void launch_bp_f64(const BPTask* tasks, int ntasks, const BPPair* pairs, const B
                    const BPKShape* kshapes, const double* A, const double* B, double* C,
                    double alpha, int is_assign, hipStream_t s, const BPXcd* xr = nullptr,
                    int tile = BP_TILE_64x64);
-void launch_assign(const AssignJob* jobs, int njobs, const int64_t* tile_prefix, int64_t ntiles,
+// box: most elements of any unit.
+void launch_assign(const AssignJob* jobs, const AssignUnit* units, int64_t nunits, int box,
                    const AssignShape* shapes, const double* src, double* dst, double scale,
                    int is_assign, hipStream_t s);
 
