@@ -5,7 +5,10 @@ using namespace tmx;
 
 namespace {
 struct GenCache {
-  DevBuf blocks;
+  DevBuf tables;  // the blocks, then den_first
+  const GenBlock* blocks = nullptr;
+  // Block that each chunk of the denominator kernel starts in, and the last block (4-mode tensors).
+  const int32_t* den_first = nullptr;
   int64_t nblocks = 0, max_block = 0;
 };
 // Heap singletons, never destroyed (see runtime.cpp).
@@ -47,7 +50,22 @@ GenCache& gen_blocks(const Tensor& t) {
   auto c = std::make_unique<GenCache>();
   c->nblocks = (int64_t)v.size();
   c->max_block = mx;
-  c->blocks = upload(v);
+  std::vector<int32_t> first;
+  if (t.nmodes() == 4 && t.total > 0) {
+    const int chunk = denominator_chunk(t.total);
+    size_t b = 0;
+    for (int64_t c0 = 0; c0 < t.total; c0 += chunk) {
+      while (b + 1 < t.offs.size() && t.offs[b + 1] <= c0) ++b;
+      first.push_back((int32_t)b);
+    }
+    first.push_back((int32_t)t.offs.size() - 1);
+  }
+  std::vector<char> bytes(v.size() * sizeof(GenBlock) + first.size() * sizeof(int32_t));
+  if (!v.empty()) std::memcpy(bytes.data(), v.data(), v.size() * sizeof(GenBlock));
+  if (!first.empty()) std::memcpy(bytes.data() + v.size() * sizeof(GenBlock), first.data(), first.size() * sizeof(int32_t));
+  c->tables = upload(bytes);
+  c->blocks = c->tables.as<GenBlock>();
+  c->den_first = reinterpret_cast<const int32_t*>(c->blocks + v.size());
   auto& ref = *c;
   g_gen[t.uid] = std::move(c);
   return ref;
@@ -92,7 +110,7 @@ int tmx_fill_normal(tmx_tensor t, double* data, uint64_t seed, uint64_t tensor_i
     GenCache& gc = gen_blocks(tt);
     std::vector<int64_t> mode_n;
     for (int d = 0; d < tt.nmodes(); ++d) mode_n.push_back(tt.modes[d]->n);
-    launch_fill_normal(gc.blocks.as<GenBlock>(), gc.nblocks, tt.nmodes(), mode_n.data(), gc.max_block,
+    launch_fill_normal(gc.blocks, gc.nblocks, tt.nmodes(), mode_n.data(), gc.max_block,
                        data, seed, tensor_id, scale, symmetrize_pairs, s);
   });
 }
@@ -138,7 +156,7 @@ int tmx_energy_denominator(tmx_tensor R, double* data, const double* e_occ, cons
     TMX_REQUIRE(e_occ && e_vir, "null orbital energies");
     GenCache& gc = gen_blocks(tt);
     TMX_REQUIRE(gc.max_block < (int64_t(1) << 31), "denominator update: a block of 2^31 or more elements");
-    launch_denominator(gc.blocks.as<GenBlock>(), gc.nblocks, tt.total, data, e_occ, e_vir, s);
+    launch_denominator(gc.blocks, gc.den_first, tt.total, data, e_occ, e_vir, s);
   });
 }
 

@@ -157,6 +157,37 @@ int HostFlag::poll() {
   return __atomic_exchange_n(host, 0, __ATOMIC_ACQ_REL) != 0 ? 1 : 0;
 }
 
+namespace {
+constexpr int kResultSlots = 64;
+constexpr int kSlotDoubles = 16;  // 128 bytes apart
+struct ResultSlots {
+  std::mutex mu;
+  double *host = nullptr, *dev = nullptr;
+  std::vector<int> free;
+};
+// Never destroyed (see the pool above).
+ResultSlots& result_slots() {
+  static auto* r = new ResultSlots();
+  return *r;
+}
+}  // namespace
+
+ResultSlot::ResultSlot() {
+  ResultSlots& r = result_slots();
+  std::lock_guard<std::mutex> g(r.mu);
+  if (r.free.empty()) return;
+  host = r.host + r.free.back() * kSlotDoubles;
+  dev = r.dev + r.free.back() * kSlotDoubles;
+  r.free.pop_back();
+}
+
+ResultSlot::~ResultSlot() {
+  if (!host) return;
+  ResultSlots& r = result_slots();
+  std::lock_guard<std::mutex> g(r.mu);
+  r.free.push_back((int)((host - r.host) / kSlotDoubles));
+}
+
 void quiesce() {
   if (g_rt.initialised) (void)hipDeviceSynchronize();
 }
@@ -217,6 +248,15 @@ int tmx_init(int device, double pool_fraction) {
       g_pool.used.clear();
       g_pool.add_free(0, cap);
     }
+    {
+      ResultSlots& r = result_slots();
+      std::lock_guard<std::mutex> g(r.mu);
+      TMX_HIP(hipHostMalloc(reinterpret_cast<void**>(&r.host), sizeof(double) * kSlotDoubles * kResultSlots,
+                            hipHostMallocMapped | hipHostMallocCoherent));
+      TMX_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&r.dev), r.host, 0));
+      r.free.clear();
+      for (int i = 0; i < kResultSlots; ++i) r.free.push_back(i);
+    }
     noalloc_setup(device);  // device-side scratch of tmx_norm_noalloc, with `device` current
     g_rt.device = device;
     g_rt.initialised = true;
@@ -236,6 +276,13 @@ int tmx_finalize(void) {
       g_pool.free_by_off.clear();
       g_pool.free_by_size.clear();
       g_pool.used.clear();
+    }
+    {
+      ResultSlots& r = result_slots();
+      std::lock_guard<std::mutex> g(r.mu);
+      r.free.clear();
+      TMX_HIP(hipHostFree(r.host));
+      r.host = r.dev = nullptr;
     }
     g_rt.initialised = false;
     g_rt.stream = nullptr;

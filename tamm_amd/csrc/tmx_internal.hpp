@@ -118,6 +118,18 @@ struct HostFlag {
   int poll();
 };
 
+// A double in pinned host memory that a kernel writes and the host reads once the stream is
+// done: borrowed for one synchronous call from the 64 that tmx_init allocates (tmx_finalize
+// frees them).  host and dev are null when none is free.
+struct ResultSlot {
+  double* host = nullptr;
+  double* dev = nullptr;
+  ResultSlot();
+  ~ResultSlot();
+  ResultSlot(const ResultSlot&) = delete;
+  ResultSlot& operator=(const ResultSlot&) = delete;
+};
+
 // Copies a host vector to a fresh device buffer (plan time only).  Ordered on the engine
 // stream and completed before returning, so it never overtakes engine work still using
 // memory the pool has handed out again.

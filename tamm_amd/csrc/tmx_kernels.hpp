@@ -68,7 +68,10 @@ struct GenBlock {  // one block of a generated tensor
 void launch_fill_normal(const GenBlock* blocks, int64_t nblocks, int nmodes, const int64_t* mode_n,
                         int64_t max_block, double* data, uint64_t seed, uint64_t tensor_id,
                         double scale, int symmetrize, hipStream_t s);
-void launch_denominator(const GenBlock* blocks, int64_t nblocks, int64_t total, double* data,
+// first: for each chunk of denominator_chunk(total) elements the block it starts in, and one
+// more entry, the last block.
+int denominator_chunk(int64_t total);
+void launch_denominator(const GenBlock* blocks, const int32_t* first, int64_t total, double* data,
                         const double* e_occ, const double* e_vir, hipStream_t s);
 
 }  // namespace tmx
