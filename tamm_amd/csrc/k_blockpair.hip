@@ -212,8 +212,194 @@ __global__ __launch_bounds__(256, TM == 64 ? 4 : 3) void k_bp_f64(const BPTask* 
   }
 }
 
-int bp_tile_rows(int tile) { return tile == BP_TILE_16x256 ? 16 : 64; }
-int bp_tile_cols(int tile) { return tile == BP_TILE_16x256 ? 256 : 64; }
+// ---------------------------------------------------------------------------
+// Fused block-pair FP64 GEMM, the reduction split over the waves of a workgroup: for small
+// blocks, whose cost in k_bp_f64 is a chain of barriers and table loads per pair, and for
+// products with too few C tiles to fill the chip.  The NW waves of a workgroup share one
+// (16 FM) x (16 FN) C tile; the reduction is a stream of chunks of up to 64 indices of one block
+// pair, dealt round-robin to the waves.  A wave needs no barrier for a chunk: its 64 lanes put
+// the chunk's K offsets into the wave's own LDS row, and operands go straight from the TAMM
+// blocks into MFMA registers (lane l: row l%16, k l/16), the next G k-steps loading while G
+// multiply.  At the end the waves' partial tiles are summed through LDS, in wave order, and
+// written along C's contiguous direction.
+// Bound by the loads: a K-contiguous operand's load touches 16 rows x 32 B, about 43 cycles of a
+// CU's address pipe averaged over both operands, so larger tiles (fewer loads per MFMA) run
+// faster where there are enough of them: 16x16 / 32x32 / 64x64 at 14.6 / 29.7 / 45 TFLOP/s of
+// padded work on a dense 20 + 80 orbital ladder (k_bp_f64 37.6).  16-byte loads of two k per
+// lane, eight or sixteen waves per tile and deeper prefetch measured the same or slower.
+// 12 + 24 orbitals in blocks of ~6x6: ladder 112 -> 18 us, Fock terms 15-23 -> 6; one pair of
+// 36x36x36x36 and 36x36x16x16 blocks: 119 -> 55 us.
+constexpr int BP_KCH = 64;
+
+// G: k-steps (of 4) per group of loads.
+template <int FM, int FN, int NW, int G, int OCC>
+__global__ __launch_bounds__(64 * NW, OCC) void k_bp_ks(const BPTask* __restrict__ tasks, int ntasks,
+                                                        const BPPair* __restrict__ pairs,
+                                                        const BPCShape* __restrict__ cshapes,
+                                                        const BPKShape* __restrict__ kshapes,
+                                                        const double* __restrict__ A,
+                                                        const double* __restrict__ B,
+                                                        double* __restrict__ C, double alpha,
+                                                        int is_assign, BPXcd xr) {
+  constexpr int TM = 16 * FM, TN = 16 * FN, LD = TN + 1;
+  constexpr int NP = NW * TM * LD * 8 <= 36 * 1024 ? NW : 1;  // partial tiles in LDS
+  __shared__ double part[NP][TM * LD];
+  __shared__ uint32_t offK[NW][2][2][BP_KCH];  // byte offsets of a chunk's K indices in A and B
+  __shared__ int offCm[TM], offCn[TN];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lk = lane >> 4;
+  const int xcd = blockIdx.x & 7, per_xcd = gridDim.x >> 3;
+  for (int task_id = xr.lo[xcd] + (blockIdx.x >> 3); task_id < xr.hi[xcd]; task_id += per_xcd) {
+    const BPTask tk = tasks[task_id];
+    const BPCShape& cs = cshapes[tk.cshape];
+    const int M = cs.M, N = cs.N;
+    for (int t = tid; t < TM + TN; t += 64 * NW) {
+      if (t < TM) offCm[t] = tk.m0 + t < M ? radix_off(cs.cm, tk.m0 + t) : -1;
+      else offCn[t - TM] = tk.n0 + t - TM < N ? radix_off(cs.cn, tk.n0 + t - TM) : -1;
+    }
+    d4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+    int turn = wave;  // chunks until this wave's next one
+    for (int p = tk.pair_begin; p < tk.pair_end; ++p) {
+      const BPPair pr = pairs[p];
+      const int K = pr.K, nch = (K + BP_KCH - 1) / BP_KCH;
+      if (turn >= nch) {
+        turn -= nch;
+        continue;
+      }
+      const BPKShape& ks = kshapes[pr.kshape];
+      const char* Ab = reinterpret_cast<const char*>(A + pr.a_off);
+      const char* Bb = reinterpret_cast<const char*>(B + pr.b_off);
+      // rows beyond the block repeat its last one: their products land in C rows never written
+      uint32_t ra[FM], rb[FN];
+#pragma unroll
+      for (int i = 0; i < FM; ++i) ra[i] = 8u * (uint32_t)radix_off(ks.am, min(tk.m0 + 16 * i + l16, M - 1));
+#pragma unroll
+      for (int j = 0; j < FN; ++j) rb[j] = 8u * (uint32_t)radix_off(ks.bn, min(tk.n0 + 16 * j + l16, N - 1));
+      int tb = 0, klen = 0, g = 0;  // offset table in use, its chunk's length, group in the chunk
+      auto open_chunk = [&](int t) {
+        klen = min(BP_KCH, K - turn * BP_KCH);
+        const int kk = turn * BP_KCH + min(lane, klen - 1);
+        offK[wave][t][0][lane] = 8u * (uint32_t)radix_off(ks.ak, kk);
+        offK[wave][t][1][lane] = 8u * (uint32_t)radix_off(ks.bk, kk);
+        tb = t;
+        g = 0;
+        __builtin_amdgcn_wave_barrier();
+      };
+      double a[2][G][FM], b[2][G][FN];
+      auto load = [&](double (&av)[G][FM], double (&bv)[G][FN]) {
+#pragma unroll
+        for (int s = 0; s < G; ++s) {
+          const int k = 4 * (G * g + s) + lk;
+          const uint32_t oa = offK[wave][tb][0][k], ob = offK[wave][tb][1][k];
+#pragma unroll
+          for (int i = 0; i < FM; ++i) av[s][i] = *reinterpret_cast<const double*>(Ab + (ra[i] + oa));
+#pragma unroll
+          for (int j = 0; j < FN; ++j) bv[s][j] = *reinterpret_cast<const double*>(Bb + (rb[j] + ob));
+        }
+      };
+      // multiplies group gg of a chunk of length len
+      auto mul = [&](double (&av)[G][FM], double (&bv)[G][FN], int gg, int len) {
+#pragma unroll
+        for (int s = 0; s < G; ++s) {
+          const int k0 = 4 * (G * gg + s);
+          if (k0 >= len) break;
+          if (k0 + 4 > len) {  // beyond the chunk: zeros on both sides
+            const bool in = k0 + lk < len;
+#pragma unroll
+            for (int i = 0; i < FM; ++i) av[s][i] = in ? av[s][i] : 0.0;
+#pragma unroll
+            for (int j = 0; j < FN; ++j) bv[s][j] = in ? bv[s][j] : 0.0;
+          }
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s][i], bv[s][j], acc[i][j], 0, 0, 0);
+        }
+      };
+      // Steps to the next group of this wave's chunks of the pair and starts its loads; then the
+      // group before it is multiplied.
+      auto step = [&](double (&na)[G][FM], double (&nb)[G][FN], double (&ca)[G][FM], double (&cb)[G][FN]) {
+        const int cg = g, clen = klen;
+        bool more = true;
+        if ((g + 1) * 4 * G < klen) {
+          ++g;
+        } else {
+          turn += NW;
+          more = turn < nch;
+          if (more) open_chunk(tb ^ 1);
+        }
+        if (more) load(na, nb);
+        mul(ca, cb, cg, clen);
+        return more;
+      };
+      open_chunk(0);
+      load(a[0], b[0]);
+      while (step(a[1], b[1], a[0], b[0]) && step(a[0], b[0], a[1], b[1])) {
+      }
+      turn -= nch;
+    }
+    // partial tiles -> LDS; v_mfma_f64_16x16x4f64 result: register e of lane l holds row
+    // 4e + l/16, col l%16
+    auto put = [&](double* pw, bool add) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            double* q = pw + (16 * i + 4 * e + lk) * LD + 16 * j + l16;
+            *q = add ? *q + acc[i][j][e] : acc[i][j][e];
+          }
+    };
+    if constexpr (NP == NW) {
+      put(part[wave], false);
+    } else {
+      for (int w = 0; w + 1 < NW; ++w) {
+        if (wave == w) put(part[0], w > 0);
+        __syncthreads();
+      }
+      if (wave == NW - 1) put(part[0], true);
+    }
+    __syncthreads();
+    double* Cblk = C + tk.c_off;
+    constexpr int PER = TM * TN / (64 * NW), STEP = PER < 4 ? PER : 4;
+    static_assert(PER * 64 * NW == TM * TN && PER % STEP == 0, "tile not a whole number of passes");
+    for (int k0 = 0; k0 < PER; k0 += STEP) {
+      double old[STEP];
+      int off[STEP], at[STEP];
+#pragma unroll
+      for (int k = 0; k < STEP; ++k) {
+        const int e = tid + 64 * NW * (k0 + k);
+        const int row = cs.ncontig ? e / TN : e % TM, col = cs.ncontig ? e % TN : e / TM;
+        const int om = offCm[row], on = offCn[col];
+        off[k] = om >= 0 && on >= 0 ? om + on : -1;
+        at[k] = row * LD + col;
+        old[k] = !is_assign && off[k] >= 0 ? Cblk[off[k]] : 0.0;
+      }
+#pragma unroll
+      for (int k = 0; k < STEP; ++k) {
+        double v = 0.0;
+#pragma unroll
+        for (int w = 0; w < NP; ++w) v += part[w][at[k]];
+        if (off[k] >= 0) Cblk[off[k]] = is_assign ? alpha * v : old[k] + alpha * v;
+      }
+    }
+    __syncthreads();  // the next tile rewrites the partials and offsets
+  }
+}
+
+int bp_tile_rows(int tile) {
+  return tile == BP_TILE_16x256 || tile == BP_TILE_KS16 ? 16 : tile == BP_TILE_KS32 ? 32 : 64;
+}
+int bp_tile_cols(int tile) {
+  return tile == BP_TILE_16x256 ? 256 : tile == BP_TILE_KS16 ? 16 : tile == BP_TILE_KS32 ? 32 : 64;
+}
 
 void launch_bp_f64(const BPTask* tasks, int ntasks, const BPPair* pairs, const BPCShape* cshapes,
                    const BPKShape* kshapes, const double* A, const double* B, double* C,
@@ -234,12 +420,15 @@ void launch_bp_f64(const BPTask* tasks, int ntasks, const BPPair* pairs, const B
     longest = std::max(longest, r.hi[x] - r.lo[x]);
   }
   const int grid = 8 * std::min(longest, 65535);
-  if (tile == BP_TILE_16x256)
-    hipLaunchKernelGGL((k_bp_f64<16, 256, 1, 8>), dim3(grid), dim3(256), 0, s, tasks, ntasks, pairs,
-                       cshapes, kshapes, A, B, C, alpha, is_assign, r);
-  else
-    hipLaunchKernelGGL((k_bp_f64<64, 64, 2, 16>), dim3(grid), dim3(256), 0, s, tasks, ntasks, pairs,
-                       cshapes, kshapes, A, B, C, alpha, is_assign, r);
+#define TMX_BP_LAUNCH(KERNEL_, THREADS_)                                                              \
+  hipLaunchKernelGGL(KERNEL_, dim3(grid), dim3(THREADS_), 0, s, tasks, ntasks, pairs, cshapes, kshapes, \
+                     A, B, C, alpha, is_assign, r)
+  if (tile == BP_TILE_16x256) TMX_BP_LAUNCH((k_bp_f64<16, 256, 1, 8>), 256);
+  else if (tile == BP_TILE_KS16) TMX_BP_LAUNCH((k_bp_ks<1, 1, 4, 8, 4>), 256);
+  else if (tile == BP_TILE_KS32) TMX_BP_LAUNCH((k_bp_ks<2, 2, 4, 4, 4>), 256);
+  else if (tile == BP_TILE_KS64) TMX_BP_LAUNCH((k_bp_ks<4, 4, 4, 2, 2>), 256);
+  else TMX_BP_LAUNCH((k_bp_f64<64, 64, 2, 16>), 256);
+#undef TMX_BP_LAUNCH
   TMX_HIP(hipGetLastError());
 }
 

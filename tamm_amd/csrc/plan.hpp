@@ -50,7 +50,7 @@ std::vector<int64_t> strides_of(const std::vector<int64_t>& dims);
 struct BPPlan {
   DevBuf tasks, pairs, cshapes, kshapes;
   int ntasks = 0;
-  int tile = 0;          // BP_TILE_64x64 or BP_TILE_16x256
+  int tile = 0;          // C-tile shape (BP_TILE_*)
   bool swapped = false;  // built for C = B*A (the call's B is the kernel's A)
   BPXcd xcd{};  // cost-balanced XCD ranges of `tasks` (C blocks in key order, tiles in a row)
   std::vector<std::pair<int, int>> per_pair;  // task ranges, one launch per pair
@@ -67,7 +67,11 @@ struct BPPlan {
 // launch per block pair variant (TAMM's loop structure).
 void build_bp_plan(BPPlan& plan, const LOperand& C, const LOperand& A, const LOperand& B,
                    const LabelInfo& li, const std::vector<CBlockWork>& work,
-                   bool per_pair_launches, double* flops, int64_t* npairs);
+                   bool per_pair_launches, double* flops, int64_t* npairs, int shape = -1);
+// The C-tile shape the launch model chooses for the grouped launch (build_bp_plan's `shape`; -1
+// there: chosen inside), and its modelled duration.
+int grouped_bp_shape(const LOperand& C, const LOperand& A, const LOperand& B, const LabelInfo& li,
+                     const std::vector<CBlockWork>& work, double* us);
 // Launches tasks [0, ntasks) of `tasks` (the plan's own or its per-pair ranges) with the call's
 // operands (swapped plans take them in the order they were built for).
 void launch_bp_plan(const BPPlan& bp, const BPTask* tasks, int ntasks, const BPXcd* xr,

@@ -3,6 +3,7 @@
 #include <atomic>
 #include <cmath>
 #include <numeric>
+#include <unordered_map>
 
 #include "plan.hpp"
 
@@ -171,7 +172,24 @@ static void build_bp_plan_as(BPPlan& plan, const LOperand& C, const LOperand& A,
   std::vector<BPPair> pairs;
   std::vector<BPCShape> cshapes;
   std::vector<BPKShape> kshapes;
-  std::map<std::vector<int64_t>, int> cidx, kidx;
+  // Shapes by the tile sizes of the labels they depend on, each size as its index among the
+  // label's distinct ones: C's labels for a C shape, those and the reduction's for a K shape.
+  std::map<std::vector<int64_t>, int> cidx;
+  std::unordered_map<std::string, int> kidx;
+  auto size_ids = [&](int l) {
+    const std::vector<int64_t>& sz = li.tile_sizes.at(l);
+    std::vector<int64_t> distinct(sz);
+    std::sort(distinct.begin(), distinct.end());
+    distinct.erase(std::unique(distinct.begin(), distinct.end()), distinct.end());
+    std::vector<uint16_t> id;
+    for (int64_t x : sz)
+      id.push_back((uint16_t)(std::lower_bound(distinct.begin(), distinct.end(), x) - distinct.begin()));
+    TMX_REQUIRE(distinct.size() < 65536, "too many distinct tile sizes");
+    return id;
+  };
+  std::vector<std::vector<uint16_t>> c_ids, r_ids;
+  for (int l : C.labels) c_ids.push_back(size_ids(l));
+  for (int l : li.red) r_ids.push_back(size_ids(l));
   std::vector<BPTask> pair_tasks;
   double flops = 0;
   int64_t npairs = 0;
@@ -226,6 +244,7 @@ static void build_bp_plan_as(BPPlan& plan, const LOperand& C, const LOperand& A,
     else if (bk) to_back(kl, B.labels.back());
   }
 
+  std::vector<BPPair> pinfo;
   for (const CBlockWork& w : work) {
     if (w.pairs.empty()) continue;
     std::vector<int64_t> rt0(li.red.size(), 0);
@@ -242,27 +261,32 @@ static void build_bp_plan_as(BPPlan& plan, const LOperand& C, const LOperand& A,
     std::memset(&cs, 0, sizeof(cs));
     cs.M = (int)M;
     cs.N = (int)N;
+    cs.ncontig = !no.empty() && !C.labels.empty() && C.labels.back() == no.back() ? 1 : 0;
     cs.cm = make_radix(cext, cstr);
     cs.cn = make_radix(nce, ncs);
     int csid = intern(cshapes, cidx, cs);
 
     // Per pair: K shape and base offsets (batch element added below).
-    struct PInfo { BPPair p; std::vector<int64_t> abt, bbt; int64_t K; };
-    std::vector<PInfo> pinfo;
+    pinfo.clear();
+    std::string key((C.labels.size() + li.red.size()) * 2, '\0');
+    auto put = [&](size_t i, uint16_t v) { std::memcpy(&key[2 * i], &v, 2); };
+    for (size_t i = 0; i < C.labels.size(); ++i) put(i, c_ids[i][(size_t)w.ct[i]]);
     for (const PairRef& pr : w.pairs) {
-      std::vector<int64_t> at = tiles_for(A, w.ct, pr.rt), bt = tiles_for(B, w.ct, pr.rt);
-      BPKShape ks;
-      std::memset(&ks, 0, sizeof(ks));
-      std::vector<int64_t> e, s, e2, s2;
-      dims_of(A, at, mo, e, s);
-      ks.am = make_radix(e, s);
-      dims_of(B, bt, no, e, s);
-      ks.bn = make_radix(e, s);
-      // K radix: extents from whichever operand holds the label, strides 0 where absent.
-      std::vector<int64_t> kext, ka, kb;
-      {
-        std::vector<int64_t> ad = block_dims(A, at), as = strides_of(ad);
-        std::vector<int64_t> bd = block_dims(B, bt), bs = strides_of(bd);
+      for (size_t i = 0; i < li.red.size(); ++i) put(C.labels.size() + i, r_ids[i][(size_t)pr.rt[i]]);
+      auto it = kidx.find(key);
+      if (it == kidx.end()) {
+        const std::vector<int64_t> at = tiles_for(A, w.ct, pr.rt), bt = tiles_for(B, w.ct, pr.rt);
+        BPKShape ks;
+        std::memset(&ks, 0, sizeof(ks));
+        std::vector<int64_t> e, s;
+        dims_of(A, at, mo, e, s);
+        ks.am = make_radix(e, s);
+        dims_of(B, bt, no, e, s);
+        ks.bn = make_radix(e, s);
+        // K radix: extents from whichever operand holds the label, strides 0 where absent.
+        std::vector<int64_t> kext, ka, kb;
+        const std::vector<int64_t> ad = block_dims(A, at), as = strides_of(ad);
+        const std::vector<int64_t> bd = block_dims(B, bt), bs = strides_of(bd);
         for (int l : kl) {
           int pa = pos_of(A.labels, l), pb = pos_of(B.labels, l);
           kext.push_back(pa >= 0 ? ad[pa] : bd[pb]);
@@ -280,18 +304,17 @@ static void build_bp_plan_as(BPPlan& plan, const LOperand& C, const LOperand& A,
         // outer mode.
         ks.a_kcontig = (!kl.empty() && !A.labels.empty() && A.labels.back() == kl.back()) ? 1 : 0;
         ks.b_kcontig = (!kl.empty() && !B.labels.empty() && B.labels.back() == kl.back()) ? 1 : 0;
-        PInfo pi;
-        pi.p.a_off = pr.a_off;
-        pi.p.b_off = pr.b_off;
-        pi.p.kshape = intern(kshapes, kidx, ks);
-        pi.p.pad = 0;
-        pi.abt = at;
-        pi.bbt = bt;
-        pi.K = K;
-        pinfo.push_back(pi);
-        flops += 2.0 * (double)M * (double)N * (double)K * (double)Bn;
-        ++npairs;
+        it = kidx.emplace(key, (int)kshapes.size()).first;
+        kshapes.push_back(ks);
       }
+      BPPair p;
+      p.a_off = pr.a_off;
+      p.b_off = pr.b_off;
+      p.kshape = it->second;
+      p.K = kshapes[(size_t)it->second].K;
+      pinfo.push_back(p);
+      flops += 2.0 * (double)M * (double)N * (double)p.K * (double)Bn;
+      ++npairs;
     }
     // Batch elements: offsets of each batch index in C, A (per pair), B (per pair).
     std::vector<int64_t> bidx(li.batch.size(), 0);
@@ -304,15 +327,18 @@ static void build_bp_plan_as(BPPlan& plan, const LOperand& C, const LOperand& A,
       }
       int pbeg = (int)pairs.size();
       int64_t kcost = 0;
-      for (const PInfo& pi : pinfo) {
-        BPPair p = pi.p;
-        std::vector<int64_t> e, s;
-        dims_of(A, pi.abt, li.batch, e, s);
-        for (size_t i = 0; i < li.batch.size(); ++i) p.a_off += bidx[i] * s[i];
-        dims_of(B, pi.bbt, li.batch, e, s);
-        for (size_t i = 0; i < li.batch.size(); ++i) p.b_off += bidx[i] * s[i];
+      for (size_t q = 0; q < pinfo.size(); ++q) {
+        BPPair p = pinfo[q];
+        if (!li.batch.empty()) {
+          const std::vector<int64_t>& rt = w.pairs[q].rt;
+          std::vector<int64_t> e, s;
+          dims_of(A, tiles_for(A, w.ct, rt), li.batch, e, s);
+          for (size_t i = 0; i < li.batch.size(); ++i) p.a_off += bidx[i] * s[i];
+          dims_of(B, tiles_for(B, w.ct, rt), li.batch, e, s);
+          for (size_t i = 0; i < li.batch.size(); ++i) p.b_off += bidx[i] * s[i];
+        }
         pairs.push_back(p);
-        kcost += pi.K;
+        kcost += p.K;
       }
       int pend = (int)pairs.size();
       for (int64_t m0 = 0; m0 < M; m0 += TM)
@@ -400,51 +426,132 @@ static void build_bp_plan_as(BPPlan& plan, const LOperand& C, const LOperand& A,
   if (npairs_out) *npairs_out = npairs;
 }
 
-void build_bp_plan(BPPlan& plan, const LOperand& C, const LOperand& A, const LOperand& B,
-                   const LabelInfo& li, const std::vector<CBlockWork>& work,
-                   bool per_pair_launches, double* flops_out, int64_t* npairs_out) {
-  // Tile shape from the C blocks' row (A-outer) and column (B-outer) extents: the MFMA work
-  // each shape pads to, weighted by the blocks' reduction lengths.  The 16x256 tile pays off
-  // when one side is a single small tile (one-body terms, their adjoints); the plan then
-  // puts that side on the rows, swapping A and B when it is the column side.
-  double w64 = 0, w_rows = 0, w_cols = 0;
-  auto pad = [](double x, double t) { return std::ceil(x / t) * t; };
+namespace {
+// Launch model of the fused block-pair kernels, one entry per C-tile shape: the launch takes the
+// longest of its padded work at the shape's full-chip rate (over whole rounds of one workgroup
+// per CU), its serial chains spread over the chip's workgroup slots, and its longest chain.  A
+// chain is a task's fixed time and, for each of its block pairs, a start and a time per `unit`
+// reduction indices.  Fitted to launches of 5 us to 5 ms (blocks of 1 to 1600 rows, 1 to 50
+// pairs, K of 2 to 6400): e.g. a 12 + 24 orbital ladder in blocks of ~6x6, 64x64 112 us, 32x32
+// 28, 16x16 16; a 20 + 80 orbital dense ladder 1250 / 1472 / 2517, split 64x64 1047; a Fock
+// term over blocks of 37 x 2600 with K = 37 340 / 421 / 495 / 610; the adjoint dV += L T of 25 +
+// 110 orbitals (K ~ 40 a pair) 908 / 1398 / 2474 / 1354.
+struct BpShape {
+  int tile, slots;
+  bool swapped;
+  double rate;                  // padded flops per second
+  double fixed, pair, per_unit;  // us
+  int unit, waves;              // the chain's pair and unit times are shared by `waves`
+};
+constexpr BpShape kBpShapes[] = {
+    {BP_TILE_64x64, 1024, false, 37.6e12, 12.5, 2.5, 1.45, 16, 1},
+    {BP_TILE_16x256, 768, false, 23.4e12, 14.0, 2.5, 1.45, 8, 1},
+    {BP_TILE_16x256, 768, true, 23.4e12, 14.0, 2.5, 1.45, 8, 1},
+    {BP_TILE_KS16, 1280, false, 14.6e12, 4.0, 0.0, 2.0, 64, 4},
+    {BP_TILE_KS32, 1024, false, 29.7e12, 8.0, 0.0, 2.5, 64, 4},
+    {BP_TILE_KS64, 512, false, 52e12, 30.0, 0.0, 9.5, 64, 4},
+};
+
+struct BpLaunch {  // running sums of one launch
+  double flops = 0, tasks = 0, chains = 0, longest = 0;
+  double us(const BpShape& sh) const {
+    if (tasks == 0) return 0;
+    const double rounds = std::ceil(tasks / 256.0) * 256.0 / tasks;
+    return std::max({flops / sh.rate * 1e6 * rounds, chains / sh.slots, longest});
+  }
+};
+}  // namespace
+
+// The fastest C-tile shape by the launch model (index into kBpShapes) and its modelled time.
+static int choose_bp_shape(const LOperand& C, const LOperand& A, const LOperand& B,
+                           const LabelInfo& li, const std::vector<CBlockWork>& work,
+                           bool per_pair_launches, double* us_out) {
+  constexpr int NS = sizeof(kBpShapes) / sizeof(BpShape);
+  BpLaunch all[NS];
+  double total[NS] = {};
+  int64_t largest = 1;  // operand block
+  for (const LOperand* o : {&A, &B})
+    for (int64_t sz : o->t->sizes) largest = std::max(largest, sz);
+  std::vector<const std::vector<int64_t>*> red_sizes;
+  for (int l : li.red) red_sizes.push_back(&li.tile_sizes.at(l));
+  std::vector<int64_t> ks;
   for (const CBlockWork& w : work) {
     if (w.pairs.empty()) continue;
     const std::vector<int64_t> cd = block_dims(C, w.ct);
-    double M = 1, N = 1, Bn = 1, K = 0;
+    double M = 1, N = 1, Bn = 1;
     for (size_t i = 0; i < C.labels.size(); ++i) {
       const int l = C.labels[i];
       if (pos_of(li.aouter, l) >= 0) M *= (double)cd[i];
       else if (pos_of(li.bouter, l) >= 0) N *= (double)cd[i];
       else Bn *= (double)cd[i];
     }
+    // K of every pair, and sums over the pairs of its k-steps of 4 and units of 8, 16 and 64
+    ks.clear();
+    double kpad = 0, u8 = 0, u16 = 0, u64 = 0;
     for (const PairRef& pr : w.pairs) {
-      double k = 1;
-      for (size_t i = 0; i < li.red.size(); ++i) k *= (double)li.tile_sizes.at(li.red[i])[pr.rt[i]];
-      K += k;
+      int64_t k = 1;
+      for (size_t i = 0; i < li.red.size(); ++i) k *= red_sizes[i]->at((size_t)pr.rt[i]);
+      kpad += (double)((k + 3) / 4 * 4);
+      u8 += (double)((k + 7) / 8);
+      u16 += (double)((k + 15) / 16);
+      u64 += (double)((k + 63) / 64);
+      if (per_pair_launches) ks.push_back(k);
     }
-    w64 += pad(M, 64) * pad(N, 64) * K * Bn;
-    w_rows += pad(M, 16) * pad(N, 256) * K * Bn;
-    w_cols += pad(N, 16) * pad(M, 256) * K * Bn;
+    for (int s = 0; s < NS; ++s) {
+      const BpShape& sh = kBpShapes[s];
+      const double tm = bp_tile_rows(sh.tile), tn = bp_tile_cols(sh.tile);
+      const double m = sh.swapped ? N : M, n = sh.swapped ? M : N;
+      const double tiles = std::ceil(m / tm) * std::ceil(n / tn) * Bn;
+      for (int64_t k : ks) {
+        BpLaunch one;
+        one.tasks = tiles;
+        one.flops = 2 * tiles * tm * tn * (double)((k + 3) / 4 * 4);
+        one.longest = sh.fixed + (sh.pair + sh.per_unit * (double)((k + sh.unit - 1) / sh.unit)) / sh.waves;
+        one.chains = tiles * one.longest;
+        total[s] += one.us(sh);
+      }
+      const double units = sh.unit == 8 ? u8 : sh.unit == 16 ? u16 : u64;
+      const double chain = sh.fixed + (sh.pair * (double)w.pairs.size() + sh.per_unit * units) / sh.waves;
+      all[s].flops += 2 * tiles * tm * tn * kpad;
+      all[s].tasks += tiles;
+      all[s].chains += tiles * chain;
+      all[s].longest = std::max(all[s].longest, chain);
+    }
   }
-  // The 16x256 tile reads (16 + 256) / (16 * 256) operand elements per MFMA product against
-  // 2 / 64 for 64x64: taken only when it saves a third of the padded work or more.
-  if (std::min(w_rows, w_cols) * 1.5 < w64) {
-    if (w_cols < w_rows) {
-      const LabelInfo li2 = analyse_labels(C, B, A);
-      const std::vector<CBlockWork> work2 = enumerate_pairs(C, B, A, li2);
-      build_bp_plan_as(plan, C, B, A, li2, work2, per_pair_launches, flops_out, npairs_out,
-                       BP_TILE_16x256);
-      plan.swapped = true;
-      return;
+  int best = 0;
+  double best_us = -1;
+  for (int s = 0; s < NS; ++s) {
+    const BpShape& sh = kBpShapes[s];
+    if (sh.waves > 1 && largest > kBpKsMaxBlock) continue;
+    const double us = per_pair_launches ? total[s] : all[s].us(sh);
+    if (best_us < 0 || us < best_us) {
+      best = s;
+      best_us = us;
     }
-    build_bp_plan_as(plan, C, A, B, li, work, per_pair_launches, flops_out, npairs_out,
-                     BP_TILE_16x256);
+  }
+  if (us_out) *us_out = std::max(best_us, 0.0);
+  return best;
+}
+
+void build_bp_plan(BPPlan& plan, const LOperand& C, const LOperand& A, const LOperand& B,
+                   const LabelInfo& li, const std::vector<CBlockWork>& work,
+                   bool per_pair_launches, double* flops_out, int64_t* npairs_out, int shape) {
+  const int best = shape >= 0 ? shape : choose_bp_shape(C, A, B, li, work, per_pair_launches, nullptr);
+  if (kBpShapes[best].swapped) {
+    const LabelInfo li2 = analyse_labels(C, B, A);
+    const std::vector<CBlockWork> work2 = enumerate_pairs(C, B, A, li2);
+    build_bp_plan_as(plan, C, B, A, li2, work2, per_pair_launches, flops_out, npairs_out,
+                     kBpShapes[best].tile);
+    plan.swapped = true;
     return;
   }
   build_bp_plan_as(plan, C, A, B, li, work, per_pair_launches, flops_out, npairs_out,
-                   BP_TILE_64x64);
+                   kBpShapes[best].tile);
+}
+
+int grouped_bp_shape(const LOperand& C, const LOperand& A, const LOperand& B, const LabelInfo& li,
+                     const std::vector<CBlockWork>& work, double* us) {
+  return choose_bp_shape(C, A, B, li, work, false, us);
 }
 
 void launch_bp_plan(const BPPlan& bp, const BPTask* tasks, int ntasks, const BPXcd* xr,
@@ -676,7 +783,7 @@ int tmx_contraction_create(const tmx_operand* C, double alpha, const tmx_operand
                 "output tensor also appears on the right-hand side (MultOp::validate)");
     LabelInfo li = analyse_labels(c->C, c->A, c->B);
     std::vector<CBlockWork> work = enumerate_pairs(c->C, c->A, c->B, li);
-    int mode = exec_mode;
+    int mode = exec_mode, bp_shape = -1;
     if (mode == TMX_EXEC_AUTO || mode == TMX_EXEC_AUTO_SPLIT) {
       // Average reduction length per output element: below kMinSectorK the contraction is
       // memory-bound, and the sector path's operand repacking and dense intermediate cost more
@@ -695,7 +802,31 @@ int tmx_contraction_create(const tmx_operand* C, double alpha, const tmx_operand
       }
       const double avg_k = celems > 0 ? fl / (2.0 * celems) : 0.0;
       constexpr double kMinSectorK = 128;
-      const bool sector = sector_eligible(li) && avg_k >= kMinSectorK;
+      bool sector = sector_eligible(li) && avg_k >= kMinSectorK;
+      // Small products: the sector path's launches, packs of blocks of a few hundred elements and
+      // few-tile GEMMs over a long K cost more than the block-pair kernel.  Its time here: four
+      // launches of 4.5 us (nine on the split path), packs and scatter at 3 TB/s or 6 us a block
+      // over 1024 workgroups, and the GEMM at its rate or its serial stages (split-K parts are
+      // at least 1024 columns), e.g. 16 + 64 orbitals: ladder 85 us grouped, 182 sector, 79 split;
+      // ring 22 / 105 / 58.  Grouped is taken when modelled twice as fast, or three times on the
+      // split path: a level computes the product of such a ring's four permutations once there
+      // (at 1.5 times, residuals of 30 + 120 orbitals with irreps took 573 us against 534).
+      // Larger products stay on the sector path, whose packed operands a constant operand keeps;
+      // so do streaming ones (few flops over large tensors), which the model does not cover.
+      constexpr double kSmallFlops = 20e9, kSmallElems = 4e7;
+      const double elems = (double)(c->A.t->total + c->B.t->total + c->C.t->total);
+      if (sector && fl < kSmallFlops && elems < kSmallElems) {
+        const bool split = exec_mode == TMX_EXEC_AUTO_SPLIT;
+        double us = 4.5 * (split ? 9 : 4);
+        for (const LOperand* o : {&c->A, &c->B, &c->C}) {
+          const double bytes = (double)o->t->total * (o == &c->C ? (split ? 27 : 24) : (split ? 27 : 16));
+          us += std::max(bytes / 3e6, 6.0 * (double)o->t->keys.size() / 1024.0);
+        }
+        us += split ? std::max(fl / 120e6, avg_k / 64.0) : std::max(fl / 50e6, 0.9 * std::min(avg_k, 1024.0) / 8.0);
+        double grouped_us = 0;
+        bp_shape = grouped_bp_shape(c->C, c->A, c->B, li, work, &grouped_us);
+        if ((split ? 3.0 : 2.0) * grouped_us < us) sector = false;
+      }
       mode = !sector ? TMX_EXEC_GROUPED_F64
                      : (exec_mode == TMX_EXEC_AUTO_SPLIT ? TMX_EXEC_SPLIT_I8 : TMX_EXEC_SECTOR_F64);
     }
@@ -743,7 +874,7 @@ int tmx_contraction_create(const tmx_operand* C, double alpha, const tmx_operand
       c->npairs = np;
     } else {
       build_bp_plan(c->bp, c->C, c->A, c->B, li, work, mode == TMX_EXEC_BLOCKPAIR_F64, &c->flops,
-                    &c->npairs);
+                    &c->npairs, bp_shape);
     }
     c->mode = mode;
     *out = contractions().add(std::move(c));

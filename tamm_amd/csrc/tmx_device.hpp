@@ -5,16 +5,32 @@
 
 namespace tmx {
 
+// n / d and n % d: in FP32 with one correction step where both are below 2^22 (float(n), float(d)
+// are exact and the estimate is within one of the quotient), else as integers.
+__device__ __forceinline__ int div_rem(int n, int d, int& rem) {
+  int q;
+  if ((n | d) < (1 << 22)) {
+    q = (int)((float)n * __builtin_amdgcn_rcpf((float)d));
+    int r = n - q * d;
+    if (r < 0) { --q; r += d; }
+    else if (r >= d) { ++q; r -= d; }
+    rem = r;
+  } else {
+    q = n / d;
+    rem = n - q * d;
+  }
+  return q;
+}
+
 // Mixed-radix offset of a row-major index.
 __device__ __forceinline__ int radix_off(const Radix& r, int idx) {
   int off = 0;
-  for (int d = r.n - 1; d >= 0; --d) {
-    int e = r.ext[d];
-    int q = idx / e;
-    off += (idx - q * e) * r.stride[d];
-    idx = q;
+  for (int d = r.n - 1; d > 0; --d) {
+    int digit;
+    idx = div_rem(idx, r.ext[d], digit);
+    off += digit * r.stride[d];
   }
-  return off;
+  return r.n > 0 ? off + idx * r.stride[0] : 0;  // idx is the slowest mode's digit
 }
 
 // Incremental mixed-radix counter over consecutive indices.

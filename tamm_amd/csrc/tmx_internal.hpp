@@ -219,12 +219,14 @@ struct BPTask {
 };
 struct BPCShape {
   int32_t M, N;
+  int32_t ncontig;  // 1 when the C block is contiguous along N
+  int32_t pad;
   Radix cm, cn;  // C strides of the M (aouter) and N (bouter) modes
 };
 struct BPPair {
   int64_t a_off, b_off;
   int32_t kshape;
-  int32_t pad;
+  int32_t K;  // reduction length of the pair (its K shape's)
 };
 // Task ranges per XCD: workgroups are dispatched round-robin over the 8 XCDs, and workgroup b
 // works through tasks [lo[b % 8], hi[b % 8]) so that neighbouring tiles, which read the same

@@ -28,8 +28,11 @@ struct AssignUnit {
 constexpr int kAssignElems = 2304, kAssignLds = 2560, kAssignTable = 512, kAssignSide = 48;
 
 // xr: XCD task ranges (null: the tasks split into 8 equal contiguous ranges).
-// C-tile shapes of the fused block-pair kernel (rows x columns of one task).
-enum { BP_TILE_64x64 = 0, BP_TILE_16x256 = 1 };
+// C-tile shapes of the fused block-pair kernels (rows x columns of one task): 64x64 and 16x256 of
+// k_bp_f64 (operands staged in LDS), 16x16, 32x32 and 64x64 of k_bp_ks (the reduction split over
+// a workgroup's waves; blocks of at most kBpKsMaxBlock elements).
+enum { BP_TILE_64x64 = 0, BP_TILE_16x256 = 1, BP_TILE_KS16 = 2, BP_TILE_KS32 = 3, BP_TILE_KS64 = 4 };
+constexpr int64_t kBpKsMaxBlock = int64_t(1) << 29;  // byte offsets inside a block in 32 bits
 int bp_tile_rows(int tile);
 int bp_tile_cols(int tile);
 void launch_bp_f64(const BPTask* tasks, int ntasks, const BPPair* pairs, const BPCShape* cshapes,
