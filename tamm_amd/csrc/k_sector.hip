@@ -11,7 +11,6 @@
 #include <fstream>
 #include <map>
 #include <mutex>
-#include <queue>
 #include <tuple>
 
 #include "sector.hpp"
@@ -1342,11 +1341,19 @@ __global__ __launch_bounds__(256) void k_scatter(const ScatterJob* __restrict__ 
 // can time faster alone yet slow the plan down as a launch of its own.  FP64 32x32 serves
 // classes of one O tile (16 padded rows, e.g. that product's 8 x 8 sectors), which a 64-row
 // tile would load four times over.
-struct I8Shape { int tm, tn; double eff; int small; };
-static const I8Shape kF64Shapes[] = {{128, 128, 1.0, 0}, {128, 160, 1.0, 0}, {64, 64, 0.5, 64}, {32, 32, 0.25, 32}};
-static const I8Shape kI8Shapes[] = {{256, 256, 1.0, 0}, {512, 160, 1.0, 0}, {256, 160, 0.95, 0},
-                                    {256, 128, 0.82, 0}, {128, 256, 0.82, 0}, {128, 128, 0.6, 0},
-                                    {64, 64, 0.3, 64}};
+// eff: MFMA efficiency for comparing shapes on one sector by padded area.  rate, fixed and
+// slots describe the shape in the launch model: multiply-adds per second of the full chip
+// (10^15 int8, 3.4 x 10^13 FP64), time per task outside its stages (pipeline fill and epilogue)
+// in us, and tasks that run at once per CU at that rate.  Fitted to GEMM stages of 30 us to 15 ms
+// (O = 20..60, V = 80..320: K of 256 to 28800, 20 to 53856 tasks), rms 6-10%.  An FP64 task
+// alone on a CU runs as fast as two sharing it, hence one slot.
+struct I8Shape { int tm, tn; double eff; int small; double rate, fixed; int slots; };
+static const I8Shape kF64Shapes[] = {{128, 128, 1.0, 0, 1.0, 8, 1}, {128, 160, 1.0, 0, 1.0, 8, 1},
+                                     {64, 64, 0.5, 64, 0.5, 4, 1}, {32, 32, 0.25, 32, 0.25, 4, 1}};
+static const I8Shape kI8Shapes[] = {{256, 256, 1.0, 0, 1.35, 8, 1}, {512, 160, 1.0, 0, 1.25, 8, 1},
+                                    {256, 160, 0.95, 0, 1.20, 6, 2}, {256, 128, 0.82, 0, 1.25, 6, 2},
+                                    {128, 256, 0.82, 0, 1.20, 6, 2}, {128, 128, 0.6, 0, 1.0, 4, 2},
+                                    {64, 64, 0.3, 64, 0.3, 4, 2}};
 static bool shape_allowed(const I8Shape& sh, int64_t mrows, int64_t nrows) {
   return sh.small == 0 || std::min(mrows, nrows) <= sh.small;
 }
@@ -1407,15 +1414,18 @@ static void cost_model_tile(const I8Shape (&shapes)[N], int64_t mrows, int64_t n
   }
 }
 
-void choose_tile(bool split, int nmod, int64_t mrows, int64_t nrows, int64_t klen, int* tm, int* tn) {
+// Tile shape of one sector: the autotuner's recorded choice for its geometry (returns true), else
+// the least padded area over efficiency.
+static bool choose_tile(bool split, int nmod, int64_t mrows, int64_t nrows, int64_t klen, int* tm, int* tn) {
   {
     std::lock_guard<std::mutex> g(tune_mu());
     tune_load_locked();
     auto it = tune_map().find(TuneKey{split ? 1 : 0, nmod, mrows, nrows, klen});
-    if (it != tune_map().end()) { *tm = it->second.tm; *tn = it->second.tn; return; }
+    if (it != tune_map().end()) { *tm = it->second.tm; *tn = it->second.tn; return true; }
   }
   if (split) cost_model_tile(kI8Shapes, mrows, nrows, tm, tn);
   else cost_model_tile(kF64Shapes, mrows, nrows, tm, tn);
+  return false;
 }
 
 // ---------------------------------------------------------------------------
@@ -1471,80 +1481,96 @@ static int gemm_wg_per_cu(bool split, int tm, int tn) {
   return nb;
 }
 
-static double shape_eff(bool split, int tm, int tn) {
+static const I8Shape& shape_of(bool split, int tm, int tn) {
   for (const I8Shape& sh : kI8Shapes)
-    if (split && sh.tm == tm && sh.tn == tn) return sh.eff;
+    if (split && sh.tm == tm && sh.tn == tn) return sh;
   for (const I8Shape& sh : kF64Shapes)
-    if (!split && sh.tm == tm && sh.tn == tn) return sh.eff;
-  return 1.0;
+    if (!split && sh.tm == tm && sh.tn == tn) return sh;
+  throw Error(TMX_ERR_INVALID, "no GEMM kernel for the requested tile shape");
 }
 
-// Modelled duration of one task: its multiply-adds (plus a pipeline fill and epilogue worth a
-// few k-steps) at one workgroup slot's share of the kernel's sustained rate.
-static double task_seconds(bool split, int tm, int tn, int64_t klen, int wgpc) {
-  const double macs = (double)tm * tn * (double)(klen + (split ? 256 : 128)) / shape_eff(split, tm, tn);
+// Two launch models.  Part counts: a task's multiply-adds (plus a pipeline fill and epilogue worth
+// a few k-steps) at one workgroup slot's share of the kernel's sustained rate, on the slots its
+// occupancy allows.  Shapes: the fitted rates and times of the shape table.
+enum class Model { kParts, kShapes };
+static double task_seconds(Model model, bool split, const I8Shape& sh, int64_t klen, int slots) {
+  if (model == Model::kShapes)
+    return (double)sh.tm * sh.tn * (double)klen / ((split ? 1.0e15 : 3.4e13) * sh.rate / (256.0 * slots)) +
+           sh.fixed * 1e-6;
+  const double macs = (double)sh.tm * sh.tn * (double)(klen + (split ? 256 : 128)) / sh.eff;
   const double chip = split ? 1.0e15 : 3.4e13;  // sustained multiply-adds per second
-  return macs / (chip / (256.0 * wgpc));
+  return macs / (chip / (256.0 * slots));
 }
 
-// Lays out one launch's tasks (given in panel order) for the XCD mapping when `out` is non-null,
-// and returns the simulated makespan in seconds.
-static double layout_launch(bool split, int tm, int tn, const std::vector<SecTask>& tasks,
-                            const std::vector<int64_t>& klens, std::vector<SecTask>* out) {
-  constexpr int kXcds = 8, kCusPerXcd = 32;
-  const int wgpc = gemm_wg_per_cu(split, tm, tn);
-  struct Group { size_t b, e; double cost, each; };
-  std::vector<Group> groups;
+// Tasks [b, e) of one M panel (of one plane): `each` seconds apiece.
+struct TaskGroup {
+  size_t b, e;
+  double each;
+  double cost() const { return each * (double)(e - b); }
+};
+constexpr int kXcds = 8, kCusPerXcd = 32;
+
+// Deals the groups, longest first, to the least loaded XCD; bins (when given) receives each XCD's
+// groups in that order.  Returns the list schedule's makespan with `slots` tasks at once per CU.
+static double deal_groups(std::vector<TaskGroup>& groups, int slots,
+                          std::vector<std::vector<const TaskGroup*>>* bins_out) {
+  std::stable_sort(groups.begin(), groups.end(),
+                   [](const TaskGroup& x, const TaskGroup& y) { return x.cost() > y.cost(); });
+  std::vector<std::vector<const TaskGroup*>> bins(kXcds);
+  std::vector<double> load(kXcds, 0.0);
+  for (const TaskGroup& g : groups) {
+    const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    bins[x].push_back(&g);
+    load[x] += g.cost();
+  }
+  double makespan = 0;
+  for (int x = 0; x < kXcds; ++x) {
+    std::map<double, size_t> free_at{{0.0, (size_t)(kCusPerXcd * slots)}};  // time -> slots
+    for (const TaskGroup* g : bins[x])
+      for (size_t left = g->e - g->b; left > 0;) {
+        const auto it = free_at.begin();
+        const size_t n = std::min(it->second, left);
+        const double f = it->first + g->each;
+        if ((it->second -= n) == 0) free_at.erase(it);
+        free_at[f] += n;
+        left -= n;
+        makespan = std::max(makespan, f);
+      }
+  }
+  if (bins_out) *bins_out = std::move(bins);
+  return makespan;
+}
+
+// Lays out one launch's tasks (given in panel order) for the XCD mapping.
+static void layout_launch(bool split, int tm, int tn, const std::vector<SecTask>& tasks,
+                          const std::vector<int64_t>& klens, std::vector<SecTask>* out) {
+  const I8Shape& shape = shape_of(split, tm, tn);
+  const int slots = gemm_wg_per_cu(split, tm, tn);
+  std::vector<TaskGroup> groups;
   for (size_t i = 0; i < tasks.size();) {
     size_t j = i;
     while (j < tasks.size() && tasks[j].c_base == tasks[i].c_base && tasks[j].m0 == tasks[i].m0 &&
            tasks[j].plane == tasks[i].plane)
       ++j;
-    const double each = task_seconds(split, tm, tn, klens[i], wgpc);
-    groups.push_back({i, j, each * (double)(j - i), each});
+    groups.push_back({i, j, task_seconds(Model::kParts, split, shape, klens[i], slots)});
     i = j;
   }
-  std::stable_sort(groups.begin(), groups.end(),
-                   [](const Group& x, const Group& y) { return x.cost > y.cost; });
-  std::vector<std::vector<const Group*>> bins(kXcds);
-  std::vector<double> load(kXcds, 0.0);
-  for (const Group& g : groups) {
-    const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-    bins[x].push_back(&g);
-    load[x] += g.cost;
+  std::vector<std::vector<const TaskGroup*>> bins;
+  deal_groups(groups, slots, &bins);
+  size_t per = 0;
+  for (const auto& b : bins) {
+    size_t n = 0;
+    for (const TaskGroup* g : b) n += g->e - g->b;
+    per = std::max(per, n);
   }
-  double makespan = 0;
-  const int slots = kCusPerXcd * wgpc;
+  SecTask empty;
+  std::memset(&empty, 0, sizeof(empty));
+  out->assign(per * kXcds, empty);
   for (int x = 0; x < kXcds; ++x) {
-    std::priority_queue<double, std::vector<double>, std::greater<double>> free_at;
-    for (int k = 0; k < slots; ++k) free_at.push(0.0);
-    double end = 0;
-    for (const Group* g : bins[x])
-      for (size_t t = g->b; t < g->e; ++t) {
-        const double f = free_at.top() + g->each;
-        free_at.pop();
-        free_at.push(f);
-        end = std::max(end, f);
-      }
-    makespan = std::max(makespan, end);
+    size_t i = per * x;
+    for (const TaskGroup* g : bins[x])
+      for (size_t t = g->b; t < g->e; ++t) (*out)[i++] = tasks[t];
   }
-  if (out) {
-    size_t per = 0;
-    for (const auto& b : bins) {
-      size_t n = 0;
-      for (const Group* g : b) n += g->e - g->b;
-      per = std::max(per, n);
-    }
-    SecTask empty;
-    std::memset(&empty, 0, sizeof(empty));
-    out->assign(per * kXcds, empty);
-    for (int x = 0; x < kXcds; ++x) {
-      size_t i = per * x;
-      for (const Group* g : bins[x])
-        for (size_t t = g->b; t < g->e; ++t) (*out)[i++] = tasks[t];
-    }
-  }
-  return makespan;
 }
 
 // Tasks of every sector in panel order (split path: plane-major, one copy per residue plane),
@@ -1579,15 +1605,68 @@ static void tasks_by_shape(const std::vector<SectorGeom>& geoms, int planes,
   }
 }
 
-double estimate_sector_seconds(bool split, int nmod, const std::vector<SectorGeom>& geoms) {
-  std::map<int, std::pair<std::vector<SecTask>, std::vector<int64_t>>> by;
-  tasks_by_shape(geoms, split ? std::max(nmod, 1) : 1, by, nullptr);
+// Duration of the launches of these sectors, one per tile shape, by the layout of their tasks.
+static double simulate_launches(bool split, int nmod, const std::vector<SectorGeom>& geoms, Model model) {
+  std::map<std::pair<int, int>, std::vector<TaskGroup>> by;
+  for (int pl = 0; pl < (split ? std::max(nmod, 1) : 1); ++pl)
+    for (const SectorGeom& g : geoms) {
+      const I8Shape& sh = shape_of(split, g.tm, g.tn);
+      const int slots = model == Model::kShapes ? sh.slots : gemm_wg_per_cu(split, g.tm, g.tn);
+      const double each = task_seconds(model, split, sh, g.klen, slots);
+      const size_t n = (size_t)((g.nrows + g.tn - 1) / g.tn);
+      std::vector<TaskGroup>& v = by[{g.tm, g.tn}];
+      for (int64_t m0 = 0; m0 < g.mrows; m0 += g.tm) v.push_back({0, n, each});
+    }
   double t = 0;
-  for (auto& kv : by)
-    t += layout_launch(split, kv.first / 1000, kv.first % 1000, kv.second.first, kv.second.second, nullptr);
+  for (auto& kv : by) {
+    const int slots = model == Model::kShapes ? shape_of(split, kv.first.first, kv.first.second).slots
+                                              : gemm_wg_per_cu(split, kv.first.first, kv.first.second);
+    t += deal_groups(kv.second, slots, nullptr) + (model == Model::kShapes ? 4e-6 : 0.0);
+  }
   return t;
 }
 
+double estimate_sector_seconds(bool split, int nmod, const std::vector<SectorGeom>& geoms) {
+  return simulate_launches(split, nmod, geoms, Model::kParts);
+}
+
+// Sectors of different shapes are launches of their own, each with a last partial round and the
+// small sectors' launch too short to fill the chip; the launch model therefore also tries every
+// shape for all sectors at once (thin ones keep the narrow shapes made for them).  Ladder, ring
+// and hole-hole GEMMs of O = 30, V = 180 in split precision: 1774 -> 1543, 351 -> 292 and 128 ->
+// 97 us; FP64 ring 1155 -> 820.
+void choose_shapes(bool split, int nmod, std::vector<SectorGeom>& geoms, bool trial) {
+  const I8Shape* shapes = split ? kI8Shapes : kF64Shapes;
+  const size_t n = split ? std::size(kI8Shapes) : std::size(kF64Shapes);
+  std::vector<size_t> wide;
+  bool tuned = false;
+  for (size_t i = 0; i < geoms.size(); ++i) {
+    SectorGeom& g = geoms[i];
+    tuned |= choose_tile(split, nmod, g.mrows_pad, g.nrows_pad, g.klen, &g.tm, &g.tn);
+    for (size_t k = 0; k < n; ++k)
+      if (shapes[k].tm == g.tm && shapes[k].tn == g.tn && shapes[k].small == 0) wide.push_back(i);
+  }
+  if (trial || tuned || wide.empty()) return;
+  std::vector<std::pair<int, int>> best;
+  double best_t = -1;
+  for (int k = -1; k < (int)n; ++k) {  // -1: the choices sector by sector
+    if (k >= 0 && shapes[k].small > 0) continue;
+    if (k >= 0)
+      for (size_t i : wide) {
+        geoms[i].tm = shapes[k].tm;
+        geoms[i].tn = shapes[k].tn;
+      }
+    const double t = simulate_launches(split, nmod, geoms, Model::kShapes);
+    if (best_t >= 0 && t >= best_t) continue;
+    best_t = t;
+    best.clear();
+    for (size_t i : wide) best.emplace_back(geoms[i].tm, geoms[i].tn);
+  }
+  for (size_t i = 0; i < wide.size(); ++i) {
+    geoms[wide[i]].tm = best[i].first;
+    geoms[wide[i]].tn = best[i].second;
+  }
+}
 // XCD-aware task lists of a plan, one per tile shape.
 void build_sector_tasks(SectorPlan& sp) {
   std::map<int, std::pair<std::vector<SecTask>, std::vector<int64_t>>> by;

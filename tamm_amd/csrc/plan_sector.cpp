@@ -481,7 +481,7 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
     while (n < kMaxModuli && have < need) have += std::log2((double)kModuli[n++]);
     return have < need ? -1 : n;
   };
-  auto make_geoms = [&](const Parts& P, int nmod) {
+  auto make_geoms = [&](const Parts& P, int nmod, bool trial) {
     std::vector<SectorGeom> geoms;
     for (const Sector& s2 : P.secs) {
       const ClassMat& am = AM[s2.mc];
@@ -500,9 +500,9 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
       g.mrows = (int32_t)am.rows;
       g.nrows = (int32_t)bm.rows;
       g.klen = s2.klen;
-      choose_tile(split, nmod, g.mrows_pad, g.nrows_pad, g.klen, &g.tm, &g.tn);
       geoms.push_back(g);
     }
+    choose_shapes(split, nmod, geoms, trial);
     return geoms;
   };
   // Parallel split: part counts per pair.  A fixed count applies to every pair; otherwise the
@@ -515,7 +515,7 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
     const int nm = split ? moduli_for(E.kmax) : 0;
     if (split && nm < 0) return 1e30;
     const double bytes_per_elem = split ? 2.0 * nm + 16.0 : 16.0;
-    return estimate_sector_seconds(split, nm, make_geoms(E, nm)) +
+    return estimate_sector_seconds(split, nm, make_geoms(E, nm, true)) +
            (double)E.extra_elems * bytes_per_elem / kScratchBytesPerSecond;
   };
   std::vector<int64_t> nparts(cpairs.size(), 1);
@@ -564,7 +564,7 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
   sp->c_total = cbase;
   sp->kmax = kmax;
   sp->split_factor = P.nrounds;
-  sp->geoms = make_geoms(P, split ? std::max(moduli_for(kmax), 0) : 0);
+  sp->geoms = make_geoms(P, split ? std::max(moduli_for(kmax), 0) : 0, false);
   sp->ksegs = upload(segs);
   for (const SectorGeom& g : sp->geoms) {
     const int64_t f[] = {g.a_base, g.b_base, g.c_base, g.seg_b, g.seg_e, g.a_kpad, g.b_kpad,

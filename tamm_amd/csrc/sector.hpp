@@ -155,9 +155,10 @@ struct SectorPlan {
   double mn_intensity = 0;
 };
 
-// Tile shape (rows of A x rows of B per workgroup) for a sector GEMM: the autotuner's
-// recorded choice for this geometry if there is one, else the cost model.
-void choose_tile(bool split, int nmod, int64_t mrows, int64_t nrows, int64_t klen, int* tm, int* tn);
+// Tile shapes (rows of A x rows of B per workgroup) of a plan's sector GEMMs: the autotuner's
+// recorded choices for the geometries if there are any, else by the launch model.  trial: sector
+// by sector only (part counts that are costed, not built).
+void choose_shapes(bool split, int nmod, std::vector<SectorGeom>& geoms, bool trial);
 // Builds the GEMM task lists of all sectors from their geometry and tile shapes, one launch
 // per shape, each laid out for the XCD-aware workgroup mapping (balanced XCD ranges, longest
 // tasks first, padded with empty tasks), and the plan's executed-flop count.
