@@ -32,11 +32,12 @@ namespace tmx {
 
 namespace {
 
-// Every K block is padded to a multiple of KGRAN columns (an int8 or FP64 MFMA fragment
-// width); on the split path to KGRAN_SPLIT, so a GEMM stage of two 32-column k-steps never
-// straddles two K segments.
-constexpr int KGRAN = 32;
-constexpr int KGRAN_SPLIT = 64;
+// Columns of a K block are padded to KBLOCK (the pack's 16-byte residue groups; an FP64 MFMA
+// k-step), and only the last block of a K class to KSTAGE, the columns of a GEMM stage: a stage
+// never straddles two K segments, which are whole K classes.  Padding every block to a stage (64
+// int8 columns) added 6% to the ladder GEMM of 36 + 18 orbital tiles and 12% to one of 20 x 20.
+constexpr int KBLOCK_F64 = 4, KSTAGE_F64 = 8;
+constexpr int KBLOCK_SPLIT = 16, KSTAGE_SPLIT = 64;
 // Longest split-K part of a split-precision sector: keeps the int32 residue sums exact
 // (K * 128 * 128 < 2^31 needs K <= 131071) and the modulus count at 11 for 35-bit operands.
 constexpr int64_t kSplitKPart = 32768;
@@ -275,8 +276,13 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
     sp->split = false;
   }
   std::vector<int64_t> kpadlen(nK);
-  const int64_t kgran = split ? KGRAN_SPLIT : KGRAN;
-  for (size_t k = 0; k < nK; ++k) kpadlen[k] = roundup(tuple_size(KL, kt[k], li), kgran);
+  const int64_t kstage = split ? KSTAGE_SPLIT : KSTAGE_F64;
+  std::vector<int64_t> classlen(kcidx.size(), 0);  // columns of each K class
+  for (size_t k = 0; k < nK; ++k) {
+    kpadlen[k] = roundup(tuple_size(KL, kt[k], li), split ? KBLOCK_SPLIT : KBLOCK_F64);
+    classlen[kcls[k]] += kpadlen[k];
+  }
+  for (int64_t& n : classlen) n = roundup(n, kstage);
 
   // Class matrices (rows, padded columns, per-K-block column offsets).
   struct ClassMat {
@@ -290,10 +296,16 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
     cm.assign(rep.size(), ClassMat());
     for (size_t c = 0; c < rep.size(); ++c) {
       cm[c].col.assign(nK, -1);
+      int cls_of_off = -1;
       int64_t off = 0;
       for (size_t k : korder)
-        if (rep[c][k]) { cm[c].col[k] = off; off += kpadlen[k]; }
-      cm[c].kpad = off;
+        if (rep[c][k]) {
+          if (off % kstage != 0 && kcls[k] != cls_of_off) off = roundup(off, kstage);
+          cls_of_off = kcls[k];
+          cm[c].col[k] = off;
+          off += kpadlen[k];
+        }
+      cm[c].kpad = roundup(off, kstage);
     }
     rowoff.assign(rt.size(), -1);
     for (size_t r = 0; r < rt.size(); ++r) {
@@ -405,14 +417,19 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
   // region (rows_pad(A) x rows_pad(B), a whole number of 32x32 tiles) and is scattered into C in
   // its own round.
   struct Sector { int mc, nc; int64_t c_base; int seg_b, seg_e; int64_t klen; int round; };
-  struct Pair { int mc, nc; std::vector<KSeg> segs; int64_t klen; };
+  // cutlen: the K blocks' columns, each padded to 64 (split) or 32: bounds the part count.
+  struct Pair { int mc, nc; std::vector<KSeg> segs; int64_t klen, cutlen; };
   std::vector<Pair> cpairs;
   for (int a = 0; a < nMC; ++a)
     for (int b = 0; b < nNC; ++b) {
-      Pair pr{a, b, {}, 0};
+      Pair pr{a, b, {}, 0, 0};
+      int prev = -1;  // the blocks of a K class are in both class matrices or in neither
       for (size_t k : korder) {
         if (AM[a].col[k] < 0 || BM[b].col[k] < 0) continue;
-        KSeg g{(int32_t)AM[a].col[k], (int32_t)BM[b].col[k], (int32_t)kpadlen[k], 0};
+        pr.cutlen += roundup(tuple_size(KL, kt[k], li), split ? 64 : 32);
+        if (kcls[k] == prev) continue;
+        prev = kcls[k];
+        KSeg g{(int32_t)AM[a].col[k], (int32_t)BM[b].col[k], (int32_t)classlen[prev], 0};
         pr.klen += g.len;
         if (!pr.segs.empty()) {
           KSeg& last = pr.segs.back();
@@ -436,7 +453,7 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
   std::vector<int64_t> min_parts(cpairs.size()), max_parts(cpairs.size());
   for (size_t i = 0; i < cpairs.size(); ++i) {
     min_parts[i] = split ? (cpairs[i].klen + kSplitKPart - 1) / kSplitKPart : 1;
-    max_parts[i] = std::max(min_parts[i], std::min<int64_t>(kMaxParts, cpairs[i].klen / kMinPartK));
+    max_parts[i] = std::max(min_parts[i], std::min<int64_t>(kMaxParts, cpairs[i].cutlen / kMinPartK));
   }
   auto make_parts = [&](const std::vector<int64_t>& nparts) {
     Parts P;
@@ -444,7 +461,7 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
       const Pair& pr = cpairs[i];
       const int64_t mr = AM[pr.mc].rows_pad, nr = BM[pr.nc].rows_pad;
       const int64_t parts = std::min(std::max(nparts[i], min_parts[i]), max_parts[i]);
-      const int64_t target = roundup((pr.klen + parts - 1) / parts, kgran);
+      const int64_t target = roundup((pr.klen + parts - 1) / parts, kstage);
       int round = 0;
       Sector cur{pr.mc, pr.nc, 0, (int)P.segs.size(), 0, 0, 0};
       auto close = [&]() {
