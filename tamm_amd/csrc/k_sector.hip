@@ -586,6 +586,41 @@ struct StageCursor {
   }
 };
 
+// Cursor of a task that reads A in place (InPlaceA): the K stream of StageCursor<8, 8>, with A's
+// position as a K block of its class and a stage inside it (K blocks are padded to stages, so a
+// stage lies in one block).  Past the end it stays on the last stage.
+struct InPlaceCursor {
+  const KSeg* segs;
+  const int2* kblk;  // first column and columns of the class's K blocks
+  int seg, last, j, len, b;
+  int kb, ja, cols;
+  __device__ __forceinline__ void open(int sg) {
+    seg = sg;
+    j = 0;
+    const KSeg k = segs[sg];
+    len = (int)((uint32_t)k.len >> 3);
+    b = (int)((uint32_t)k.b_col >> 3);
+    kb = k.a_blk;
+    const int2 kk = kblk[kb];
+    cols = kk.y;
+    ja = (int)((uint32_t)(k.a_col - kk.x) >> 3);
+  }
+  __device__ __forceinline__ int unit_b() const { return b + j; }
+  // True when A moved to another K block.
+  __device__ __forceinline__ bool advance() {
+    if (j + 1 < len) {
+      ++j;
+      if (++ja * 8 < cols) return false;
+      cols = kblk[++kb].y;
+      ja = 0;
+      return true;
+    }
+    if (seg >= last) return false;
+    open(seg + 1);
+    return true;
+  }
+};
+
 // FP64 sector GEMM: workgroup tile TM x TN over 4 waves (2x2), each (TM/2) x (TN/2) =
 // (TM/32) x (TN/32) v_mfma_f64_16x16x4f64 tiles (128x128 and 128x160 instantiated; the
 // 16-column granularity lets 160 cover N = 800 exactly).  The fragment-major class matrices
@@ -597,23 +632,33 @@ struct StageCursor {
 // stage (spares read the zero fragment into a scratch slot), so the vmcnt thresholds are
 // constants.  Fragment reads are double-buffered in registers: the next k-step's reads go out
 // right after the first MFMA of the current one.  Two workgroups share a CU.
-template <int TM, int TN, int NS>
+// INP: A is read from the tensor's blocks instead of a packed copy (InPlaceA): lane 4r + c of an A
+// load takes 16 bytes, columns 2p and 2p + 1 (p = (c - r/2) mod 4) of row r's run, so four lanes
+// read 64 contiguous bytes and the LDS reads of a fragment (one 8-byte half of every lane's 16)
+// spread over the banks.  MFMA lane group g then holds columns 2g and 2g + 1 in the two k-steps,
+// of A and, by another read address, of the packed B.  Columns past a block's end read a zero.
+// The pass that copied A (8 B read and written per element, V(a,b,c,d) the largest tensor of
+// all) is gone, and the GEMM, whose loads are 64-byte pieces of rows now instead of whole KB,
+// loses 4 to 8 %: pack + GEMM of the pp ladder at O=30, V=180 1506 + 4760 -> 0 + 4942 us (61 TF),
+// of 20 + 80 orbitals 149 + 648 -> 0 + 701 us.
+template <int TM, int TN, int NS, bool INP = false>
 __global__ __launch_bounds__(256, 2) void k_gemm_f64(const SecTask* __restrict__ tasks, int ntasks,
                                                      const KSeg* __restrict__ segs,
                                                      const double* __restrict__ Ap,
                                                      const double* __restrict__ Bp,
-                                                     double* __restrict__ Cd) {
+                                                     double* __restrict__ Cd, InPlaceA ip) {
   constexpr int AF = TM / 16, BF = TN / 16, SF = AF + BF;  // 1 KB units per stage
   constexpr int FPW = (SF + 3) / 4;
   constexpr int SLOT = SF;
   constexpr int WTM = TM / 32, WTN = TN / 32;
   static_assert(WTM * 32 == TM && WTN * 32 == TN, "tile must split over 2x2 waves");
   __shared__ i4 lds[NS][SLOT * 64];
+  __shared__ int64_t ip_tab[INP ? kInPlaceTable : 1];  // block offsets of the tile's row blocks
   const int task = xcd_task(ntasks);
   if (task >= ntasks) return;
   const SecTask tk = tasks[task];
   if (tk.mrows == 0) return;  // padding of the XCD layout
-  const uint8_t* A = reinterpret_cast<const uint8_t*>(Ap + tk.a_base);
+  const uint8_t* A = reinterpret_cast<const uint8_t*>(Ap + (INP ? 0 : tk.a_base));
   const uint8_t* B = reinterpret_cast<const uint8_t*>(Bp + tk.b_base);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wv = __builtin_amdgcn_readfirstlane(wave);
@@ -623,8 +668,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64(const SecTask* __restrict__
   const int rt0 = tk.m0 >> 4, ct0 = tk.n0 >> 4;
   int nst = 0;
   for (int sg = tk.kseg_begin; sg < tk.kseg_end; ++sg) nst += (int)((uint32_t)segs[sg].len >> 3);
-  StageCursor<8, 8> kc;
-  kc.init(segs, tk.kseg_begin, tk.kseg_end);
+  std::conditional_t<INP, InPlaceCursor, StageCursor<8, 8>> kc;
+  if constexpr (!INP) kc.init(segs, tk.kseg_begin, tk.kseg_end);
   // This wave's loads: base address (row tile, unit 0), operand and LDS unit of each.  Spare
   // loads (when the units do not split evenly over the waves) repeat unit 0's load (same data,
   // same LDS place), so every wave issues the same count.
@@ -643,7 +688,53 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64(const SecTask* __restrict__
   }
   const uint32_t lane16 = (uint32_t)lane * 16u;
   uint8_t* const lds0 = reinterpret_cast<uint8_t*>(&lds[0][0]);
+  // In-place A: this lane's row of each A load (table row and index in its row block), its column
+  // pair, and its run in the current K block.
+  int tabrow[INP ? FPW : 1], rin[INP ? FPW : 1];
+  const double* run[INP ? FPW : 1];
+  const int pcol = INP ? 2 * (((lane & 3) - (lane >> 3)) & 3) : 0;
+  auto open_block = [&] {
+    if constexpr (INP)
+#pragma unroll
+      for (int q = 0; q < FPW; ++q)
+        if (qa[q]) run[q] = Ap + ip_tab[tabrow[q] + kc.kb] + (int64_t)rin[q] * kc.cols + pcol;
+  };
+  if constexpr (INP) {
+    const InPlaceClass cl = ip.classes[tk.plane];
+    const int2* rows = ip.rows + cl.row0;
+    const int last_row = min(tk.m0 + TM, cl.rows) - 1;
+    const int rb0 = rows[tk.m0].x, nrb = rows[last_row].x - rb0 + 1;
+    for (int i = tid; i < nrb * cl.nkb; i += 256) ip_tab[i] = ip.boff[cl.boff0 + (int64_t)rb0 * cl.nkb + i];
+#pragma unroll
+    for (int q = 0; q < FPW; ++q) {
+      const int f = wv * FPW + q;
+      const int2 r = rows[min(tk.m0 + 16 * (f < AF ? f : 0) + (lane >> 2), last_row)];
+      tabrow[q] = (r.x - rb0) * cl.nkb;
+      rin[q] = r.y;
+    }
+    kc.segs = segs;
+    kc.kblk = ip.kblk + cl.kblk0;
+    kc.last = tk.kseg_end - 1;
+    kc.open(tk.kseg_begin);
+    __syncthreads();  // the table
+    open_block();
+  }
+  auto next_stage = [&] {
+    if constexpr (INP) {
+      if (kc.advance()) open_block();
+    } else {
+      kc.advance();
+    }
+  };
   auto dma = [&](int q, uint32_t slot_off, int64_t ca, int64_t cb) {
+    if constexpr (INP) {
+      if (qa[q]) {
+        const int c = kc.ja * 8;
+        const double* src = c + pcol < kc.cols ? run[q] + c : ip.zeros;
+        lds_dma16(src, (__attribute__((address_space(3))) void*)(lds0 + slot_off + ql[q]));
+        return;
+      }
+    }
     const uint8_t* base = qb[q] + (qa[q] ? ca : cb);
     uint32_t lo = lane16;
     asm volatile("" : "+v"(lo));  // per-lane offset stays a fresh VGPR (scalar-base addressing)
@@ -655,12 +746,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64(const SecTask* __restrict__
 #pragma unroll
     for (int j = 0; j < WTN; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
   double fa[2][WTM], fb[2][WTN];
-  const int abase = wm * WTM * 128 + lane, bbase = (AF + wn * WTN) * 128 + lane;
-#define TMX_RD(BUF, SLOT_, KK)                                                                     \
-  {                                                                                               \
-    const double* L = reinterpret_cast<const double*>(&lds[SLOT_][0]);                            \
-    _Pragma("unroll") for (int i = 0; i < WTM; ++i) fa[BUF][i] = L[abase + i * 128 + (KK) * 64]; \
-    _Pragma("unroll") for (int j = 0; j < WTN; ++j) fb[BUF][j] = L[bbase + j * 128 + (KK) * 64]; \
+  // In-place: row l%16's lane of columns 2(l/16), and of B the fragment row of that column.
+  constexpr int ASTEP = INP ? 1 : 64, BSTEP = INP ? 16 : 64;
+  const int g4 = lane >> 4, r16 = lane & 15;
+  const int abase = wm * WTM * 128 + (INP ? 2 * (4 * r16 + ((g4 + (r16 >> 1)) & 3)) : lane);
+  const int bbase = (AF + wn * WTN) * 128 + (INP ? (g4 >> 1) * 64 + (g4 & 1) * 32 + r16 : lane);
+#define TMX_RD(BUF, SLOT_, KK)                                                                        \
+  {                                                                                                  \
+    const double* L = reinterpret_cast<const double*>(&lds[SLOT_][0]);                               \
+    _Pragma("unroll") for (int i = 0; i < WTM; ++i) fa[BUF][i] = L[abase + i * 128 + (KK) * ASTEP]; \
+    _Pragma("unroll") for (int j = 0; j < WTN; ++j) fb[BUF][j] = L[bbase + j * 128 + (KK) * BSTEP]; \
   }
 #define TMX_MM1(BUF, I, J) \
   acc[I][J] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[BUF][I], fb[BUF][J], acc[I][J], 0, 0, 0);
@@ -670,10 +765,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64(const SecTask* __restrict__
       if (i + j > 0) { TMX_MM1(BUF, i, j) }
 #pragma unroll
   for (int s0 = 0; s0 < NS; ++s0) {
-    const int64_t ca = (int64_t)kc.unit_a() * 1024, cb = (int64_t)kc.unit_b() * 1024;
+    int64_t ca = 0;
+    if constexpr (!INP) ca = (int64_t)kc.unit_a() * 1024;
+    const int64_t cb = (int64_t)kc.unit_b() * 1024;
 #pragma unroll
     for (int q = 0; q < FPW; ++q) dma(q, (uint32_t)s0 * SLOT * 1024u, ca, cb);
-    kc.advance();
+    next_stage();
   }
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * FPW) : "memory");
   TMX_RD(0, 0, 0)
@@ -705,13 +802,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64(const SecTask* __restrict__
       if (t < NMM) { TMX_MM1(1, (t + 1) / WTN, (t + 1) % WTN) }
       __builtin_amdgcn_sched_barrier(0);
       if (t == 0) {
-        ca = (int64_t)kc.unit_a() * 1024;
+        if constexpr (!INP) ca = (int64_t)kc.unit_a() * 1024;
         cb = (int64_t)kc.unit_b() * 1024;
       } else if (t == 1) {
         TMX_RD(0, nslot, 0)
       } else if (t - 2 < FPW) {
         dma(t - 2, (uint32_t)slot * SLOT * 1024u, ca, cb);
-        if (t - 2 == FPW - 1) kc.advance();
+        if (t - 2 == FPW - 1) next_stage();
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -1460,10 +1557,10 @@ static int gemm_wg_per_cu(bool split, int tm, int tn) {
   const void* fn = nullptr;
   int threads = 256;
   if (!split) {
-    if (tm == 128 && tn == 128) fn = reinterpret_cast<const void*>(&k_gemm_f64<128, 128, 4>);
-    else if (tm == 128 && tn == 160) fn = reinterpret_cast<const void*>(&k_gemm_f64<128, 160, 4>);
-    else if (tm == 64 && tn == 64) fn = reinterpret_cast<const void*>(&k_gemm_f64<64, 64, 4>);
-    else if (tm == 32 && tn == 32) fn = reinterpret_cast<const void*>(&k_gemm_f64<32, 32, 8>);
+    if (tm == 128 && tn == 128) fn = reinterpret_cast<const void*>(&k_gemm_f64<128, 128, 4, false>);
+    else if (tm == 128 && tn == 160) fn = reinterpret_cast<const void*>(&k_gemm_f64<128, 160, 4, false>);
+    else if (tm == 64 && tn == 64) fn = reinterpret_cast<const void*>(&k_gemm_f64<64, 64, 4, false>);
+    else if (tm == 32 && tn == 32) fn = reinterpret_cast<const void*>(&k_gemm_f64<32, 32, 8, false>);
   } else {
 #define TMX_I8_FN(TM_, TN_, WGM_, WGN_, NS_)                                             \
   if (!fn && tm == TM_ && tn == TN_) {                                                  \
@@ -1597,7 +1694,7 @@ static void tasks_by_shape(const std::vector<SectorGeom>& geoms, int planes,
         t.ldc = g.nrows_pad;
         t.mrows = g.mrows_pad;
         t.nrows = g.nrows_pad;
-        t.plane = pl;
+        t.plane = pl + g.acls;  // FP64: the A class (planes = 1); split: acls is 0
         dst.first.push_back(t);
         dst.second.push_back(g.klen);
         if (exec_flops && pl == 0) *exec_flops += 2.0 * g.tm * g.tn * (double)g.klen;
@@ -1792,17 +1889,21 @@ static void pack_side(PackSide& side, const double* src, bool split, const Secto
   side.last_src = src;
 }
 
-static void launch_gemm(SectorPlan& sp, const ShapeTasks& st, hipStream_t s) {
+// inplace: the tensor data of an A operand read in place (null: packed).
+static void launch_gemm(SectorPlan& sp, const ShapeTasks& st, hipStream_t s, const double* inplace = nullptr) {
   const int grid = (st.ntasks + 7) / 8 * 8;
   if (!sp.split) {
-#define TMX_F64_LAUNCH(TM_, TN_, NS_)                                                          \
-  hipLaunchKernelGGL((k_gemm_f64<TM_, TN_, NS_>), dim3(grid), dim3(256), 0, s, st.tasks.as<SecTask>(), \
-                     st.ntasks, sp.ksegs.as<KSeg>(), sp.A.buf.as<double>(), sp.B.buf.as<double>(), \
-                     sp.cdense.as<double>())
-    if (st.tm == 128 && st.tn == 128) TMX_F64_LAUNCH(128, 128, 4);
-    else if (st.tm == 128 && st.tn == 160) TMX_F64_LAUNCH(128, 160, 4);
-    else if (st.tm == 64 && st.tn == 64) TMX_F64_LAUNCH(64, 64, 4);
-    else if (st.tm == 32 && st.tn == 32) TMX_F64_LAUNCH(32, 32, 8);
+#define TMX_F64_LAUNCH(TM_, TN_, NS_, INP_)                                                          \
+  hipLaunchKernelGGL((k_gemm_f64<TM_, TN_, NS_, INP_>), dim3(grid), dim3(256), 0, s, st.tasks.as<SecTask>(), \
+                     st.ntasks, sp.ksegs.as<KSeg>(), INP_ ? inplace : sp.A.buf.as<double>(),        \
+                     sp.B.buf.as<double>(), sp.cdense.as<double>(), sp.inplace_args)
+    if (inplace && st.tm == 128 && st.tn == 128) TMX_F64_LAUNCH(128, 128, 4, true);
+    else if (inplace && st.tm == 128 && st.tn == 160) TMX_F64_LAUNCH(128, 160, 4, true);
+    else if (inplace) throw Error(TMX_ERR_INVALID, "no in-place FP64 kernel for the tile shape");
+    else if (st.tm == 128 && st.tn == 128) TMX_F64_LAUNCH(128, 128, 4, false);
+    else if (st.tm == 128 && st.tn == 160) TMX_F64_LAUNCH(128, 160, 4, false);
+    else if (st.tm == 64 && st.tn == 64) TMX_F64_LAUNCH(64, 64, 4, false);
+    else if (st.tm == 32 && st.tn == 32) TMX_F64_LAUNCH(32, 32, 8, false);
     else throw Error(TMX_ERR_INVALID, "no FP64 kernel for the requested tile shape");
 #undef TMX_F64_LAUNCH
   } else {
@@ -1953,6 +2054,8 @@ void set_sector_constant(SectorPlan& sp, bool a, bool b) {
   sp.B.constant = b;
 }
 
+void set_sector_inplace(SectorPlan& sp, bool on) { sp.inplace_off = !on; }
+
 void forget_sector_packing(SectorPlan& sp) {
   sp.A.packed_src = sp.B.packed_src = nullptr;
 }
@@ -2015,12 +2118,16 @@ void execute_sector_plan(SectorPlan& sp, const double* A, const double* B, doubl
                          hipStream_t s, hipEvent_t* ev, hipEvent_t* gemm_ev, hipEvent_t* pack_ev_a,
                          hipEvent_t* pack_ev_b) {
   if (ev) TMX_HIP(hipEventRecord(ev[0], s));
-  pack_side(sp.A, A, sp.split, sp, s, pack_ev_a);
+  // In place unless the operand is constant (its packed copy is made once and kept), the pointer
+  // does not allow 16-byte loads, or a shape has no such kernel.
+  bool inplace = sp.inplace && !sp.inplace_off && !sp.A.constant && reinterpret_cast<uintptr_t>(A) % 16 == 0;
+  for (const ShapeTasks& st : sp.shapes) inplace = inplace && st.tm == 128;
+  if (!inplace) pack_side(sp.A, A, sp.split, sp, s, pack_ev_a);
   if (ev) TMX_HIP(hipEventRecord(ev[1], s));
   pack_side(sp.B, B, sp.split, sp, s, pack_ev_b);
   if (ev) TMX_HIP(hipEventRecord(ev[2], s));
   for (size_t i = 0; i < sp.shapes.size(); ++i) {
-    launch_gemm(sp, sp.shapes[i], s);
+    launch_gemm(sp, sp.shapes[i], s, inplace ? A : nullptr);
     if (gemm_ev && i + 1 < sp.shapes.size()) TMX_HIP(hipEventRecord(gemm_ev[i], s));
   }
   if (ev) TMX_HIP(hipEventRecord(ev[3], s));

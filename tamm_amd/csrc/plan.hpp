@@ -115,6 +115,8 @@ bool sector_is_split(const SectorPlan& sp);
 void set_sector_assign(SectorPlan& sp, bool assign);
 // Marks the plan's operands constant (packed once per source address and kept) or not.
 void set_sector_constant(SectorPlan& sp, bool a, bool b);
+// Whether a plan that can read its A operand in place does (default) or packs it.
+void set_sector_inplace(SectorPlan& sp, bool on);
 // Drops what the plan remembers of earlier packings (the next execution packs both operands).
 void forget_sector_packing(SectorPlan& sp);
 // Per-sector tile-shape autotuning on the plan's current packed operands (sector.hpp).

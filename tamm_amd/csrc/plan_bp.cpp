@@ -735,7 +735,10 @@ static int autotune_split_k(tmx_contraction_s* c, const double* A, const double*
     }
   }
   if (!best) return 0;
+  set_sector_inplace(*best, false);
+  run_sector(c, *best, A, B, sc, 1.0, s);
   autotune_sector_plan(*best, s);
+  set_sector_inplace(*best, true);
   c->sec = std::move(best);
   return 1;
 }
@@ -906,8 +909,10 @@ int tmx_contraction_autotune(tmx_contraction c, const double* A, const double* B
                   "rebuilt under them): destroy them before autotuning");
     int n = 0;
     if (c->mode == TMX_EXEC_SECTOR_F64 || c->mode == TMX_EXEC_SPLIT_I8) {
+      set_sector_inplace(*c->sec, false);  // the shapes are timed on packed operands
       run_sector(c, *c->sec, A, B, C, c->alpha, s);
       n = autotune_sector_plan(*c->sec, s);
+      set_sector_inplace(*c->sec, true);
       if (c->parallel_split == 0) n += autotune_split_k(c, A, B, s);
     } else {
       const int rc = tmx_contraction_execute(c, A, B, C, stream);

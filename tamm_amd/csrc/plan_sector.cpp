@@ -275,11 +275,31 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
     split = false;
     sp->split = false;
   }
+  // An FP64 A operand whose labels are the rows' then the reduction's is read in place by the
+  // GEMM (InPlaceA), with 16-byte loads: every block at an even offset, with an even number of
+  // columns and at least 64 of them on average: a GEMM stage reads 64 bytes of a row, and a block
+  // below a few stages is mostly padding and changes of base (pp ladder, in place against packed:
+  // 16 columns 232 and 225 us, 36 columns 164 and 172, 64 columns 368 and 476, 100 columns 404 and
+  // 599, 900 columns 5179 and 6494).
+  bool inplace = !split && nMC > 0;
+  {
+    std::vector<int> mk(ML);
+    mk.insert(mk.end(), KL.begin(), KL.end());
+    inplace = inplace && A.labels == mk;
+    int64_t cols = 0;
+    for (size_t k = 0; inplace && k < nK; ++k) {
+      const int64_t n = tuple_size(KL, kt[k], li);
+      inplace = n % 2 == 0;
+      cols += n;
+    }
+    inplace = inplace && cols >= 64 * (int64_t)nK;
+    for (size_t i = 0; inplace && i < A.t->offs.size(); ++i) inplace = A.t->offs[i] % 2 == 0;
+  }
   std::vector<int64_t> kpadlen(nK);
   const int64_t kstage = split ? KSTAGE_SPLIT : KSTAGE_F64;
   std::vector<int64_t> classlen(kcidx.size(), 0);  // columns of each K class
   for (size_t k = 0; k < nK; ++k) {
-    kpadlen[k] = roundup(tuple_size(KL, kt[k], li), split ? KBLOCK_SPLIT : KBLOCK_F64);
+    kpadlen[k] = roundup(tuple_size(KL, kt[k], li), split ? KBLOCK_SPLIT : inplace ? KSTAGE_F64 : KBLOCK_F64);
     classlen[kcls[k]] += kpadlen[k];
   }
   for (int64_t& n : classlen) n = roundup(n, kstage);
@@ -330,6 +350,62 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
   build_side(Arep, mcls, mt, ML, AM, arow, atotal, agrows);
   build_side(Brep, ncls, nt, NL, BM, brow, btotal, bgrows);
   TMX_REQUIRE(agrows < (1ll << 31) && bgrows < (1ll << 31), "class matrices too large");
+
+  if (inplace) {
+    std::vector<InPlaceClass> classes;
+    std::vector<int2> rows((size_t)agrows, int2{0, 0}), kblk;
+    std::vector<int64_t> boff;
+    for (int c = 0; c < nMC && inplace; ++c) {
+      InPlaceClass ic;
+      std::memset(&ic, 0, sizeof(ic));
+      ic.boff0 = (int64_t)boff.size();
+      ic.kblk0 = (int32_t)kblk.size();
+      ic.row0 = (int32_t)AM[c].growbase;
+      ic.rows = (int32_t)AM[c].rows;
+      inplace = inplace && ic.rows > 0;
+      for (size_t k : korder)
+        if (AM[c].col[k] >= 0) kblk.push_back(int2{(int)AM[c].col[k], (int)tuple_size(KL, kt[k], li)});
+      ic.nkb = (int32_t)kblk.size() - ic.kblk0;
+      int nrb = 0;
+      for (size_t r = 0; r < mt.size() && inplace; ++r) {
+        if (mcls[r] != c) continue;
+        const int64_t n = tuple_size(ML, mt[r], li);
+        for (int64_t i = 0; i < n; ++i) rows[(size_t)(AM[c].growbase + arow[r] + i)] = int2{nrb, (int)i};
+        for (size_t k : korder) {
+          if (AM[c].col[k] < 0) continue;
+          const int64_t off = A.t->find(bid_of(A, ML, mt[r], KL, kt[k]).data());
+          boff.push_back(off);
+          inplace = inplace && off >= 0;
+        }
+        ++nrb;
+      }
+      // the widest tile (128 rows) keeps its row blocks' offsets in LDS
+      for (int64_t m0 = 0; m0 < AM[c].rows && inplace; m0 += 128) {
+        const int first = rows[(size_t)(AM[c].growbase + m0)].x;
+        const int last = rows[(size_t)(AM[c].growbase + std::min<int64_t>(m0 + 128, AM[c].rows) - 1)].x;
+        inplace = (int64_t)(last - first + 1) * ic.nkb <= kInPlaceTable;
+      }
+      classes.push_back(ic);
+    }
+    if (inplace) {
+      std::vector<char> bytes(16, 0);  // the zeros first
+      auto put = [&](const auto& v) {
+        const size_t at = bytes.size(), n = v.size() * sizeof(v[0]);
+        bytes.resize(at + (n + 15) / 16 * 16);
+        if (n) std::memcpy(bytes.data() + at, v.data(), n);
+        return at;
+      };
+      const size_t o_cls = put(classes), o_rows = put(rows), o_kblk = put(kblk), o_boff = put(boff);
+      sp->inplace_buf = upload(bytes);
+      const char* base = sp->inplace_buf.as<char>();
+      sp->inplace_args = InPlaceA{reinterpret_cast<const InPlaceClass*>(base + o_cls),
+                                  reinterpret_cast<const int2*>(base + o_rows),
+                                  reinterpret_cast<const int64_t*>(base + o_boff),
+                                  reinterpret_cast<const int2*>(base + o_kblk),
+                                  reinterpret_cast<const double*>(base)};
+    }
+    sp->inplace = inplace;
+  }
 
   // Pack jobs.
   uint64_t key = 0xcbf29ce484222325ull;  // product fingerprint (FNV-1a)
@@ -517,6 +593,7 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
       g.mrows = (int32_t)am.rows;
       g.nrows = (int32_t)bm.rows;
       g.klen = s2.klen;
+      g.acls = split ? 0 : s2.mc;
       geoms.push_back(g);
     }
     choose_shapes(split, nmod, geoms, trial);
@@ -582,6 +659,14 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
   sp->kmax = kmax;
   sp->split_factor = P.nrounds;
   sp->geoms = make_geoms(P, split ? std::max(moduli_for(kmax), 0) : 0, false);
+  if (sp->inplace)
+    for (const Sector& s2 : secs) {
+      std::vector<int64_t> col0;  // first columns of the class's K blocks, ascending
+      for (size_t k : korder)
+        if (AM[s2.mc].col[k] >= 0) col0.push_back(AM[s2.mc].col[k]);
+      for (int i = s2.seg_b; i < s2.seg_e; ++i)
+        segs[i].a_blk = (int32_t)(std::upper_bound(col0.begin(), col0.end(), (int64_t)segs[i].a_col) - col0.begin()) - 1;
+    }
   sp->ksegs = upload(segs);
   for (const SectorGeom& g : sp->geoms) {
     const int64_t f[] = {g.a_base, g.b_base, g.c_base, g.seg_b, g.seg_e, g.a_kpad, g.b_kpad,

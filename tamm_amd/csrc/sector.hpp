@@ -50,6 +50,22 @@ struct CrtPair {
   int32_t bgrow0;   // global B row of dense col 0 (column scales)
 };
 
+// An FP64 A operand that the GEMM reads from the tensor's blocks: every block of a class is a plain
+// row-major matrix, its row tuple's rows by its K tuple's columns.  Rows map to (row block of the
+// class, row in it); boff holds each class's block offsets, row block by K block.
+struct InPlaceClass {
+  int64_t boff0;
+  int32_t kblk0, nkb, row0, rows;
+};
+struct InPlaceA {
+  const InPlaceClass* classes;
+  const int2* rows;
+  const int64_t* boff;
+  const int2* kblk;     // first (padded) column and columns of each class's K blocks
+  const double* zeros;  // 16 zero bytes
+};
+constexpr int kInPlaceTable = 512;  // block offsets of one tile's row blocks, kept in LDS
+
 struct PackSide {
   DevBuf jobs;
   int njobs = 0;
@@ -91,6 +107,7 @@ struct SectorGeom {
   int32_t mrows, nrows;          // rows that carry data
   int64_t klen;
   int tm, tn;
+  int32_t acls;  // A class (FP64; 0 on the split path)
 };
 
 struct ShapeTasks {
@@ -108,6 +125,10 @@ struct SectorPlan {
   std::vector<SectorGeom> geoms;
   std::vector<ShapeTasks> shapes;
   DevBuf ksegs;
+  bool inplace = false;      // A may be read in place (inplace_args)
+  bool inplace_off = false;  // switched off (the autotuner times GEMMs on packed operands)
+  InPlaceA inplace_args{};
+  DevBuf inplace_buf;
   DevBuf cdense;        // dense FP64 result, row-major per sector (ld = nrows_pad)
   DevBuf cres;          // split: nmod residue planes of the dense result, 32x32-tile native
   DevBuf crt_secs;      // split: CrtSector per sector

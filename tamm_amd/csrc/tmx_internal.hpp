@@ -277,10 +277,11 @@ struct SecTask {
   int32_t a_kpad, b_kpad;  // padded column counts of the A / B class matrices
   int32_t ldc;             // leading dimension of the dense result
   int32_t mrows, nrows;    // valid rows of the A / B class matrices (0: empty task)
-  int32_t plane;           // residue plane (split path)
+  int32_t plane;           // residue plane (split path) or A class (FP64)
 };
 struct KSeg {
-  int32_t a_col, b_col, len, pad;
+  int32_t a_col, b_col, len;
+  int32_t a_blk;  // K block of the A class that holds a_col (plans that read A in place)
 };
 
 // Scatter of a dense sector result into the C tensor's block layout.
