@@ -128,6 +128,16 @@ __device__ __forceinline__ void residues16(const double* cells, const RowScale& 
 }
 
 // ---------------------------------------------------------------------------
+// Unit of iteration i when n units are dealt over the 8 XCDs in contiguous eighths (workgroups,
+// and iterations a whole number of 8 apart, go to the XCDs in turn); iterations run to
+// xcd_rounds(n), and units past n are none.  Units that follow each other share lines: a row that
+// does not begin on a line ends its piece inside one, and a row tile that does not begin on a
+// fragment shares its output lines with the next tile, so both want the same L2 (split V(a,b,c,d)
+// of 60 + 300 orbitals in 4 irreps, odd rows: 4019 -> 3035 us; of O=30, V=180: 1615 -> 1490; with
+// 8, 32 and 128 units a turn instead of eighths 3798, 3364 and 3099).
+__device__ __forceinline__ int64_t xcd_unit(int64_t i, int64_t n) { return (i & 7) * ((n + 7) >> 3) + (i >> 3); }
+__host__ __device__ __forceinline__ int64_t xcd_rounds(int64_t n) { return (n + 7) / 8 * 8; }
+
 // Loads the 64x64 tile (rows nr, columns nc valid; the rest reads 0) of a pack job that is not
 // contiguous along whole rows into LDS, lanes along the source's contiguous direction.  When
 // the fastest column digit (kcontig) or row digit (otherwise) has an extent L dividing 64, one
@@ -135,39 +145,42 @@ __device__ __forceinline__ void residues16(const double* cells, const RowScale& 
 // the next-fastest source mode is the other side's fastest digit, e.g. T(a,c,i,k) with rows
 // (a,i) and K = (c,k).  Otherwise lanes run along 64 columns or 64 rows.  Addresses always come
 // from the row and column offset tables; the mapping only decides which lanes share a load.
-__device__ __forceinline__ void load_tile64(double (*tile)[65], const PackJob& jb, const double* s,
+// All 16 loads of a lane are in flight at once: no load is conditional (the tables hold 0 past
+// the tile, so such a lane reads the tile's first row or column and its value is replaced by 0);
+// behind a condition each waited for the one before it (FP64 L(a,b,c,d) of O=30, V=180 with its
+// rows along K: 2122 -> 1640 us).
+template <class At>
+__device__ __forceinline__ void load_tile16(double* tile, int ld, const double* s, const int* roff,
+                                            const int* coff, int nr, int nc, const At& at) {
+  double v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int2 rc = at(i);
+    v[i] = s[roff[rc.x] + coff[rc.y]];
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int2 rc = at(i);
+    tile[rc.x * ld + rc.y] = rc.x < nr && rc.y < nc ? v[i] : 0.0;
+  }
+}
+
+__device__ __forceinline__ void load_tile64(double* tile, const PackJob& jb, const double* s,
                                             const int* roff, const int* coff, int nr, int nc,
                                             int tid) {
   const int lane = tid & 63, w = tid >> 6;
   const int L = jb.kcontig ? jb.c.ext[jb.c.n - 1] : jb.r.ext[jb.r.n - 1];
-  if (L >= 2 && L < 64 && (L & (L - 1)) == 0) {
-    const int lg = __builtin_ctz(L), sh = 6 - lg;  // 2^sh = 64 / L
-#pragma unroll 4
-    for (int i = 0; i < 16; ++i) {
-      const int f = w + 4 * i;  // wave load 0..63: group f >> sh, sub-group f & (2^sh - 1)
-      int rr, cc;
-      if (jb.kcontig) {
-        rr = (f >> sh) * (64 >> lg) + (lane >> lg);
-        cc = (f & ((1 << sh) - 1)) * L + (lane & (L - 1));
-      } else {
-        rr = (f & ((1 << sh) - 1)) * L + (lane & (L - 1));
-        cc = (f >> sh) * (64 >> lg) + (lane >> lg);
-      }
-      tile[rr][cc] = (rr < nr && cc < nc) ? s[roff[rr] + coff[cc]] : 0.0;
-    }
-  } else if (jb.kcontig) {
-#pragma unroll 4
-    for (int i = 0; i < 16; ++i) {
-      const int rr = w + 4 * i, cc = lane;
-      tile[rr][cc] = (rr < nr && cc < nc) ? s[roff[rr] + coff[cc]] : 0.0;
-    }
-  } else {
-#pragma unroll 4
-    for (int i = 0; i < 16; ++i) {
-      const int rr = lane, cc = w + 4 * i;
-      tile[rr][cc] = (rr < nr && cc < nc) ? s[roff[rr] + coff[cc]] : 0.0;
-    }
-  }
+  // wave load f = w + 4 i (0..63); lanes along columns (kcontig) or along rows
+  int lg = 6;
+  if (L >= 2 && L < 64 && (L & (L - 1)) == 0) lg = __builtin_ctz(L);
+  const int sh = 6 - lg;  // load f: group f >> sh, sub-group f & (2^sh - 1)
+  const bool k = jb.kcontig;
+  load_tile16(tile, 65, s, roff, coff, nr, nc, [&](int i) {
+    const int f = w + 4 * i;
+    const int x = (f >> sh << sh) + (lane >> lg);  // across the lanes' direction
+    const int y = ((f & ((1 << sh) - 1)) << lg) + (lane & ((1 << lg) - 1));
+    return k ? make_int2(x, y) : make_int2(y, x);
+  });
 }
 
 // Row stride in doubles of an LDS pack tile of 2^lt rows x 4096 / 2^lt columns (lt = 3..8):
@@ -188,17 +201,15 @@ __device__ __forceinline__ void load_pack_tile(double* tile, int lt, const PackJ
                                                const int* roff, const int* coff, int nr, int nc,
                                                int tid) {
   if (lt == 6) {
-    load_tile64(reinterpret_cast<double(*)[65]>(tile), jb, s, roff, coff, nr, nc, tid);
+    load_tile64(tile, jb, s, roff, coff, nr, nc, tid);
     return;
   }
-  const int ld = pack_ld(lt), ltc = 12 - lt;
-#pragma unroll 4
-  for (int i = 0; i < 16; ++i) {
+  const int ltc = 12 - lt;
+  const bool k = jb.kcontig;
+  load_tile16(tile, pack_ld(lt), s, roff, coff, nr, nc, [&](int i) {
     const int e = tid + 256 * i;
-    const int rr = jb.kcontig ? e >> ltc : e & ((1 << lt) - 1);
-    const int cc = jb.kcontig ? e & ((1 << ltc) - 1) : e >> lt;
-    tile[rr * ld + cc] = (rr < nr && cc < nc) ? s[roff[rr] + coff[cc]] : 0.0;
-  }
+    return k ? make_int2(e >> ltc, e & ((1 << ltc) - 1)) : make_int2(e & ((1 << lt) - 1), e >> lt);
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -213,7 +224,7 @@ __device__ __forceinline__ void load_pack_tile(double* tile, int lt, const PackJ
 // atomicMax per row and tile), with `gate` the whole grid returns unless *gate != 0, and with
 // `zero_flag` the first block clears that flag (for a check that runs after the pass).
 template <int MODE>  // 0: FP64 copy, 2: int8 residues
-__global__ __launch_bounds__(256) void k_pack(const PackJob* __restrict__ jobs,
+__global__ __launch_bounds__(256, 4) void k_pack(const PackJob* __restrict__ jobs,
                                               const TileUnit* __restrict__ units, int64_t nunits,
                                               const double* __restrict__ src,
                                               double* __restrict__ dst64,
@@ -230,7 +241,9 @@ __global__ __launch_bounds__(256) void k_pack(const PackJob* __restrict__ jobs,
   const int tid = threadIdx.x;
   if (gate != nullptr && *gate == 0) return;
   if (zero_flag != nullptr && blockIdx.x == 0 && tid == 0) *zero_flag = 0;
-  for (int64_t u = blockIdx.x; u < nunits; u += gridDim.x) {
+  for (int64_t it = blockIdx.x; it < xcd_rounds(nunits); it += gridDim.x) {
+    const int64_t u = xcd_unit(it, nunits);
+    if (u >= nunits) continue;
     const TileUnit un = units[u];
     const PackJob& jb = jobs[un.job];
     const int lt = un.lt, TR = 1 << lt, TC = 4096 >> lt, ld = pack_ld(lt);
@@ -322,9 +335,13 @@ __global__ __launch_bounds__(256) void k_rowmax_t(const PackJob* __restrict__ jo
 // (K labels trail the source block's modes in order, e.g. V(a,b,c,d) with K = (c,d); such
 // blocks with fewer rows go through k_pack's wider tiles).  A workgroup iteration takes
 // 32 rows x 128 columns: each wave reads 8 rows with 16-byte loads, 1 KB of one row per
-// instruction (8-byte loads when a row run is not 16-byte aligned), into an LDS tile; then each
-// thread emits one row's 16 consecutive columns in fragment order, as k_pack does.
-// `rowmax`, `maxout`, `gate` and `zero_flag` as in k_pack.
+// instruction (two 8-byte loads of 64 columns each in blocks whose rows are not all 16-byte
+// aligned), all of them in flight, into an LDS tile; then each thread emits one row's 16
+// consecutive columns in fragment order, as k_pack does.
+// `rowmax`, `maxout`, `gate` and `zero_flag` as in k_pack.  Bound by memory: split V(a,b,c,d)
+// (8 B read, 11 B written an element) of O=30, V=180 1672 -> 1490 us (5.0 TB/s), of 50 + 320
+// orbitals in 4 irreps 3942 -> 3555 (5.4 TB/s), of 60 + 300 with odd rows 3758 -> 3040 (4.7 TB/s)
+// against loads one by one, 8192 looping workgroups and units dealt singly.
 template <int MODE>  // 0: FP64 copy, 2: int8 residues
 __global__ __launch_bounds__(256, 4) void k_pack_kf(const PackJob* __restrict__ jobs,
                                                  const TileUnit* __restrict__ units, int64_t nunits,
@@ -344,31 +361,39 @@ __global__ __launch_bounds__(256, 4) void k_pack_kf(const PackJob* __restrict__ 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   if (gate != nullptr && *gate == 0) return;
   if (zero_flag != nullptr && blockIdx.x == 0 && tid == 0) *zero_flag = 0;
-  for (int64_t u = blockIdx.x; u < nunits; u += gridDim.x) {
+  for (int64_t it = blockIdx.x; it < xcd_rounds(nunits); it += gridDim.x) {
+    const int64_t u = xcd_unit(it, nunits);
+    if (u >= nunits) continue;
     const TileUnit un = units[u];
     const PackJob& jb = jobs[un.job];
     const int nr = min(TR, jb.rows - un.r0), nc = min(TC, jb.cols - un.c0);
     if (tid < TR) roff[tid] = tid < nr ? radix_off(jb.r, un.r0 + tid) : 0;
     __syncthreads();
     const double* s = src + jb.src_off + un.c0;
-    const int cc = 2 * lane;
+    // Row offsets are multiples of the block's columns; rows past the tile read its first row
+    // (offset 0 in the table, not used) and columns past it its first column (replaced by 0).
+    if (((reinterpret_cast<uintptr_t>(s) & 15) | (jb.cols & 1)) == 0) {
+      const int cc = 2 * lane, cr = cc < nc ? cc : 0;
+      double2 v[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int rr = w * 8 + i;
-      double v0 = 0.0, v1 = 0.0;
-      if (rr < nr) {
-        const double* rp = s + roff[rr];
-        if (cc + 1 < nc && ((reinterpret_cast<uintptr_t>(rp) & 15) == 0)) {
-          const double2 v = *reinterpret_cast<const double2*>(rp + cc);
-          v0 = v.x;
-          v1 = v.y;
-        } else {
-          if (cc < nc) v0 = rp[cc];
-          if (cc + 1 < nc) v1 = rp[cc + 1];
-        }
+      for (int i = 0; i < 8; ++i) v[i] = *reinterpret_cast<const double2*>(s + roff[w * 8 + i] + cr);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        tile[w * 8 + i][cc] = cc < nc ? v[i].x : 0.0;
+        tile[w * 8 + i][cc + 1] = cc < nc ? v[i].y : 0.0;
       }
-      tile[rr][cc] = v0;
-      tile[rr][cc + 1] = v1;
+    } else {
+      double v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int cc = 64 * (i & 1) + lane;
+        v[i] = s[roff[w * 8 + (i >> 1)] + (cc < nc ? cc : 0)];
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int cc = 64 * (i & 1) + lane;
+        tile[w * 8 + (i >> 1)][cc] = cc < nc ? v[i] : 0.0;
+      }
     }
     __syncthreads();
     const int rr = tid & 31, q = tid >> 5;  // row, 16-column group
@@ -1401,28 +1426,40 @@ __global__ __launch_bounds__(256) void k_scatter(const ScatterJob* __restrict__ 
     const int nr = min(64, jb.rows - un.r0), nc = min(64, jb.cols - un.c0);
     if (tid < 64) roff[tid] = tid < nr ? radix_off(jb.r, un.r0 + tid) : 0;
     else if (tid < 128) coff[tid - 64] = (tid - 64) < nc ? radix_off(jb.c, un.c0 + tid - 64) : 0;
-#pragma unroll 4
-    for (int i = 0; i < 16; ++i) {
-      const int rr = (tid >> 6) + 4 * i, cc = tid & 63;
-      double v = 0.0;
-      if (rr < nr && cc < nc) {
-        const double* src = Cd + jb.src_base + (int64_t)(jb.row0 + un.r0 + rr) * jb.ldc + jb.col0 + un.c0 + cc;
-        for (int p = 0; p < jb.nparts; ++p) v += src[(int64_t)p * jb.pstride];
+    {
+      // No load is conditional (rows and columns past the tile repeat its last), so a lane's 16
+      // are in flight at once (1.1e7 results of 4 parts 163 -> 94 us; 3.9e8 of one 2265 -> 1335).
+      const int cc = tid & 63;
+      const double* src = Cd + jb.src_base + (int64_t)(jb.row0 + un.r0) * jb.ldc + jb.col0 + un.c0 + min(cc, nc - 1);
+      double v[16], x[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = src[(int64_t)min((tid >> 6) + 4 * i, nr - 1) * jb.ldc];
+      for (int p = 1; p < jb.nparts; ++p) {
+        src += jb.pstride;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] = src[(int64_t)min((tid >> 6) + 4 * i, nr - 1) * jb.ldc];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] += x[i];
       }
-      tile[rr][cc] = alpha * v;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) tile[(tid >> 6) + 4 * i][cc] = alpha * v[i];
     }
     __syncthreads();
     double* cb = C + jb.c_off;
-    if (jb.ccontig) {
-      for (int i = 0; i < 16; ++i) {
-        const int rr = (tid >> 6) + 4 * i, cc = tid & 63;
-        if (rr < nr && cc < nc) cb[roff[rr] + coff[cc]] = (assign ? 0.0 : cb[roff[rr] + coff[cc]]) + tile[rr][cc];
-      }
-    } else {
-      for (int i = 0; i < 16; ++i) {
-        const int rr = tid & 63, cc = (tid >> 6) + 4 * i;
-        if (rr < nr && cc < nc) cb[roff[rr] + coff[cc]] = (assign ? 0.0 : cb[roff[rr] + coff[cc]]) + tile[rr][cc];
-      }
+    const bool cc_lanes = jb.ccontig;
+    const auto place = [&](int i) {  // lanes along C's contiguous direction
+      return cc_lanes ? make_int2((tid >> 6) + 4 * i, tid & 63) : make_int2(tid & 63, (tid >> 6) + 4 * i);
+    };
+    double old[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int2 rc = place(i);  // past the tile: the offset tables hold 0
+      old[i] = assign ? 0.0 : cb[roff[rc.x] + coff[rc.y]];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int2 rc = place(i);
+      if (rc.x < nr && rc.y < nc) cb[roff[rc.x] + coff[rc.y]] = old[i] + tile[rc.x][rc.y];
     }
     __syncthreads();
   }
@@ -1793,6 +1830,9 @@ void sector_schedule_info(const SectorPlan& sp, int* rounds, int* launches, int6
 }
 
 static int grid_units(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(n, 8192)); }
+// A packing pass: a workgroup per unit (a workgroup that loops waits for its own stores before it
+// loads again: split V(a,b,c,d) of 50 + 320 orbitals 3871 us with 8192, 3654 so), or at most `cap`.
+static int grid_pack(int64_t n, int64_t cap = 1ll << 30) { return (int)std::min(xcd_rounds(n), cap); }
 
 static std::atomic<bool> g_scale_reuse{true};  // tmx_set_scale_reuse, read at execution
 constexpr int kScaleReuseBackoff = 8;
@@ -1813,12 +1853,12 @@ static void pack_side(PackSide& side, const double* src, bool split, const Secto
   if (!split) {
     mark(0);
     if (side.nunits > 0)
-      hipLaunchKernelGGL(k_pack<0>, dim3(grid_units(side.nunits)), dim3(256), 0, s,
+      hipLaunchKernelGGL(k_pack<0>, dim3(grid_pack(side.nunits)), dim3(256), 0, s,
                          side.jobs.as<PackJob>(), side.units.as<TileUnit>(), side.nunits, src,
                          side.buf.as<double>(), nullptr, (int64_t)0, nullptr, nullptr, sp.crt, 0.0,
                          nullptr, nullptr, nullptr);
     if (side.nkfunits > 0)
-      hipLaunchKernelGGL(k_pack_kf<0>, dim3(grid_units(side.nkfunits)), dim3(256), 0, s,
+      hipLaunchKernelGGL(k_pack_kf<0>, dim3(grid_pack(side.nkfunits)), dim3(256), 0, s,
                          side.jobs.as<PackJob>(), side.kfunits.as<TileUnit>(), side.nkfunits, src,
                          side.buf.as<double>(), nullptr, (int64_t)0, nullptr, nullptr, sp.crt, 0.0,
                          nullptr, nullptr, nullptr);
@@ -1831,16 +1871,16 @@ static void pack_side(PackSide& side, const double* src, bool split, const Secto
   // smaller (it returns at once unless enabled, and its blocks loop over the units);
   // zero_flag: cleared by the first block of the first launch.
   auto pack = [&](unsigned long long* maxout, const int* gate, int* zero_flag) {
-    const int64_t cap = gate ? 1024 : 8192;
+    const int64_t cap = gate ? 1024 : 1ll << 30;
     if (side.nunits > 0) {
-      hipLaunchKernelGGL(k_pack<2>, dim3(std::min<int64_t>(grid_units(side.nunits), cap)), dim3(256), 0, s,
+      hipLaunchKernelGGL(k_pack<2>, dim3(grid_pack(side.nunits, cap)), dim3(256), 0, s,
                          side.jobs.as<PackJob>(), side.units.as<TileUnit>(), side.nunits, src, nullptr,
                          side.buf.as<uint8_t>(), side.total, side.rowmax.as<unsigned long long>(),
                          side.invscale.as<double2>(), sp.crt, top, maxout, gate, zero_flag);
       zero_flag = nullptr;
     }
     if (side.nkfunits > 0)
-      hipLaunchKernelGGL(k_pack_kf<2>, dim3(std::min<int64_t>(grid_units(side.nkfunits), cap)), dim3(256), 0, s,
+      hipLaunchKernelGGL(k_pack_kf<2>, dim3(grid_pack(side.nkfunits, cap)), dim3(256), 0, s,
                          side.jobs.as<PackJob>(), side.kfunits.as<TileUnit>(), side.nkfunits, src,
                          nullptr, side.buf.as<uint8_t>(), side.total,
                          side.rowmax.as<unsigned long long>(), side.invscale.as<double2>(), sp.crt, top,
