@@ -997,7 +997,15 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_i8(
 #undef TMX_MM_REST
   // No LDS-DMA may still be writing when the workgroup retires.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  const double md = (double)cc.m[l], rm = cc.rcp[l];
+  // Residues as in residues16: |acc| < 2^31, so fma(acc, 1/m, 1.5*2^52) rounds to q within 2^-20/m
+  // of the quotient, inside the rounding margin 1/(2m) of odd m (m = 256 is exact; a tie rounds to
+  // even), and its low 32 bits are q; acc - q m lies in [-(m-1)/2, (m-1)/2] (odd m) or [-128, 128]
+  // (128 and -128 share the byte 0x80 and are congruent) and its low byte is that of
+  // acc + q (2^24 - m), one 24-bit multiply-add.  One conversion, one FP64 and one integer operation
+  // an element, and the byte merge: with five FP64 operations instead the products of a short K
+  // (L(a,b,i,j) T(c,d,i,j), K = 450, 3.9e8 results) took 2765 us, with FP32 ones 2806, so 2620.
+  const double rm = cc.rcp[l];
+  const uint32_t negm = (1u << 24) - (uint32_t)cc.m[l];
   uint8_t* Cp = Cr + (int64_t)l * cplane + tk.c_base;
   const int ntc = tk.ldc >> 5;
 #pragma unroll
@@ -1006,15 +1014,17 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_i8(
     for (int j = 0; j < WTN; ++j) {
       const int tr = rt0 + wm * WTM + i, tc = ct0 + wn * WTN + j;
       if (tr < art && tc < brt) {
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
+        uint32_t w[4];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          // |acc| < 2^31: the FP64 quotient is exact to far below the rounding margin, so the
-          // residue lies in [-(m-1)/2, (m-1)/2] (odd m) or [-128, 128] (m = 256; 128 and -128
-          // share the byte 0x80 and are congruent).
-          const double xd = (double)acc[i][j][e];
-          const int r = (int)fma(-rint(xd * rm), md, xd);
-          w[e >> 2] |= ((uint32_t)r & 0xffu) << (8 * (e & 3));
+        for (int k = 0; k < 4; ++k) {
+          uint32_t d[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int x = acc[i][j][4 * k + e];
+            const uint32_t q = (uint32_t)__double_as_longlong(fma((double)x, rm, 0x1.8p52));
+            d[e] = (uint32_t)x + __umul24(q, negm);
+          }
+          w[k] = __builtin_amdgcn_perm(d[1], d[0], 0x0c0c0400u) | __builtin_amdgcn_perm(d[3], d[2], 0x04000c0cu);
         }
         *reinterpret_cast<i4*>(Cp + ((int64_t)tr * ntc + tc) * 1024 + lane * 16) =
             i4{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
@@ -1033,7 +1043,7 @@ __global__ __launch_bounds__(256) void k_crt(const CrtSector* __restrict__ secs,
                                              const double2* __restrict__ invB,
                                              double* __restrict__ Cd) {
   const int lane = threadIdx.x & 63;
-  const double L1 = 0x1p42, L2 = 0x1p84, iL1 = 0x1p-42;
+  const double L1 = 0x1p42, L2 = 0x1p84;
   for (int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); t < ntiles;
        t += (int64_t)gridDim.x * 4) {
     // sector of tile t (sectors are few; linear scan over cumulative tile counts)
@@ -1067,16 +1077,11 @@ __global__ __launch_bounds__(256) void k_crt(const CrtSector* __restrict__ secs,
       // S = S2*2^84 + S1*2^42 + S0 (exact limbs); q = round(S / M); x = S - q*M, exact per limb.
       const double D = fma(S2[e], L2, fma(S1[e], L1, S0[e]));
       const double qq = rint(D * cc.inv_m_total);
-      double x0 = fma(-qq, cc.M[0], S0[e]);
-      double x1 = fma(-qq, cc.M[1], S1[e]);
-      double x2 = fma(-qq, cc.M[2], S2[e]);
-      const double c0 = rint(x0 * iL1);
-      x0 = fma(-c0, L1, x0);
-      x1 += c0;
-      const double c1 = rint(x1 * iL1);
-      x1 = fma(-c1, L1, x1);
-      x2 += c1;
-      const double x = fma(x2, L2, fma(x1, L1, x0));
+      const double x0 = fma(-qq, cc.M[0], S0[e]);
+      const double x1 = fma(-qq, cc.M[1], S1[e]);
+      const double x2 = fma(-qq, cc.M[2], S2[e]);
+      // x2*2^42 + x1 is (x - x0) / 2^42: exact below 2^53, and above it |x0| < 2^53 cannot cancel it
+      const double x = fma(fma(x2, L1, x1), L1, x0);
       const int row = tr * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
       Cd[sc.c_base + (int64_t)row * sc.ldc + col] = unscale(x, invA[sc.agrow0 + row], sb, sbe);
     }
@@ -1099,28 +1104,24 @@ __device__ __forceinline__ void crt_tile_values(const FusedTile& ft, const CrtPa
                                                 double2 sb2, double v[16]) {
   const double sb = sb2.x;
   const int sbe = inv_exp(sb2);
-  const double L1 = 0x1p42, L2 = 0x1p84, iL1 = 0x1p-42;
   const int64_t toff = ((int64_t)ft.tr * pr.ntc + ft.tc) * 1024 + lane * 16;
-  // Reconstruction of one element from its limb sums over the planes: the exact reduction mod
-  // M (as k_crt).
+  // Reconstruction of one element from its limb sums: the exact reduction mod M (as k_crt).
+  constexpr double L1 = NM > 0 ? 0x1p27 : 0x1p42, L2 = L1 * L1;
+  const double* M = NM > 0 ? cc.pM : cc.M;
   auto finish = [&](double s0, double s1, double s2) {
     const double D = fma(s2, L2, fma(s1, L1, s0));
     const double qq = rint(D * cc.inv_m_total);
-    double x0 = fma(-qq, cc.M[0], s0);
-    double x1 = fma(-qq, cc.M[1], s1);
-    double x2 = fma(-qq, cc.M[2], s2);
-    const double c0 = rint(x0 * iL1);
-    x0 = fma(-c0, L1, x0);
-    x1 += c0;
-    const double c1 = rint(x1 * iL1);
-    x1 = fma(-c1, L1, x1);
-    x2 += c1;
-    return fma(x2, L2, fma(x1, L1, x0));
+    return fma(fma(fma(-qq, M[2], s2), L1, fma(-qq, M[1], s1)), L1, fma(-qq, M[0], s0));
   };
 #pragma unroll
   for (int e = 0; e < 16; ++e) v[e] = 0.0;
   if constexpr (NM > 0) {
-    // moduli count known: a part's 16 bytes per plane are loaded once into registers
+    // kPairModuli: a part's 16 bytes per plane are loaded once into registers, and the residues
+    // r, r' of two moduli are combined first, t = r c + r' c' (|t| < 2^23, one conversion), with a
+    // weight 16 bits shorter: 18 multiply-adds in FP64 over three limbs of 27 bits (sums below
+    // 2^51, exact) instead of 33.  These kernels follow a GEMM at the card's power limit and their
+    // FP64 units were busiest: CRT scatter of 1.1e7 results 89 -> 80 us, of 3.9e8 1943 -> 1862.
+    static_assert(NM == kPairModuli);
     for (int p = 0; p < pr.nparts; ++p) {
       const int8_t* rp = Cr + pr.c_base + p * pr.pstride + toff;
       i4 q[NM];
@@ -1132,12 +1133,14 @@ __device__ __forceinline__ void crt_tile_values(const FusedTile& ft, const CrtPa
 #pragma unroll
         for (int e = 0; e < 4; ++e) S0[e] = S1[e] = S2[e] = 0.0;
 #pragma unroll
-        for (int k = 0; k < NM; ++k) {
-          const double w0 = cc.w[k][0], w1 = cc.w[k][1], w2 = cc.w[k][2];
-          const uint32_t word = (uint32_t)q[k][g];
+        for (int k = 0; k < NM; k += 2) {
+          const double w0 = cc.pw[k / 2][0], w1 = cc.pw[k / 2][1], w2 = cc.pw[k / 2][2];
+          const uint32_t word = (uint32_t)q[k][g], next = k + 1 < NM ? (uint32_t)q[k + 1 < NM ? k + 1 : k][g] : 0u;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const double r = (double)(int)(int8_t)(word >> (8 * e));
+            int t = (int8_t)(word >> (8 * e));
+            if (k + 1 < NM) t = __mul24(t, cc.pc[k]) + __mul24((int)(int8_t)(next >> (8 * e)), cc.pc[k + 1 < NM ? k + 1 : k]);
+            const double r = (double)t;
             S0[e] = fma(r, w0, S0[e]);
             S1[e] = fma(r, w1, S1[e]);
             S2[e] = fma(r, w2, S2[e]);
@@ -1830,9 +1833,10 @@ void sector_schedule_info(const SectorPlan& sp, int* rounds, int* launches, int6
 }
 
 static int grid_units(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(n, 8192)); }
-// A packing pass: a workgroup per unit (a workgroup that loops waits for its own stores before it
-// loads again: split V(a,b,c,d) of 50 + 320 orbitals 3871 us with 8192, 3654 so), or at most `cap`.
-static int grid_pack(int64_t n, int64_t cap = 1ll << 30) { return (int)std::min(xcd_rounds(n), cap); }
+// A packing or CRT scatter pass: a workgroup per unit (a workgroup that loops waits for its own stores before it
+// loads again: split V(a,b,c,d) of 50 + 320 orbitals 3871 us with 8192, 3654 so;
+// CRT scatter of 3.9e8 results 1865 and 1801), or at most `cap`.
+static int grid_full(int64_t n, int64_t cap = 1ll << 30) { return (int)std::min(xcd_rounds(n), cap); }
 
 static std::atomic<bool> g_scale_reuse{true};  // tmx_set_scale_reuse, read at execution
 constexpr int kScaleReuseBackoff = 8;
@@ -1853,12 +1857,12 @@ static void pack_side(PackSide& side, const double* src, bool split, const Secto
   if (!split) {
     mark(0);
     if (side.nunits > 0)
-      hipLaunchKernelGGL(k_pack<0>, dim3(grid_pack(side.nunits)), dim3(256), 0, s,
+      hipLaunchKernelGGL(k_pack<0>, dim3(grid_full(side.nunits)), dim3(256), 0, s,
                          side.jobs.as<PackJob>(), side.units.as<TileUnit>(), side.nunits, src,
                          side.buf.as<double>(), nullptr, (int64_t)0, nullptr, nullptr, sp.crt, 0.0,
                          nullptr, nullptr, nullptr);
     if (side.nkfunits > 0)
-      hipLaunchKernelGGL(k_pack_kf<0>, dim3(grid_pack(side.nkfunits)), dim3(256), 0, s,
+      hipLaunchKernelGGL(k_pack_kf<0>, dim3(grid_full(side.nkfunits)), dim3(256), 0, s,
                          side.jobs.as<PackJob>(), side.kfunits.as<TileUnit>(), side.nkfunits, src,
                          side.buf.as<double>(), nullptr, (int64_t)0, nullptr, nullptr, sp.crt, 0.0,
                          nullptr, nullptr, nullptr);
@@ -1873,14 +1877,14 @@ static void pack_side(PackSide& side, const double* src, bool split, const Secto
   auto pack = [&](unsigned long long* maxout, const int* gate, int* zero_flag) {
     const int64_t cap = gate ? 1024 : 1ll << 30;
     if (side.nunits > 0) {
-      hipLaunchKernelGGL(k_pack<2>, dim3(grid_pack(side.nunits, cap)), dim3(256), 0, s,
+      hipLaunchKernelGGL(k_pack<2>, dim3(grid_full(side.nunits, cap)), dim3(256), 0, s,
                          side.jobs.as<PackJob>(), side.units.as<TileUnit>(), side.nunits, src, nullptr,
                          side.buf.as<uint8_t>(), side.total, side.rowmax.as<unsigned long long>(),
                          side.invscale.as<double2>(), sp.crt, top, maxout, gate, zero_flag);
       zero_flag = nullptr;
     }
     if (side.nkfunits > 0)
-      hipLaunchKernelGGL(k_pack_kf<2>, dim3(grid_pack(side.nkfunits, cap)), dim3(256), 0, s,
+      hipLaunchKernelGGL(k_pack_kf<2>, dim3(grid_full(side.nkfunits, cap)), dim3(256), 0, s,
                          side.jobs.as<PackJob>(), side.kfunits.as<TileUnit>(), side.nkfunits, src,
                          nullptr, side.buf.as<uint8_t>(), side.total,
                          side.rowmax.as<unsigned long long>(), side.invscale.as<double2>(), sp.crt, top,
@@ -2111,7 +2115,7 @@ static void scatter_stage(const SectorPlan& sp, const SectorPlan& src, double* C
     launch_zero_ranges(sp.zero_off.as<int64_t>(), sp.zero_prefix.as<int64_t>(), sp.nzero,
                        sp.zero_elems, C, s);
   if (sp.split && sp.nfused > 0) {
-    const int g = (int)std::max<int64_t>(1, std::min<int64_t>((sp.nfused + 3) / 4, 8192));
+    const int g = grid_full((sp.nfused + 3) / 4);
 #define TMX_CRT_SCATTER(NM_)                                                                  \
   hipLaunchKernelGGL(k_crt_scatter<NM_>, dim3(g), dim3(256), 0, s, sp.fused_tiles.as<FusedTile>(), \
                      sp.nfused, sp.crt_pairs.as<CrtPair>(), sp.scatter[0].jobs.as<ScatterJob>(),  \

@@ -135,17 +135,19 @@ int inv_mod(int a, int m) {
   throw Error(TMX_ERR_INVALID, "moduli are not coprime");
 }
 
-// Balanced base-2^42 limbs of a signed 128-bit integer: v = l2*2^84 + l1*2^42 + l0.
-void limbs42(__int128 v, double out[3]) {
-  const __int128 L = (__int128)1 << 42;
-  for (int k = 0; k < 3; ++k) {
+// Balanced base-2^bits limbs of a signed 128-bit integer, v = l2*4^bits + l1*2^bits + l0; the last
+// takes what is left.
+void limbs(__int128 v, int bits, double out[3]) {
+  const __int128 L = (__int128)1 << bits;
+  for (int k = 0; k < 2; ++k) {
     __int128 d = v % L;
     if (d > L / 2) d -= L;
     else if (d < -L / 2) d += L;
     out[k] = (double)(long long)d;
     v = (v - d) / L;
   }
-  TMX_REQUIRE(v == 0, "CRT constant exceeds three limbs");
+  TMX_REQUIRE(v < ((__int128)1 << 43) && v > -((__int128)1 << 43), "CRT constant exceeds three limbs");
+  out[2] = (double)(long long)v;
 }
 
 }  // namespace
@@ -164,10 +166,28 @@ CrtConsts make_crt_consts(int n, const int* mod) {
     const int inv = inv_mod((int)(Mi % (unsigned)mod[i]), mod[i]);
     const unsigned __int128 w = Mi * (unsigned)inv;  // < M
     const __int128 ws = w > M / 2 ? (__int128)w - (__int128)M : (__int128)w;
-    limbs42(ws, c.w[i]);
+    limbs(ws, 42, c.w[i]);
   }
-  limbs42((__int128)M, c.M);
+  limbs((__int128)M, 42, c.M);
   c.inv_m_total = 1.0 / (double)M;
+  if (n == kPairModuli) {
+    // r w + r' w' = (M / (m m')) (r m' inv + r' m inv') modulo M, with inv, inv' as in w and w';
+    // the coefficients are taken modulo m m' around 0.
+    for (int i = 0; i < n; ++i) {
+      const int j = i ^ 1;
+      if (j >= n) continue;
+      const int mm = mod[i] * mod[j];
+      const unsigned __int128 Mi = M / (unsigned)mod[i];
+      const int k = (int)((int64_t)mod[j] * inv_mod((int)(Mi % (unsigned)mod[i]), mod[i]) % mm);
+      c.pc[i] = k > mm / 2 ? k - mm : k;
+      limbs((__int128)(M / (unsigned)mm), 27, c.pw[i / 2]);
+    }
+    const int e = n - 1;
+    const unsigned __int128 Me = M / (unsigned)mod[e];
+    const unsigned __int128 w = Me * (unsigned)inv_mod((int)(Me % (unsigned)mod[e]), mod[e]);
+    limbs(w > M / 2 ? (__int128)w - (__int128)M : (__int128)w, 27, c.pw[e / 2]);
+    limbs((__int128)M, 27, c.pM);
+  }
   return c;
 }
 

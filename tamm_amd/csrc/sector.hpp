@@ -19,7 +19,13 @@ struct CrtConsts {
   double w[kMaxModuli][3];  // limbs: w = w2*2^84 + w1*2^42 + w0
   double M[3];
   double inv_m_total;       // 1/M (rounded)
+  // Residues taken in pairs (kPairModuli of them): pair p's two residues combine into one integer
+  // of weight M / (m m'), and the last one keeps its own weight (limbs in base 2^27).
+  int pc[kMaxModuli];            // coefficient of each residue in its pair
+  double pw[kMaxModuli / 2][3];  // weights of the pairs, then of the last residue
+  double pM[3];
 };
+constexpr int kPairModuli = 11;  // the usual count at 35 bits; other counts go residue by residue
 
 // Dense-result region of one sector, for the CRT pass over 32x32 tiles.
 struct CrtSector {
