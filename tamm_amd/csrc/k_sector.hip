@@ -646,9 +646,11 @@ struct InPlaceCursor {
   }
 };
 
-// FP64 sector GEMM: workgroup tile TM x TN over 4 waves (2x2), each (TM/2) x (TN/2) =
-// (TM/32) x (TN/32) v_mfma_f64_16x16x4f64 tiles (128x128 and 128x160 instantiated; the
-// 16-column granularity lets 160 cover N = 800 exactly).  The fragment-major class matrices
+// FP64 sector GEMM: workgroup tile TM x TN over 4 waves (WGM along the rows) of
+// v_mfma_f64_16x16x4f64 tiles.  128x128 and 128x160 (2x2 waves of 64x64 and 64x80) keep the matrix
+// cores 85% busy with two workgroups on a CU; 256x80 (4x1 waves of 64x80) reads more of A per
+// product and runs at 0.93 of that rate, but N = 400 fills five of its tiles where 160 pads it to
+// 480 and 128 to 512 (the choice is the launch model's).  The fragment-major class matrices
 // hold a 16-row tile's k-steps back to back (512 bytes each), so one global_load_lds_dwordx4
 // wave instruction copies two k-steps of one row tile (1 KB).  A stage is those two k-steps
 // for every row tile of A and B; stages go into a ring of NS LDS slots and stage st+NS is
@@ -666,7 +668,7 @@ struct InPlaceCursor {
 // all) is gone, and the GEMM, whose loads are 64-byte pieces of rows now instead of whole KB,
 // loses 4 to 8 %: pack + GEMM of the pp ladder at O=30, V=180 1506 + 4760 -> 0 + 4942 us (61 TF),
 // of 20 + 80 orbitals 149 + 648 -> 0 + 701 us.
-template <int TM, int TN, int NS, bool INP = false>
+template <int TM, int TN, int WGM, int NS, bool INP>
 __global__ __launch_bounds__(256, 2) void k_gemm_f64(const SecTask* __restrict__ tasks, int ntasks,
                                                      const KSeg* __restrict__ segs,
                                                      const double* __restrict__ Ap,
@@ -675,10 +677,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64(const SecTask* __restrict__
   constexpr int AF = TM / 16, BF = TN / 16, SF = AF + BF;  // 1 KB units per stage
   constexpr int FPW = (SF + 3) / 4;
   constexpr int SLOT = SF;
-  constexpr int WTM = TM / 32, WTN = TN / 32;
-  static_assert(WTM * 32 == TM && WTN * 32 == TN, "tile must split over 2x2 waves");
+  constexpr int WGN = 4 / WGM, WTM = AF / WGM, WTN = BF / WGN;
+  static_assert(WTM * WGM * 16 == TM && WTN * WGN * 16 == TN, "tile must split over the waves");
+  // a tile of 2 x 128 rows has at most the entries of two tiles of 128
+  constexpr int IPT = kInPlaceTable * ((TM + 127) / 128);
   __shared__ i4 lds[NS][SLOT * 64];
-  __shared__ int64_t ip_tab[INP ? kInPlaceTable : 1];  // block offsets of the tile's row blocks
+  __shared__ int64_t ip_tab[INP ? IPT : 1];  // block offsets of the tile's row blocks
   const int task = xcd_task(ntasks);
   if (task >= ntasks) return;
   const SecTask tk = tasks[task];
@@ -687,7 +691,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f64(const SecTask* __restrict__
   const uint8_t* B = reinterpret_cast<const uint8_t*>(Bp + tk.b_base);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wv = __builtin_amdgcn_readfirstlane(wave);
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % WGM, wn = wave / WGM;
   const int art = tk.mrows >> 4, brt = tk.nrows >> 4;
   const int64_t akt = tk.a_kpad >> 2, bkt = tk.b_kpad >> 2;  // k-steps per 16-row tile
   const int rt0 = tk.m0 >> 4, ct0 = tk.n0 >> 4;
@@ -1485,7 +1489,11 @@ __global__ __launch_bounds__(256) void k_scatter(const ScatterJob* __restrict__ 
 // (O = 20..60, V = 80..320: K of 256 to 28800, 20 to 53856 tasks), rms 6-10%.  An FP64 task
 // alone on a CU runs as fast as two sharing it, hence one slot.
 struct I8Shape { int tm, tn; double eff; int small; double rate, fixed; int slots; };
+// FP64 256x80 beside 128x160 on the same sectors: 3.0 to 3.1 against 3.3 x 10^13 multiply-adds per
+// second; ladder of 20 + 80 orbitals (N = 400) 677 us in 128x160, 541 in 256x80, of O=30, V=180
+// (N = 450 and 225) 4841 us in 128x160 and 128x128, 4962 in 256x80.
 static const I8Shape kF64Shapes[] = {{128, 128, 1.0, 0, 1.0, 8, 1}, {128, 160, 1.0, 0, 1.0, 8, 1},
+                                     {256, 80, 0.93, 0, 0.93, 8, 1},
                                      {64, 64, 0.5, 64, 0.5, 4, 1}, {32, 32, 0.25, 32, 0.25, 4, 1}};
 static const I8Shape kI8Shapes[] = {{256, 256, 1.0, 0, 1.35, 8, 1}, {512, 160, 1.0, 0, 1.25, 8, 1},
                                     {256, 160, 0.95, 0, 1.20, 6, 2}, {256, 128, 0.82, 0, 1.25, 6, 2},
@@ -1571,7 +1579,7 @@ static bool choose_tile(bool split, int nmod, int64_t mrows, int64_t nrows, int6
 // [x*per, (x+1)*per).  A split-path task is one residue plane of an output tile.  Tasks are
 // laid out so that each XCD's range holds an equal share of the work, longest tasks first,
 // with the M panels (the tasks sharing a tile row of A, and for the split path one plane of
-// it) kept whole on one XCD so they share its L2; short ranges are padded with empty tasks
+// it) on one XCD so they share its L2, but for those at its end; short ranges are padded with empty tasks
 // (mrows = 0).  The same list schedule, simulated
 // on the host, estimates a launch's duration for choosing the split-K factor.
 
@@ -1587,6 +1595,14 @@ static bool choose_tile(bool split, int nmod, int64_t mrows, int64_t nrows, int6
   X(128, 128, 2, 2, 4)    \
   X(64, 64, 2, 2, 4)
 
+// FP64 GEMM instantiations: (TM, TN, WGM, NS, has a kernel that reads A in place).
+#define TMX_F64_KERNELS(X)  \
+  X(128, 128, 2, 4, true)   \
+  X(128, 160, 2, 4, true)   \
+  X(256, 80, 4, 3, true)    \
+  X(64, 64, 2, 4, false)    \
+  X(32, 32, 2, 8, false)
+
 static int gemm_wg_per_cu(bool split, int tm, int tn) {
   static std::mutex mu;
   static std::map<int, int> cache;
@@ -1597,10 +1613,10 @@ static int gemm_wg_per_cu(bool split, int tm, int tn) {
   const void* fn = nullptr;
   int threads = 256;
   if (!split) {
-    if (tm == 128 && tn == 128) fn = reinterpret_cast<const void*>(&k_gemm_f64<128, 128, 4, false>);
-    else if (tm == 128 && tn == 160) fn = reinterpret_cast<const void*>(&k_gemm_f64<128, 160, 4, false>);
-    else if (tm == 64 && tn == 64) fn = reinterpret_cast<const void*>(&k_gemm_f64<64, 64, 4, false>);
-    else if (tm == 32 && tn == 32) fn = reinterpret_cast<const void*>(&k_gemm_f64<32, 32, 8, false>);
+#define TMX_F64_FN(TM_, TN_, WGM_, NS_, INP_) \
+  if (tm == TM_ && tn == TN_) fn = reinterpret_cast<const void*>(&k_gemm_f64<TM_, TN_, WGM_, NS_, false>);
+    TMX_F64_KERNELS(TMX_F64_FN)
+#undef TMX_F64_FN
   } else {
 #define TMX_I8_FN(TM_, TN_, WGM_, WGN_, NS_)                                             \
   if (!fn && tm == TM_ && tn == TN_) {                                                  \
@@ -1647,27 +1663,36 @@ struct TaskGroup {
 };
 constexpr int kXcds = 8, kCusPerXcd = 32;
 
-// Deals the groups, longest first, to the least loaded XCD; bins (when given) receives each XCD's
-// groups in that order.  Returns the list schedule's makespan with `slots` tasks at once per CU.
+// Deals the groups, longest first, to the least loaded XCD, up to an eighth of the work each: a
+// panel that does not fit goes on to the next XCD, since one task too many on an XCD is a round
+// more of its CUs (FP64 ladder of 20 + 80 orbitals in 500 tasks of 256x80, 512 slots: 65 tasks of
+// whole panels on one XCD 807 us, 63 536).  bins (when given) receives each XCD's groups in that
+// order.  Returns the list schedule's makespan with `slots` tasks at once per CU.
 static double deal_groups(std::vector<TaskGroup>& groups, int slots,
-                          std::vector<std::vector<const TaskGroup*>>* bins_out) {
+                          std::vector<std::vector<TaskGroup>>* bins_out) {
   std::stable_sort(groups.begin(), groups.end(),
                    [](const TaskGroup& x, const TaskGroup& y) { return x.cost() > y.cost(); });
-  std::vector<std::vector<const TaskGroup*>> bins(kXcds);
+  std::vector<std::vector<TaskGroup>> bins(kXcds);
   std::vector<double> load(kXcds, 0.0);
-  for (const TaskGroup& g : groups) {
-    const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-    bins[x].push_back(&g);
-    load[x] += g.cost();
-  }
+  double share = 0;
+  for (const TaskGroup& g : groups) share += g.cost() / kXcds;
+  for (TaskGroup g : groups)
+    while (g.b < g.e) {
+      const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+      const double fit = std::ceil((share - load[x]) / g.each - 1e-6);
+      const size_t n = (size_t)std::min((double)(g.e - g.b), std::max(1.0, fit));
+      bins[x].push_back({g.b, g.b + n, g.each});
+      load[x] += bins[x].back().cost();
+      g.b += n;
+    }
   double makespan = 0;
   for (int x = 0; x < kXcds; ++x) {
     std::map<double, size_t> free_at{{0.0, (size_t)(kCusPerXcd * slots)}};  // time -> slots
-    for (const TaskGroup* g : bins[x])
-      for (size_t left = g->e - g->b; left > 0;) {
+    for (const TaskGroup& g : bins[x])
+      for (size_t left = g.e - g.b; left > 0;) {
         const auto it = free_at.begin();
         const size_t n = std::min(it->second, left);
-        const double f = it->first + g->each;
+        const double f = it->first + g.each;
         if ((it->second -= n) == 0) free_at.erase(it);
         free_at[f] += n;
         left -= n;
@@ -1692,12 +1717,12 @@ static void layout_launch(bool split, int tm, int tn, const std::vector<SecTask>
     groups.push_back({i, j, task_seconds(Model::kParts, split, shape, klens[i], slots)});
     i = j;
   }
-  std::vector<std::vector<const TaskGroup*>> bins;
+  std::vector<std::vector<TaskGroup>> bins;
   deal_groups(groups, slots, &bins);
   size_t per = 0;
   for (const auto& b : bins) {
     size_t n = 0;
-    for (const TaskGroup* g : b) n += g->e - g->b;
+    for (const TaskGroup& g : b) n += g.e - g.b;
     per = std::max(per, n);
   }
   SecTask empty;
@@ -1705,8 +1730,8 @@ static void layout_launch(bool split, int tm, int tn, const std::vector<SecTask>
   out->assign(per * kXcds, empty);
   for (int x = 0; x < kXcds; ++x) {
     size_t i = per * x;
-    for (const TaskGroup* g : bins[x])
-      for (size_t t = g->b; t < g->e; ++t) (*out)[i++] = tasks[t];
+    for (const TaskGroup& g : bins[x])
+      for (size_t t = g.b; t < g.e; ++t) (*out)[i++] = tasks[t];
   }
 }
 
@@ -1937,19 +1962,18 @@ static void pack_side(PackSide& side, const double* src, bool split, const Secto
 static void launch_gemm(SectorPlan& sp, const ShapeTasks& st, hipStream_t s, const double* inplace = nullptr) {
   const int grid = (st.ntasks + 7) / 8 * 8;
   if (!sp.split) {
-#define TMX_F64_LAUNCH(TM_, TN_, NS_, INP_)                                                          \
-  hipLaunchKernelGGL((k_gemm_f64<TM_, TN_, NS_, INP_>), dim3(grid), dim3(256), 0, s, st.tasks.as<SecTask>(), \
-                     st.ntasks, sp.ksegs.as<KSeg>(), INP_ ? inplace : sp.A.buf.as<double>(),        \
-                     sp.B.buf.as<double>(), sp.cdense.as<double>(), sp.inplace_args)
-    if (inplace && st.tm == 128 && st.tn == 128) TMX_F64_LAUNCH(128, 128, 4, true);
-    else if (inplace && st.tm == 128 && st.tn == 160) TMX_F64_LAUNCH(128, 160, 4, true);
-    else if (inplace) throw Error(TMX_ERR_INVALID, "no in-place FP64 kernel for the tile shape");
-    else if (st.tm == 128 && st.tn == 128) TMX_F64_LAUNCH(128, 128, 4, false);
-    else if (st.tm == 128 && st.tn == 160) TMX_F64_LAUNCH(128, 160, 4, false);
-    else if (st.tm == 64 && st.tn == 64) TMX_F64_LAUNCH(64, 64, 4, false);
-    else if (st.tm == 32 && st.tn == 32) TMX_F64_LAUNCH(32, 32, 8, false);
-    else throw Error(TMX_ERR_INVALID, "no FP64 kernel for the requested tile shape");
-#undef TMX_F64_LAUNCH
+    bool launched = false;
+#define TMX_F64_CASE(TM_, TN_, WGM_, NS_, INP_)                                                         \
+  if (!launched && st.tm == TM_ && st.tn == TN_ && (INP_ || !inplace)) {                                \
+    auto* const fn = inplace ? &k_gemm_f64<TM_, TN_, WGM_, NS_, INP_> : &k_gemm_f64<TM_, TN_, WGM_, NS_, false>; \
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, s, st.tasks.as<SecTask>(), st.ntasks,              \
+                       sp.ksegs.as<KSeg>(), inplace ? inplace : sp.A.buf.as<double>(),                  \
+                       sp.B.buf.as<double>(), sp.cdense.as<double>(), sp.inplace_args);                 \
+    launched = true;                                                                                    \
+  }
+    TMX_F64_KERNELS(TMX_F64_CASE)
+#undef TMX_F64_CASE
+    TMX_REQUIRE(launched, "no FP64 kernel for the requested tile shape");
   } else {
 #define TMX_I8_LAUNCH(TM_, TN_, WGM_, WGN_, NS_)                                                \
   hipLaunchKernelGGL((k_gemm_i8<TM_, TN_, WGM_, WGN_, NS_>), dim3(grid),                        \
@@ -2165,7 +2189,7 @@ void execute_sector_plan(SectorPlan& sp, const double* A, const double* B, doubl
   // In place unless the operand is constant (its packed copy is made once and kept), the pointer
   // does not allow 16-byte loads, or a shape has no such kernel.
   bool inplace = sp.inplace && !sp.inplace_off && !sp.A.constant && reinterpret_cast<uintptr_t>(A) % 16 == 0;
-  for (const ShapeTasks& st : sp.shapes) inplace = inplace && st.tm == 128;
+  for (const ShapeTasks& st : sp.shapes) inplace = inplace && st.tm >= 128;
   if (!inplace) pack_side(sp.A, A, sp.split, sp, s, pack_ev_a);
   if (ev) TMX_HIP(hipEventRecord(ev[1], s));
   pack_side(sp.B, B, sp.split, sp, s, pack_ev_b);

@@ -399,7 +399,7 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
         }
         ++nrb;
       }
-      // the widest tile (128 rows) keeps its row blocks' offsets in LDS
+      // a tile keeps its row blocks' offsets in LDS (kInPlaceTable for each 128 of its rows)
       for (int64_t m0 = 0; m0 < AM[c].rows && inplace; m0 += 128) {
         const int first = rows[(size_t)(AM[c].growbase + m0)].x;
         const int last = rows[(size_t)(AM[c].growbase + std::min<int64_t>(m0 + 128, AM[c].rows) - 1)].x;

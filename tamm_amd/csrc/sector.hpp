@@ -70,7 +70,7 @@ struct InPlaceA {
   const int2* kblk;     // first (padded) column and columns of each class's K blocks
   const double* zeros;  // 16 zero bytes
 };
-constexpr int kInPlaceTable = 512;  // block offsets of one tile's row blocks, kept in LDS
+constexpr int kInPlaceTable = 512;  // block offsets of 128 rows' blocks, kept in LDS
 
 struct PackSide {
   DevBuf jobs;
