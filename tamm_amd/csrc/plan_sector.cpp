@@ -45,8 +45,14 @@ constexpr int64_t kSplitKPart = 32768;
 // fused-scatter tiles are 32x32) and of 16 on the FP64 path (its MFMA and fragments are 16
 // rows): a class of 8 rows, e.g. one O tile, then streams 2x its bytes through the GEMM, not 4x.
 constexpr int RGRAN_SPLIT = 32, RGRAN_F64 = 16;
-// Shortest split-K part cut for parallelism (columns).
-constexpr int64_t kMinPartK = 1024;
+// Shortest split-K part cut for parallelism (columns).  Where an FP64 product has at most two tiles
+// a CU, and such parts at most four, parts of 128 columns (16 us a task, besides 8 of fill and
+// epilogue) fill the idle CUs, and the launch model is the one fitted to whole stages, which knows
+// that a CU's only task has nearly all of its rate: ring of 20 + 80 orbitals 223 -> 146 us in 3
+// parts of 533, ladder of 17 + 109 orbitals 400 -> 285 in 16 of 371.  Larger products gain less
+// than that model errs by: ring of O=30, V=180 (572 tiles) 801 us whole, 985 in the 2 parts that it
+// takes; L(a,b,i,j) V(a,b,c,d) of 19 + 133 orbitals 818 in 8 parts, 936 in its 4.
+constexpr int64_t kMinPartK = 1024, kMinPartKFew = 128, kFewTiles = 512, kFewTasks = 1024;
 // Most split-K parts of one sector.
 constexpr int64_t kMaxParts = 256;
 // Cost model of an extra split-K part: rate of its scratch traffic.
@@ -624,12 +630,21 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
   // (up to eight) doubled or stepped one by one while that helps -- charging each extra
   // part's partial result (written by the GEMM, read back by the scatter, and for the split
   // path reduced from its residue planes).  A change must gain 3% to be taken.
+  bool few = false;
+  if (!split && parallel_split <= 0 && !cpairs.empty()) {  // a fixed count keeps to parts of kMinPartK
+    const int64_t tiles = sector_tasks(split, make_geoms(make_parts(min_parts), 0, true));
+    few = tiles >= 0 && tiles <= kFewTiles &&
+          sector_tasks(split, make_geoms(make_parts(max_parts), 0, true)) <= kFewTasks;
+    if (few)
+      for (size_t i = 0; i < cpairs.size(); ++i)
+        max_parts[i] = std::max(max_parts[i], std::min<int64_t>(kMaxParts, cpairs[i].cutlen / kMinPartKFew));
+  }
   auto estimate = [&](const std::vector<int64_t>& np) {
     Parts E = make_parts(np);
     const int nm = split ? moduli_for(E.kmax) : 0;
     if (split && nm < 0) return 1e30;
     const double bytes_per_elem = split ? 2.0 * nm + 16.0 : 16.0;
-    return estimate_sector_seconds(split, nm, make_geoms(E, nm, true)) +
+    return estimate_sector_seconds(split, nm, make_geoms(E, nm, true), few) +
            (double)E.extra_elems * bytes_per_elem / kScratchBytesPerSecond;
   };
   std::vector<int64_t> nparts(cpairs.size(), 1);

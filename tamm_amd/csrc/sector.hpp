@@ -192,7 +192,9 @@ void choose_shapes(bool split, int nmod, std::vector<SectorGeom>& geoms, bool tr
 void build_sector_tasks(SectorPlan& sp);
 // Simulated duration of the GEMM launches of these sectors (list schedule of the same layout
 // over the CU slots each kernel's occupancy allows), for choosing the split-K factor.
-double estimate_sector_seconds(bool split, int nmod, const std::vector<SectorGeom>& geoms);
+// few: by the model for launches of few wide FP64 tasks.
+double estimate_sector_seconds(bool split, int nmod, const std::vector<SectorGeom>& geoms, bool few);
+int64_t sector_tasks(bool split, const std::vector<SectorGeom>& geoms);
 // Times every candidate tile shape of every sector on the plan's packed operands (which must
 // be current: run after an execution) and keeps the fastest; records the choices in the tune
 // cache.  Returns the number of sectors whose shape changed.
