@@ -1670,8 +1670,8 @@ constexpr int kXcds = 8, kCusPerXcd = 32;
 // order.  Returns the list schedule's makespan with `slots` tasks at once per CU.
 static double deal_groups(std::vector<TaskGroup>& groups, int slots,
                           std::vector<std::vector<TaskGroup>>* bins_out) {
-  std::stable_sort(groups.begin(), groups.end(),
-                   [](const TaskGroup& x, const TaskGroup& y) { return x.cost() > y.cost(); });
+  const auto longer = [](const TaskGroup& x, const TaskGroup& y) { return x.cost() > y.cost(); };
+  if (!std::is_sorted(groups.begin(), groups.end(), longer)) std::stable_sort(groups.begin(), groups.end(), longer);
   std::vector<std::vector<TaskGroup>> bins(kXcds);
   std::vector<double> load(kXcds, 0.0);
   double share = 0;
@@ -1681,23 +1681,30 @@ static double deal_groups(std::vector<TaskGroup>& groups, int slots,
       const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
       const double fit = std::ceil((share - load[x]) / g.each - 1e-6);
       const size_t n = (size_t)std::min((double)(g.e - g.b), std::max(1.0, fit));
-      bins[x].push_back({g.b, g.b + n, g.each});
-      load[x] += bins[x].back().cost();
+      if (bins_out || bins[x].empty() || bins[x].back().each != g.each)
+        bins[x].push_back({g.b, g.b + n, g.each});
+      else
+        bins[x].back().e += n;  // only counted
+      load[x] += g.each * (double)n;
       g.b += n;
     }
   double makespan = 0;
   for (int x = 0; x < kXcds; ++x) {
     std::map<double, size_t> free_at{{0.0, (size_t)(kCusPerXcd * slots)}};  // time -> slots
-    for (const TaskGroup& g : bins[x])
-      for (size_t left = g.e - g.b; left > 0;) {
+    for (size_t k = 0; k < bins[x].size();) {  // groups of equal tasks in a row as one
+      const double each = bins[x][k].each;
+      size_t left = 0;
+      for (; k < bins[x].size() && bins[x][k].each == each; ++k) left += bins[x][k].e - bins[x][k].b;
+      while (left > 0) {
         const auto it = free_at.begin();
         const size_t n = std::min(it->second, left);
-        const double f = it->first + g.each;
+        const double f = it->first + each;
         if ((it->second -= n) == 0) free_at.erase(it);
         free_at[f] += n;
         left -= n;
         makespan = std::max(makespan, f);
       }
+    }
   }
   if (bins_out) *bins_out = std::move(bins);
   return makespan;
@@ -1770,15 +1777,24 @@ static void tasks_by_shape(const std::vector<SectorGeom>& geoms, int planes,
 // Duration of the launches of these sectors, one per tile shape, by the layout of their tasks.
 static double simulate_launches(bool split, int nmod, const std::vector<SectorGeom>& geoms, Model model) {
   std::map<std::pair<int, int>, std::vector<TaskGroup>> by;
-  for (int pl = 0; pl < (split ? std::max(nmod, 1) : 1); ++pl)
-    for (const SectorGeom& g : geoms) {
-      const I8Shape& sh = shape_of(split, g.tm, g.tn);
-      const int slots = model == Model::kShapes ? sh.slots : gemm_wg_per_cu(split, g.tm, g.tn);
-      const double each = task_seconds(model, split, sh, g.klen, slots);
-      const size_t n = (size_t)((g.nrows + g.tn - 1) / g.tn);
-      std::vector<TaskGroup>& v = by[{g.tm, g.tn}];
-      for (int64_t m0 = 0; m0 < g.mrows; m0 += g.tm) v.push_back({0, n, each});
-    }
+  std::vector<std::pair<double, size_t>> order;  // sectors, their panels' cost
+  for (size_t i = 0; i < geoms.size(); ++i) {
+    const SectorGeom& g = geoms[i];
+    const I8Shape& sh = shape_of(split, g.tm, g.tn);
+    const int slots = model == Model::kShapes ? sh.slots : gemm_wg_per_cu(split, g.tm, g.tn);
+    const double each = task_seconds(model, split, sh, g.klen, slots);
+    const size_t n = (size_t)((g.nrows + g.tn - 1) / g.tn);
+    order.emplace_back(TaskGroup{0, n, each}.cost(), i);
+  }
+  // longest panels first, as deal_groups takes them
+  std::stable_sort(order.begin(), order.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+  for (const auto& [cost, i] : order) {
+    const SectorGeom& g = geoms[i];
+    const size_t n = (size_t)((g.nrows + g.tn - 1) / g.tn);
+    const size_t panels = (size_t)((g.mrows + g.tm - 1) / g.tm) * (split ? std::max(nmod, 1) : 1);
+    std::vector<TaskGroup>& v = by[{g.tm, g.tn}];
+    v.insert(v.end(), panels, {0, n, cost / (double)n});
+  }
   double t = 0;
   for (auto& kv : by) {
     const int slots = model == Model::kShapes ? shape_of(split, kv.first.first, kv.first.second).slots
