@@ -812,9 +812,10 @@ int tmx_contraction_create(const tmx_operand* C, double alpha, const tmx_operand
       // over 1024 workgroups, and the GEMM at its rate or the stages of 1024 columns, e.g. 16 + 64
       // orbitals: ladder 83 us grouped, 65 sector, 79 split; ring 21 / 46 / 58.  FP64 parts may be
       // shorter, but with stages of 256 columns and grouped at 1.25 times ladders of this size
-      // gained 18 us and rings of 25 + 147 or 17 + 109 orbitals lost 8 to 25.  Grouped is taken when modelled twice as fast, or three times on the
-      // split path: a level computes the product of such a ring's four permutations once there
-      // (at 1.5 times, residuals of 30 + 120 orbitals with irreps took 573 us against 534).
+      // gained 18 us and rings of 25 + 147 or 17 + 109 orbitals lost 8 to 25.  Grouped is taken when
+      // modelled twice as fast, or three times on the split path: a level computes the product of
+      // such a ring's four permutations once there (at 1.5 times, residuals of 30 + 120 orbitals
+      // with irreps took 573 us against 534).
       // Larger products stay on the sector path, whose packed operands a constant operand keeps;
       // so do streaming ones (few flops over large tensors), which the model does not cover.
       constexpr double kSmallFlops = 20e9, kSmallElems = 4e7;
