@@ -449,9 +449,8 @@ void launch_bp_f64(const BPTask* tasks, int ntasks, const BPPair* pairs, const B
 // fastest, then Y, then Z (the source's contiguous mode along the lanes), pass through an LDS
 // tile and are written with Y fastest, then X, then Z.  Without X modes both orders are the same
 // and the tile is skipped.  Each thread has its PER source loads and, accumulating, its PER
-// destination loads in flight together: 9 for whole boxes, 1 for the 256-element boxes of small
-// ops.  Boxes span as many modes as it takes to hold about 2304
-// elements: with one workgroup per 32x32 tile or per run of the contiguous mode, amplitude blocks
+// destination loads in flight together: 1, 4 or 9 for boxes of 256, 1024 or 2304 elements.  Boxes
+// span as many modes as it takes to hold that many: with one workgroup per 32x32 tile or per run of the contiguous mode, amplitude blocks
 // of 48x48x16x16 gave each workgroup 256 or 16 elements: over 3.5e7 elements, R(a,b,i,j) -=
 // T(b,a,i,j) went from 9.49 to 0.17 ms (5.0 TB/s) and R(a,b,i,j) -= T(a,b,j,i) from 0.93 to 0.17.
 struct AssignTable {
@@ -470,8 +469,8 @@ __global__ __launch_bounds__(256) void k_assign(const AssignJob* __restrict__ jo
                                                 const double* __restrict__ src,
                                                 double* __restrict__ dst, double scale,
                                                 int is_assign) {
-  __shared__ double tile[kAssignLds];
-  __shared__ AssignTable tx[kAssignSide], ty[kAssignTable], tz[kAssignTable];
+  __shared__ double tile[kAssignLds * PER];
+  __shared__ AssignTable tab[kAssignTable];
   __shared__ int act[MAXR];
   __shared__ int64_t first_s[MAXR], first_d[MAXR];
   const int tid = threadIdx.x;
@@ -519,6 +518,7 @@ __global__ __launch_bounds__(256) void k_assign(const AssignJob* __restrict__ jo
       return t;
     };
     const int XY = X * Y, n = XY * Z;
+    AssignTable *tx = tab, *ty = tx + X, *tz = ty + Y;
     for (int i = tid; i < X; i += 256) tx[i] = entry(0, by, i);
     for (int i = tid; i < Y; i += 256) ty[i] = entry(by, bz, i);
     for (int i = tid; i < Z; i += 256) tz[i] = entry(bz, n_modes, i);
@@ -580,17 +580,77 @@ __global__ __launch_bounds__(256) void k_assign(const AssignJob* __restrict__ jo
   }
 }
 
+// Whole tiles (make_assign_shape without `elems`): 32 x 32 of the source's and the destination's
+// contiguous modes through LDS, or 1024 elements of a shared contiguous mode.  No tables and hardly
+// any index arithmetic, so blocks that fill such tiles, and small ones, run faster than in boxes
+// (the rule is at build_assign_plan): 64x64x64x64 with the last two modes exchanged 41 against 49 us
+// (6.5 TB/s), 3e7 contiguous elements 88 against 191, 17x40000 transposed 4.7 against 7.1.  The
+// order of the tiles: with X first instead of Y, 94x92x60x161 to modes (3,1,2,0) 417 against 373 us.
+__global__ __launch_bounds__(256) void k_assign_tile(const AssignJob* __restrict__ jobs,
+                                                     const AssignUnit* __restrict__ units, int64_t nunits,
+                                                     const AssignShape* __restrict__ shapes,
+                                                     const double* __restrict__ src,
+                                                     double* __restrict__ dst, double scale,
+                                                     int is_assign) {
+  __shared__ double tile[kAssignTile][kAssignTile + 1];
+  const int tid = threadIdx.x, lx = tid & 31, ly = tid >> 5;  // 32 x 8
+  for (int64_t u = blockIdx.x; u < nunits; u += gridDim.x) {
+    const AssignUnit un = units[u];
+    const AssignJob jb = jobs[un.job];
+    const AssignShape& sh = shapes[jb.shape];
+    int64_t sb = jb.src_off, db = jb.dst_off;
+    int left[2] = {1, 1};  // elements of the first two listed modes from the tile's start on
+    uint32_t t = (uint32_t)un.tile;
+    for (int i = 0; i < sh.n; ++i) {  // tiles along Y first, then X, then the rest, fastest first
+      const int k = i <= sh.nx ? sh.nx - i : sh.n + sh.nx - i;
+      const uint32_t q = i + 1 < sh.n ? t / (uint32_t)sh.nt[k] : 0;
+      const int start = (int)(t - q * (uint32_t)sh.nt[k]) * sh.box[k];
+      t = q;
+      sb += start * sh.sstr[k];
+      db += start * sh.dstr[k];
+      if (k < 2) left[k] = sh.ext[k] - start;
+    }
+    const double* sp = src + sb;
+    double* dp = dst + db;
+    if (sh.nx == 0) {
+      for (int e = tid; e < min(kAssignTile * kAssignTile, left[0]); e += 256) {
+        const double r = scale * sp[e];
+        dp[e] = is_assign ? r : dp[e] + r;
+      }
+      continue;
+    }
+    const int64_t ys = sh.sstr[1], xd = sh.dstr[0];  // the other stride of X and of Y is 1
+    double v[4], old[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int y = ly + 8 * k;
+      v[k] = lx < left[0] && y < left[1] ? sp[lx + y * ys] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int x = ly + 8 * k;
+      old[k] = !is_assign && x < left[0] && lx < left[1] ? dp[lx + x * xd] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) tile[ly + 8 * k][lx] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int x = ly + 8 * k;
+      const double r = scale * tile[lx][x];
+      if (x < left[0] && lx < left[1]) dp[lx + x * xd] = is_assign ? r : old[k] + r;
+    }
+    __syncthreads();  // the next tile is written
+  }
+}
+
 void launch_assign(const AssignJob* jobs, const AssignUnit* units, int64_t nunits, int box,
                    const AssignShape* shapes, const double* src, double* dst, double scale,
                    int is_assign, hipStream_t s) {
   if (nunits <= 0) return;
   const int grid = (int)std::min<int64_t>(nunits, 65536);
-  if (box <= 256)
-    hipLaunchKernelGGL(k_assign<1>, dim3(grid), dim3(256), 0, s, jobs, units, nunits, shapes, src, dst,
-                       scale, is_assign);
-  else
-    hipLaunchKernelGGL(k_assign<kAssignElems / 256>, dim3(grid), dim3(256), 0, s, jobs, units, nunits,
-                       shapes, src, dst, scale, is_assign);
+  const auto kernel = box == 0 ? &k_assign_tile : box == 256 ? &k_assign<1> : box == 1024 ? &k_assign<4> : &k_assign<9>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, jobs, units, nunits, shapes, src, dst, scale, is_assign);
   TMX_HIP(hipGetLastError());
 }
 

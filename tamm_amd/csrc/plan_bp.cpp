@@ -1184,7 +1184,7 @@ struct AssignPlan {
   const AssignJob* jobs = nullptr;
   const AssignUnit* units = nullptr;
   int64_t nunits = 0;
-  int box = 0;  // most elements of a unit
+  int box = 0;  // launch_assign's
   // Destination blocks whose source block is zero (element ranges; zero_prefix holds running
   // lengths), zeroed when the op assigns.
   const int64_t *zero_off = nullptr, *zero_prefix = nullptr;
@@ -1229,16 +1229,19 @@ LOperand single_block_operand(int n, const int64_t* dims, const int* labels) {
 
 namespace tmx {
 
-// Tile shape of a block permutation: dims of the destination block and the source stride of
-// each of its modes (see AssignShape).  Boxes hold up to `elems` elements.  X starts as the
+// Box of a block permutation: dims of the destination block and the source stride of each of its
+// modes (see AssignShape).  elems = 0: whole tiles (k_assign_tile), 32 x 32 of the two contiguous
+// modes or 1024 of a shared one.  Else boxes of up to `elems` elements: X starts as the
 // source's contiguous mode and Y as the destination's; each side of fewer than 32 indices takes
 // in the next mode of its own block's order unless that mode is already on the other side (the
 // two sides together are then one contiguous piece of that block), so reads and writes come in
 // runs of at least 256 bytes wherever the blocks allow it.  Z then fills the box with the
-// remaining modes, the destination's fastest first.  A mode is cut into boxes of equal size.
+// remaining modes, the destination's fastest first; where these are too few to fill it, a cut side
+// grows first.  A mode is cut into boxes of equal size.
 static AssignShape make_assign_shape(const std::vector<int64_t>& dd, const std::vector<int64_t>& src_stride,
                                      int64_t elems) {
-  const int64_t side = elems >= kAssignElems ? kAssignSide : 16;
+  const int64_t side = elems == kAssignElems ? 48 : elems == 1024 ? 32 : 16;
+  const int64_t lds = kAssignLds * elems / 256;
   AssignShape sh;
   std::memset(&sh, 0, sizeof(sh));
   std::vector<int64_t> ext, ss;
@@ -1277,27 +1280,48 @@ static AssignShape make_assign_shape(const std::vector<int64_t>& dd, const std::
   std::iota(by_src.begin(), by_src.end(), 0);
   std::sort(by_src.begin(), by_src.end(), [&](int a, int b) { return ss[a] < ss[b]; });
   const bool same = by_src[0] == n - 1;
-  int64_t nx = 1, ny = 1, nz = 1;
-  if (same) {
-    const int64_t run = std::min<int64_t>(kAssignTable, elems);
-    ny = take(Y, 1, n - 1, 1, run);
-    for (int m = n - 2; m >= 0 && ny < 64 && box[Y.back()] == ext[Y.back()]; --m) ny = take(Y, 1, m, ny, run);
+  if (elems == 0) {
+    if (!same) X.push_back(by_src[0]);
+    Y.push_back(n - 1);
+    for (int m = n - 2; m >= 0; --m)
+      if (same || m != X[0]) Z.push_back(m);
+    if (same) box[n - 1] = kAssignTile * kAssignTile;
+    else box[X[0]] = box[n - 1] = kAssignTile;
   } else {
-    nx = take(X, 0, by_src[0], 1, side);
-    ny = take(Y, 1, n - 1, 1, side);
-    for (int k = 1; k < n && nx < std::min<int64_t>(side, 32) && box[X.back()] == ext[X.back()] && role[by_src[k]] < 0; ++k)
-      nx = take(X, 0, by_src[k], nx, side);
-    for (int m = n - 2; m >= 0 && ny < std::min<int64_t>(side, 32) && box[Y.back()] == ext[Y.back()] && role[m] < 0; --m)
-      ny = take(Y, 1, m, ny, side);
-  }
-  const int64_t room = std::min<int64_t>(std::min<int64_t>(elems / (nx * ny), kAssignTable),
-                                         same ? kAssignTable : kAssignLds / (nx * (ny | 1)));
-  for (int m = n - 1; m >= 0; --m) {
-    if (role[m] >= 0) continue;
-    // a side's cut mode, or Z's own, ends the run: later modes stay outside the box
-    if (nz < room) nz = take(Z, 2, m, nz, room);
-    else {
-      Z.push_back(m);
+    int64_t nx = 1, ny = 1, nz = 1;
+    if (same) {
+      const int64_t run = std::min<int64_t>(kAssignRole, elems);
+      ny = take(Y, 1, n - 1, 1, run);
+      for (int m = n - 2; m >= 0 && ny < 64 && box[Y.back()] == ext[Y.back()]; --m) ny = take(Y, 1, m, ny, run);
+    } else {
+      nx = take(X, 0, by_src[0], 1, side);
+      ny = take(Y, 1, n - 1, 1, side);
+      for (int k = 1; k < n && nx < std::min<int64_t>(side, 32) && box[X.back()] == ext[X.back()] && role[by_src[k]] < 0; ++k)
+        nx = take(X, 0, by_src[k], nx, side);
+      for (int m = n - 2; m >= 0 && ny < std::min<int64_t>(side, 32) && box[Y.back()] == ext[Y.back()] && role[m] < 0; --m)
+        ny = take(Y, 1, m, ny, side);
+      int64_t rest = 1;  // what Z could take
+      for (int m = 0; m < n; ++m)
+        if (role[m] < 0) rest = std::min(rest * ext[m], elems);
+      // re-takes a side's last mode up to `cap` when it is cut
+      auto grow = [&](std::vector<int>& v, int r, int64_t have, int64_t cap) {
+        const int m = v.back();
+        if (box[m] == ext[m] || cap < 2 * have) return have;
+        have /= box[m];
+        span += (box[m] - 1) * std::max(ss[m], ds[m]);
+        v.pop_back();
+        return take(v, r, m, have, std::min<int64_t>(cap, kAssignRole));
+      };
+      nx = grow(X, 0, nx, std::min(elems / (ny * rest), lds / ((ny | 1) * rest)));
+      ny = grow(Y, 1, ny, std::min(elems / (nx * rest), lds / (nx * rest) - 1));
+    }
+    const int64_t room = std::min<int64_t>(std::min<int64_t>(elems / (nx * ny), kAssignRole),
+                                           same ? kAssignRole : lds / (nx * (ny | 1)));
+    for (int m = n - 1; m >= 0; --m) {
+      if (role[m] >= 0) continue;
+      // a side's cut mode, or Z's own, ends the run: later modes stay outside the box
+      if (nz < room) nz = take(Z, 2, m, nz, room);
+      else Z.push_back(m);
     }
   }
   sh.nx = (int)X.size();
@@ -1324,13 +1348,9 @@ static AssignShape make_assign_shape(const std::vector<int64_t>& dd, const std::
 std::unique_ptr<AssignPlan> build_assign_plan(const LOperand& D, const LOperand& S, bool zeroing) {
   TMX_REQUIRE(D.labels.size() == S.labels.size(), "assign: label sets differ");
   for (int l : D.labels) TMX_REQUIRE(pos_of(S.labels, l) >= 0, "assign: labels are not a permutation");
-  // Box size: whole boxes once the destination makes 1024 of them (four workgroups per CU),
-  // else boxes of a workgroup's 256 threads, so that small ops spread over the chip (one
-  // 36x36x16x16 block: 7.9 us in 256-element boxes, 9.0 in whole ones).
-  const int64_t elems = D.t->total >= 1024 * kAssignElems ? kAssignElems : 256;
   std::vector<AssignJob> jobs;
-  std::vector<AssignUnit> units;
-  std::vector<AssignShape> shapes;
+  std::vector<std::vector<int64_t>> geoms;  // dims and source strides of the distinct shapes
+  std::vector<int64_t> uses;                // jobs of each
   std::map<std::vector<int64_t>, int> sidx;
   std::vector<int64_t> zoff, zpre{0};
   const size_t r = D.labels.size();
@@ -1359,20 +1379,16 @@ std::unique_ptr<AssignPlan> build_assign_plan(const LOperand& D, const LOperand&
         std::vector<int64_t> key(dd), st(r);
         for (size_t i = 0; i < r; ++i) st[i] = ss[pos_of(S.labels, D.labels[i])];
         key.insert(key.end(), st.begin(), st.end());
-        auto f = sidx.find(key);
-        if (f == sidx.end()) {
-          f = sidx.emplace(key, (int)shapes.size()).first;
-          shapes.push_back(make_assign_shape(dd, st, elems));
+        const auto f = sidx.emplace(key, (int)geoms.size());
+        if (f.second) {
+          geoms.push_back(key);
+          uses.push_back(0);
         }
-        const AssignShape& sh = shapes[f->second];
-        int64_t tiles = 1;
-        for (int i = 0; i < sh.n; ++i) tiles *= sh.nt[i];
-        TMX_REQUIRE(tiles < (1ll << 31), "block too large");
-        for (int64_t t = 0; t < tiles; ++t) units.push_back({(int32_t)jobs.size(), (int32_t)t});
+        ++uses[f.first->second];
         AssignJob jb;
         jb.src_off = soff;
         jb.dst_off = doff;
-        jb.shape = f->second;
+        jb.shape = f.first->second;
         jb.pad = 0;
         jobs.push_back(jb);
       }
@@ -1384,6 +1400,47 @@ std::unique_ptr<AssignPlan> build_assign_plan(const LOperand& D, const LOperand&
     }
     if (d < 0) break;
   }
+  auto make_shapes = [&](int64_t elems) {
+    std::vector<AssignShape> v;
+    for (const std::vector<int64_t>& g : geoms)
+      v.push_back(make_assign_shape({g.begin(), g.begin() + r}, {g.begin() + r, g.end()}, elems));
+    return v;
+  };
+  auto tiles_of = [](const AssignShape& sh) {
+    int64_t n = 1;
+    for (int i = 0; i < sh.n; ++i) n *= sh.nt[i];
+    return n;
+  };
+  // Whole tiles or boxes, by a model of the launch fitted to blocks of 10^2 to 3e8 elements: whole
+  // tiles are cheap (1.6 ns each while all fit the chip at once, then 2.8), boxes of 256, 1024 and
+  // 2304 elements cost 2, 4.5 and 7.5 ns each and a longer start.  48x48x16x16 with the outer two
+  // modes exchanged, in whole tiles and in boxes: 86 and 7 us; 64x64x64x64, the last two: 41 and 49;
+  // 17x40000 transposed: 4.7 and 7.1.
+  struct Cut { int64_t elems; double start, each; };
+  int64_t elems = 0;
+  std::vector<AssignShape> shapes;
+  double best_us = -1;
+  for (const Cut& c : {Cut{0, 3.0, 1.6e-3}, Cut{256, 3.5, 2e-3}, Cut{1024, 4.7, 4.5e-3}, Cut{kAssignElems, 6.3, 7.5e-3}}) {
+    std::vector<AssignShape> v = make_shapes(c.elems);
+    double n = 0;
+    for (size_t i = 0; i < v.size(); ++i) n += (double)tiles_of(v[i]) * (double)uses[i];
+    const double us = c.start + n * c.each + (c.elems == 0 ? std::max(0.0, n - 2048) * 1.2e-3 : 0.0);
+    if (best_us >= 0 && us >= best_us) continue;
+    best_us = us;
+    elems = c.elems;
+    shapes = std::move(v);
+  }
+  std::vector<int64_t> tiles;
+  for (const AssignShape& sh : shapes) {
+    tiles.push_back(tiles_of(sh));
+    TMX_REQUIRE(tiles.back() < (1ll << 31), "block too large");
+  }
+  std::vector<AssignUnit> units;
+  size_t nunits = 0;
+  for (const AssignJob& jb : jobs) nunits += (size_t)tiles[jb.shape];
+  units.reserve(nunits);
+  for (size_t j = 0; j < jobs.size(); ++j)
+    for (int64_t t = 0; t < tiles[jobs[j].shape]; ++t) units.push_back({(int32_t)j, (int32_t)t});
   auto p = std::make_unique<AssignPlan>();
   p->nunits = (int64_t)units.size();
   p->box = (int)elems;

@@ -13,7 +13,7 @@ namespace tmx {
 struct AssignShape {
   int32_t n, nx, ny;
   int32_t ext[MAXR], box[MAXR], nt[MAXR];  // extent, box extent and boxes of each mode
-  int32_t tdiv[MAXR];              // tile / tdiv % nt: the mode's box (tiles in destination order)
+  int32_t tdiv[MAXR];              // boxes: tile / tdiv % nt is the mode's box (destination order)
   int64_t sstr[MAXR], dstr[MAXR];  // source and destination strides
 };
 struct AssignJob {
@@ -23,9 +23,11 @@ struct AssignJob {
 struct AssignUnit {
   int32_t job, tile;
 };
-// Limits of a tile: elements, LDS doubles of a staged tile (X * Z rows of Y | 1), entries of the
-// Y and Z offset tables, and of X and of Y when both are present.
-constexpr int kAssignElems = 2304, kAssignLds = 2560, kAssignTable = 512, kAssignSide = 48;
+// Boxes hold 256, 1024 or 2304 elements.  kAssignLds: LDS doubles of a staged box (X * Z rows of
+// Y | 1) for each 256 of them; kAssignTable: entries of the X, Y and Z offset tables together, where
+// no role has more than kAssignRole indices.  kAssignTile: side of a whole tile, whose square is its
+// elements.
+constexpr int kAssignElems = 2304, kAssignLds = 288, kAssignTable = 520, kAssignRole = 480, kAssignTile = 32;
 
 // xr: XCD task ranges (null: the tasks split into 8 equal contiguous ranges).
 // C-tile shapes of the fused block-pair kernels (rows x columns of one task): 64x64 and 16x256 of
@@ -39,7 +41,7 @@ void launch_bp_f64(const BPTask* tasks, int ntasks, const BPPair* pairs, const B
                    const BPKShape* kshapes, const double* A, const double* B, double* C,
                    double alpha, int is_assign, hipStream_t s, const BPXcd* xr = nullptr,
                    int tile = BP_TILE_64x64);
-// box: most elements of any unit.
+// box: elements of a unit's box (256, 1024 or kAssignElems), or 0 for whole tiles.
 void launch_assign(const AssignJob* jobs, const AssignUnit* units, int64_t nunits, int box,
                    const AssignShape* shapes, const double* src, double* dst, double scale,
                    int is_assign, hipStream_t s);
