@@ -44,7 +44,9 @@ enum {
   TMX_EXEC_SECTOR_F64 = 2,    /* block pairs gathered into dense sector GEMMs, FP64 MFMA */
   TMX_EXEC_SPLIT_I8 = 3,      /* sector GEMMs on int8 residues (Ozaki scheme II), FP64 result */
   TMX_EXEC_AUTO = 4,          /* engine picks, FP64: SECTOR_F64 when eligible and the average
-                                 reduction length per output element is >= 128, else GROUPED_F64 */
+                                 reduction length per output element is >= 128, unless the product
+                                 is small (under 20 GFLOP and 4e7 elements) and its blocks' own
+                                 kernel is modelled clearly faster; else GROUPED_F64 */
   TMX_EXEC_AUTO_SPLIT = 5     /* as AUTO, with SPLIT_I8 in place of SECTOR_F64 where the GEMMs
                                  are MFMA-bound: memory-bound contractions stay FP64, those
                                  with short reductions on the grouped path and those with thin
@@ -224,6 +226,14 @@ int tmx_set_scale_reuse(int on);
 /* Schedule of a sector plan: split-K rounds (most parts of any sector), GEMM launches (one
  * per tile shape) and GEMM tasks; 1, 1, 0 for other plans. */
 int tmx_contraction_schedule_info(tmx_contraction c, int* rounds, int* launches, int64_t* tasks);
+
+/* Kernel a plan has chosen.  tile_rows x tile_cols: the output tile of a workgroup (sector plans: of
+ * their first GEMM launch, in the operand order of the plan; 0 x 0 without launches).  shared_k: 1
+ * when a block-pair plan's workgroups share one tile's reduction over their waves.  in_place: 1 when
+ * the GEMMs of an FP64 sector plan read their first operand from the tensor's blocks, without a
+ * packing pass, at 16-byte addresses. */
+int tmx_contraction_kernel_info(tmx_contraction c, int* tile_rows, int* tile_cols, int* shared_k,
+                                int* in_place);
 
 /* ---- tensor I/O in TAMM's HDF5 format (write_to_disk / read_from_disk,
  * tamm_io.hpp:223-460, :735-980): a 1-D dataset "tensor" of doubles with the tensor's dense

@@ -403,6 +403,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void k_bp_ks(const BPTask* __restrict
   }
 }
 
+bool bp_tile_shares_k(int tile) { return tile == BP_TILE_KS16 || tile == BP_TILE_KS32 || tile == BP_TILE_KS64; }
 int bp_tile_rows(int tile) {
   return tile == BP_TILE_16x256 || tile == BP_TILE_KS16 ? 16 : tile == BP_TILE_KS32 ? 32 : 64;
 }

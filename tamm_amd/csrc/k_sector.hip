@@ -2211,14 +2211,22 @@ static void scatter_stage(const SectorPlan& sp, const SectorPlan& src, double* C
   }
 }
 
+void sector_kernel_info(const SectorPlan& sp, int* rows, int* cols, bool* in_place) {
+  if (rows) *rows = sp.shapes.empty() ? 0 : sp.shapes[0].tm;
+  if (cols) *cols = sp.shapes.empty() ? 0 : sp.shapes[0].tn;
+  *in_place = sp.inplace;
+  for (const ShapeTasks& st : sp.shapes) *in_place = *in_place && st.tm >= 128;  // has such a kernel
+}
+
 void execute_sector_plan(SectorPlan& sp, const double* A, const double* B, double* C, double alpha,
                          hipStream_t s, hipEvent_t* ev, hipEvent_t* gemm_ev, hipEvent_t* pack_ev_a,
                          hipEvent_t* pack_ev_b) {
   if (ev) TMX_HIP(hipEventRecord(ev[0], s));
-  // In place unless the operand is constant (its packed copy is made once and kept), the pointer
-  // does not allow 16-byte loads, or a shape has no such kernel.
-  bool inplace = sp.inplace && !sp.inplace_off && !sp.A.constant && reinterpret_cast<uintptr_t>(A) % 16 == 0;
-  for (const ShapeTasks& st : sp.shapes) inplace = inplace && st.tm >= 128;
+  // In place unless the operand is constant (its packed copy is made once and kept) or the pointer
+  // does not allow 16-byte loads.
+  bool inplace = false;
+  sector_kernel_info(sp, nullptr, nullptr, &inplace);
+  inplace = inplace && !sp.inplace_off && !sp.A.constant && reinterpret_cast<uintptr_t>(A) % 16 == 0;
   if (!inplace) pack_side(sp.A, A, sp.split, sp, s, pack_ev_a);
   if (ev) TMX_HIP(hipEventRecord(ev[1], s));
   pack_side(sp.B, B, sp.split, sp, s, pack_ev_b);

@@ -117,6 +117,9 @@ void set_sector_assign(SectorPlan& sp, bool assign);
 void set_sector_constant(SectorPlan& sp, bool a, bool b);
 // Whether a plan that can read its A operand in place does (default) or packs it.
 void set_sector_inplace(SectorPlan& sp, bool on);
+// Tile of the plan's first GEMM launch, and whether the launches can read an operand A that is not
+// constant and lies at a 16-byte address in place.
+void sector_kernel_info(const SectorPlan& sp, int* rows, int* cols, bool* in_place);
 // Drops what the plan remembers of earlier packings (the next execution packs both operands).
 void forget_sector_packing(SectorPlan& sp);
 // Per-sector tile-shape autotuning on the plan's current packed operands (sector.hpp).

@@ -431,25 +431,29 @@ namespace {
 // longest of its padded work at the shape's full-chip rate (over whole rounds of one workgroup
 // per CU), its serial chains spread over the chip's workgroup slots, and its longest chain.  A
 // chain is a task's fixed time and, for each of its block pairs, a start and a time per `unit`
-// reduction indices.  Fitted to launches of 5 us to 5 ms (blocks of 1 to 1600 rows, 1 to 50
-// pairs, K of 2 to 6400): e.g. a 12 + 24 orbital ladder in blocks of ~6x6, 64x64 112 us, 32x32
+// reduction indices.  Where waves share a reduction, the tasks' fixed time (the sum of the partial
+// tiles and the write) comes on top of the work.  Fitted to launches of 5 us to 5 ms (blocks of 1 to
+// 1600 rows, 1 to 50 pairs, K of 2 to 6400); over 324 of them the shapes taken are 2% above the
+// fastest in the mean.  E.g. a 12 + 24 orbital ladder in blocks of ~6x6, 64x64 112 us, 32x32
 // 28, 16x16 16; a 20 + 80 orbital dense ladder 1250 / 1472 / 2517, split 64x64 1047; a Fock
 // term over blocks of 37 x 2600 with K = 37 340 / 421 / 495 / 610; the adjoint dV += L T of 25 +
-// 110 orbitals (K ~ 40 a pair) 908 / 1398 / 2474 / 1354.
+// 110 orbitals (K ~ 40 a pair) 908 / 1398 / 2474 / 1354, of 16 + 40 (2 pairs of K = 64) 24 / 34 /
+// 42 / 32.
 struct BpShape {
   int tile, slots;
   bool swapped;
   double rate;                  // padded flops per second
   double fixed, pair, per_unit;  // us
   int unit, waves;              // the chain's pair and unit times are shared by `waves`
+  double alone;                 // fixed time of a chain that waits for no other
 };
 constexpr BpShape kBpShapes[] = {
-    {BP_TILE_64x64, 1024, false, 37.6e12, 12.5, 2.5, 1.45, 16, 1},
-    {BP_TILE_16x256, 768, false, 23.4e12, 14.0, 2.5, 1.45, 8, 1},
-    {BP_TILE_16x256, 768, true, 23.4e12, 14.0, 2.5, 1.45, 8, 1},
-    {BP_TILE_KS16, 1280, false, 14.6e12, 4.0, 0.0, 2.0, 64, 4},
-    {BP_TILE_KS32, 1024, false, 29.7e12, 8.0, 0.0, 2.5, 64, 4},
-    {BP_TILE_KS64, 512, false, 52e12, 30.0, 0.0, 9.5, 64, 4},
+    {BP_TILE_64x64, 1024, false, 37.6e12, 12.5, 2.5, 1.45, 16, 1, 4.0},
+    {BP_TILE_16x256, 768, false, 23.4e12, 14.0, 2.5, 1.45, 8, 1, 14.0},
+    {BP_TILE_16x256, 768, true, 23.4e12, 14.0, 2.5, 1.45, 8, 1, 14.0},
+    {BP_TILE_KS16, 1280, false, 14.6e12, 5.0, 0.0, 2.0, 64, 4, 5.0},
+    {BP_TILE_KS32, 1024, false, 24.8e12, 8.0, 0.0, 2.5, 64, 4, 8.0},
+    {BP_TILE_KS64, 512, false, 45e12, 30.0, 0.0, 9.5, 64, 4, 30.0},
 };
 
 struct BpLaunch {  // running sums of one launch
@@ -457,7 +461,8 @@ struct BpLaunch {  // running sums of one launch
   double us(const BpShape& sh) const {
     if (tasks == 0) return 0;
     const double rounds = std::ceil(tasks / 256.0) * 256.0 / tasks;
-    return std::max({flops / sh.rate * 1e6 * rounds, chains / sh.slots, longest});
+    const double work = flops / sh.rate * 1e6 * rounds + (sh.waves > 1 ? sh.fixed * tasks / sh.slots : 0.0);
+    return std::max({work, chains / sh.slots, longest});
   }
 };
 }  // namespace
@@ -506,16 +511,17 @@ static int choose_bp_shape(const LOperand& C, const LOperand& A, const LOperand&
         BpLaunch one;
         one.tasks = tiles;
         one.flops = 2 * tiles * tm * tn * (double)((k + 3) / 4 * 4);
-        one.longest = sh.fixed + (sh.pair + sh.per_unit * (double)((k + sh.unit - 1) / sh.unit)) / sh.waves;
-        one.chains = tiles * one.longest;
+        const double links = (sh.pair + sh.per_unit * (double)((k + sh.unit - 1) / sh.unit)) / sh.waves;
+        one.longest = sh.alone + links;
+        one.chains = tiles * (sh.fixed + links);
         total[s] += one.us(sh);
       }
       const double units = sh.unit == 8 ? u8 : sh.unit == 16 ? u16 : u64;
-      const double chain = sh.fixed + (sh.pair * (double)w.pairs.size() + sh.per_unit * units) / sh.waves;
+      const double links = (sh.pair * (double)w.pairs.size() + sh.per_unit * units) / sh.waves;
       all[s].flops += 2 * tiles * tm * tn * kpad;
       all[s].tasks += tiles;
-      all[s].chains += tiles * chain;
-      all[s].longest = std::max(all[s].longest, chain);
+      all[s].chains += tiles * (sh.fixed + links);
+      all[s].longest = std::max(all[s].longest, sh.alone + links);
     }
   }
   int best = 0;
@@ -809,13 +815,13 @@ int tmx_contraction_create(const tmx_operand* C, double alpha, const tmx_operand
       // Small products: the sector path's launches, packs of blocks of a few hundred elements and
       // few-tile GEMMs over a long K cost more than the block-pair kernel.  Its time here: four
       // launches of 4.5 us (nine on the split path), packs and scatter at 3 TB/s or 6 us a block
-      // over 1024 workgroups, and the GEMM at its rate or the stages of 1024 columns, e.g. 16 + 64
-      // orbitals: ladder 83 us grouped, 65 sector, 79 split; ring 21 / 46 / 58.  FP64 parts may be
-      // shorter, but with stages of 256 columns and grouped at 1.25 times ladders of this size
-      // gained 18 us and rings of 25 + 147 or 17 + 109 orbitals lost 8 to 25.  Grouped is taken when
-      // modelled twice as fast, or three times on the split path: a level computes the product of
-      // such a ring's four permutations once there (at 1.5 times, residuals of 30 + 120 orbitals
-      // with irreps took 573 us against 534).
+      // over 1024 workgroups, and the GEMM at its rate or the stages of 1024 columns.  Over 528
+      // products of 4 to 40 and 20 to 147 orbitals the grouped model is right in the mean (rms
+      // 22%), this one 17 (split) to 45% (FP64) too high, so grouped is taken when modelled 1.6
+      // times as fast (what is taken is then 2% above the faster path in the mean, at 1 and 2 times
+      // 3.5 and 3), e.g. 10 + 100 orbitals: ladder 150 us grouped, 279 sector; 30 + 60: hole-hole 66
+      // and 56.  On the split path 2 times: a level computes the product of a ring's four
+      // permutations once there.
       // Larger products stay on the sector path, whose packed operands a constant operand keeps;
       // so do streaming ones (few flops over large tensors), which the model does not cover.
       constexpr double kSmallFlops = 20e9, kSmallElems = 4e7;
@@ -830,7 +836,7 @@ int tmx_contraction_create(const tmx_operand* C, double alpha, const tmx_operand
         us += split ? std::max(fl / 120e6, avg_k / 64.0) : std::max(fl / 50e6, 0.9 * std::min(avg_k, 1024.0) / 8.0);
         double grouped_us = 0;
         bp_shape = grouped_bp_shape(c->C, c->A, c->B, li, work, &grouped_us);
-        if ((split ? 3.0 : 2.0) * grouped_us < us) sector = false;
+        if ((split ? 2.0 : 1.6) * grouped_us < us) sector = false;
       }
       mode = !sector ? TMX_EXEC_GROUPED_F64
                      : (exec_mode == TMX_EXEC_AUTO_SPLIT ? TMX_EXEC_SPLIT_I8 : TMX_EXEC_SECTOR_F64);
@@ -1029,6 +1035,26 @@ int tmx_contraction_schedule_info(tmx_contraction c, int* rounds, int* launches,
       return;
     }
     sector_schedule_info(*c->sec, rounds, launches, tasks);
+  });
+}
+
+int tmx_contraction_kernel_info(tmx_contraction c, int* tile_rows, int* tile_cols, int* shared_k, int* in_place) {
+  return guarded([&] {
+    TMX_REQUIRE(c, "null contraction");
+    int rows = 0, cols = 0;
+    bool ks = false, inp = false;
+    if (c->sec) {
+      sector_kernel_info(*c->sec, &rows, &cols, &inp);
+      inp = inp && !(c->swapped ? c->const_b : c->const_a);
+    } else {
+      rows = bp_tile_rows(c->bp.tile);
+      cols = bp_tile_cols(c->bp.tile);
+      ks = bp_tile_shares_k(c->bp.tile);
+    }
+    if (tile_rows) *tile_rows = rows;
+    if (tile_cols) *tile_cols = cols;
+    if (shared_k) *shared_k = ks ? 1 : 0;
+    if (in_place) *in_place = inp ? 1 : 0;
   });
 }
 

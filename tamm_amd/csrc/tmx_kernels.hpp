@@ -37,6 +37,7 @@ enum { BP_TILE_64x64 = 0, BP_TILE_16x256 = 1, BP_TILE_KS16 = 2, BP_TILE_KS32 = 3
 constexpr int64_t kBpKsMaxBlock = int64_t(1) << 29;  // byte offsets inside a block in 32 bits
 int bp_tile_rows(int tile);
 int bp_tile_cols(int tile);
+bool bp_tile_shares_k(int tile);  // of k_bp_ks
 void launch_bp_f64(const BPTask* tasks, int ntasks, const BPPair* pairs, const BPCShape* cshapes,
                    const BPKShape* kshapes, const double* A, const double* B, double* C,
                    double alpha, int is_assign, hipStream_t s, const BPXcd* xr = nullptr,

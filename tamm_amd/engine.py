@@ -83,6 +83,7 @@ _PROTOS = [
     ("tmx_set_parallel_split", C.c_int, [C.c_int]),
     ("tmx_set_scale_reuse", C.c_int, [C.c_int]),
     ("tmx_contraction_schedule_info", C.c_int, [vp, i32p, i32p, i64p]),
+    ("tmx_contraction_kernel_info", C.c_int, [vp, i32p, i32p, i32p, i32p]),
     ("tmx_contraction_autotune", C.c_int, [vp, vp, vp, vp, vp, C.POINTER(C.c_int)]),
     ("tmx_tensor_write_hdf5", C.c_int, [vp, vp, C.c_char_p, vp]),
     ("tmx_tensor_read_hdf5", C.c_int, [vp, vp, C.c_char_p, vp]),
@@ -401,6 +402,13 @@ class Contraction:
         r, l, t = C.c_int(), C.c_int(), C.c_int64()
         check(lib().tmx_contraction_schedule_info(self.h, C.byref(r), C.byref(l), C.byref(t)))
         return r.value, l.value, t.value
+
+    def kernel_info(self):
+        """(tile rows, tile columns, reduction shared by a workgroup's waves, first operand read in
+        place) of the kernel the plan has chosen."""
+        r, c, k, p = C.c_int(), C.c_int(), C.c_int(), C.c_int()
+        check(lib().tmx_contraction_kernel_info(self.h, C.byref(r), C.byref(c), C.byref(k), C.byref(p)))
+        return r.value, c.value, bool(k.value), bool(p.value)
 
     def execute(self, stream=None, A: Optional[int] = None, B: Optional[int] = None,
                 Cp: Optional[int] = None) -> None:
