@@ -177,7 +177,10 @@ int tmx_contraction_autotune(tmx_contraction c, const double* A, const double* B
  * calling it again after the operand's values changed makes the next execution pack afresh.
  * Refused (TMX_ERR_STATE) while a captured graph holds the contraction; a graph captured after
  * the packing replays without it.  Block-pair plans read operands in place and ignore the
- * flags.  No counterpart in TAMM, which re-reads every block at every execution. */
+ * flags, except that a small product which AUTO or AUTO_SPLIT had put on the grouped path moves to
+ * the sector path here, for good, where packing the constant operands once makes that faster
+ * (tmx_contraction_info then reports the new mode and workspace).  No counterpart in TAMM, which
+ * re-reads every block at every execution. */
 int tmx_contraction_set_constant(tmx_contraction c, int a_constant, int b_constant);
 /* assign != 0: later executions compute C = alpha*A*B instead of C += alpha*A*B, TAMM's
  * `C(..) = alpha*A(..)*B(..)` (a MultOp with is_assign, multop.hpp:207-239).  TAMM runs it as a

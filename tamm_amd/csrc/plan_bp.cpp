@@ -595,6 +595,12 @@ struct tmx_contraction_s {
   bool const_a = false, const_b = false;
   // tmx_contraction_set_assign: C = alpha*A*B instead of C += alpha*A*B.
   bool assign = false;
+  // AUTO's estimates for a product that it took off the sector path as small (factor 0: none such):
+  // both paths, the packing of A and of B in the sector one, and how much faster grouped must be.
+  struct Small {
+    double factor = 0, grouped_us = 0, sector_us = 0, pack_us[2] = {0, 0};
+    int exec_mode = 0;
+  } small;
   // Holds of live graphs that captured an execution of the contraction (GraphHold).
   std::atomic<int> graph_holds{0};
   const LOperand& sa() const { return swapped ? B : A; }
@@ -754,6 +760,46 @@ static bool sector_eligible(const LabelInfo& li) {
          !li.bouter.empty() && !li.inner.empty();
 }
 
+// Builds the sector plan of a contraction whose label analysis and pair list are li and work;
+// returns the mode it executes in.
+static int build_sector(tmx_contraction_s& c, const LabelInfo& li, const std::vector<CBlockWork>& work,
+                        int mode, int exec_mode) {
+  std::vector<int> ab(li.aouter), ba(li.bouter);
+  ab.insert(ab.end(), li.bouter.begin(), li.bouter.end());
+  ba.insert(ba.end(), li.aouter.begin(), li.aouter.end());
+  c.swapped = c.C.labels != ab && c.C.labels == ba;
+  c.li = c.swapped ? analyse_labels(c.C, c.B, c.A) : li;
+  c.work = c.swapped ? enumerate_pairs(c.C, c.B, c.A, c.li) : work;
+  // AUTO_SPLIT: split precision pays only where the FP64 GEMM is MFMA-bound.  A sector GEMM
+  // reads (mrows + nrows) K operand elements for 2 mrows nrows K flops; below
+  // kMinSplitMN (flops-weighted mrows nrows / (mrows + nrows) of the sectors, e.g. the one-O-
+  // tile classes of Fo(k,i) += U(k,l,c,d) T(c,d,i,l)) both precisions stream their packed
+  // operands at the same HBM rate and split packs 11 bytes per element against 8, so the
+  // planner builds the plan in FP64 (before allocating anything).
+  constexpr double kMinSplitMN = 32;
+  c.sec = build_sector_plan(c.C, c.sa(), c.sb(), c.li, c.work, mode == TMX_EXEC_SPLIT_I8, c.split_bits,
+                            c.parallel_split, exec_mode == TMX_EXEC_AUTO_SPLIT ? kMinSplitMN : 0.0);
+  return mode == TMX_EXEC_SPLIT_I8 && !sector_is_split(*c.sec) ? TMX_EXEC_SECTOR_F64 : mode;
+}
+
+// A small product that AUTO put on the grouped path, once operands of it are constant: the sector
+// path then packs them once, and takes the product over where that is modelled fast enough (ladder of
+// 10 + 100 orbitals with constant V: 212 us grouped, 122 split; of 24 + 96 in tiles of 2 to 6: 587
+// and 206 in FP64).  For good: a level may have given the plan's product to other terms.
+static void reconsider_small(tmx_contraction_s& c) {
+  if (c.small.factor == 0 || c.sec || !(c.const_a || c.const_b)) return;
+  const double us = c.small.sector_us - (c.const_a ? c.small.pack_us[0] : 0) - (c.const_b ? c.small.pack_us[1] : 0);
+  if (c.small.factor * c.small.grouped_us < us || stream_capturing(runtime().stream)) return;
+  const bool split = c.small.exec_mode == TMX_EXEC_AUTO_SPLIT;
+  const LabelInfo li = analyse_labels(c.C, c.A, c.B);
+  try {
+    c.mode = build_sector(c, li, enumerate_pairs(c.C, c.A, c.B, li),
+                          split ? TMX_EXEC_SPLIT_I8 : TMX_EXEC_SECTOR_F64, c.small.exec_mode);
+  } catch (const Error&) {
+    c.sec = nullptr;  // e.g. no memory for the packed copies: it stays grouped
+  }
+}
+
 extern "C" {
 
 int tmx_set_split_bits(int bits) {
@@ -822,25 +868,35 @@ int tmx_contraction_create(const tmx_operand* C, double alpha, const tmx_operand
       // 3.5 and 3), e.g. 10 + 100 orbitals: ladder 150 us grouped, 279 sector; 30 + 60: hole-hole 66
       // and 56.  On the split path 2 times: a level computes the product of a ring's four
       // permutations once there.
-      // Larger products stay on the sector path, whose packed operands a constant operand keeps;
-      // so do streaming ones (few flops over large tensors), which the model does not cover.
+      // Larger products stay on the sector path (so does, from tmx_contraction_set_constant on, what
+      // the sector path runs faster once it has packed a constant operand); so do streaming ones (few flops over large tensors), which the model does not cover.
       constexpr double kSmallFlops = 20e9, kSmallElems = 4e7;
       const double elems = (double)(c->A.t->total + c->B.t->total + c->C.t->total);
       if (sector && fl < kSmallFlops && elems < kSmallElems) {
         const bool split = exec_mode == TMX_EXEC_AUTO_SPLIT;
-        double us = 4.5 * (split ? 9 : 4);
-        for (const LOperand* o : {&c->A, &c->B, &c->C}) {
-          const double bytes = (double)o->t->total * (o == &c->C ? (split ? 27 : 24) : (split ? 27 : 16));
-          us += std::max(bytes / 3e6, 6.0 * (double)o->t->keys.size() / 1024.0);
+        double us = 4.5 * (split ? 9 : 4), pass_us[3];
+        const LOperand* ops[3] = {&c->A, &c->B, &c->C};
+        for (int i = 0; i < 3; ++i) {
+          const double bytes = (double)ops[i]->t->total * (i == 2 ? (split ? 27 : 24) : (split ? 27 : 16));
+          pass_us[i] = std::max(bytes / 3e6, 6.0 * (double)ops[i]->t->keys.size() / 1024.0);
+          us += pass_us[i];
         }
         us += split ? std::max(fl / 120e6, avg_k / 64.0) : std::max(fl / 50e6, 0.9 * std::min(avg_k, 1024.0) / 8.0);
         double grouped_us = 0;
         bp_shape = grouped_bp_shape(c->C, c->A, c->B, li, work, &grouped_us);
-        if ((split ? 2.0 : 1.6) * grouped_us < us) sector = false;
+        const double factor = split ? 2.0 : 1.6;
+        if (factor * grouped_us < us) {
+          sector = false;
+          const double launches = 4.5 * (split ? 3 : 1);
+          c->small = {factor, grouped_us, us, {pass_us[0] + launches, pass_us[1] + launches}, exec_mode};
+        }
       }
       mode = !sector ? TMX_EXEC_GROUPED_F64
                      : (exec_mode == TMX_EXEC_AUTO_SPLIT ? TMX_EXEC_SPLIT_I8 : TMX_EXEC_SECTOR_F64);
     }
+    // One read of each setting: the plan and the fields the autotuner rebuilds it from agree.
+    c->split_bits = g_split_bits.load();
+    c->parallel_split = g_parallel_split.load();
     if (mode == TMX_EXEC_SECTOR_F64 || mode == TMX_EXEC_SPLIT_I8) {
       if (!sector_eligible(li))
         throw Error(TMX_ERR_UNSUPPORTED,
@@ -849,26 +905,7 @@ int tmx_contraction_create(const tmx_operand* C, double alpha, const tmx_operand
       double fl = 0;
       int64_t np = 0;
       for (const CBlockWork& w : work) np += (int64_t)w.pairs.size();
-      std::vector<int> ab(li.aouter), ba(li.bouter);
-      ab.insert(ab.end(), li.bouter.begin(), li.bouter.end());
-      ba.insert(ba.end(), li.aouter.begin(), li.aouter.end());
-      c->swapped = c->C.labels != ab && c->C.labels == ba;
-      c->li = c->swapped ? analyse_labels(c->C, c->B, c->A) : li;
-      c->work = c->swapped ? enumerate_pairs(c->C, c->B, c->A, c->li) : work;
-      // One read of each setting: the plan and the fields the autotuner rebuilds it from agree.
-      c->split_bits = g_split_bits.load();
-      c->parallel_split = g_parallel_split.load();
-      // AUTO_SPLIT: split precision pays only where the FP64 GEMM is MFMA-bound.  A sector GEMM
-      // reads (mrows + nrows) K operand elements for 2 mrows nrows K flops; below
-      // kMinSplitMN (flops-weighted mrows nrows / (mrows + nrows) of the sectors, e.g. the one-O-
-      // tile classes of Fo(k,i) += U(k,l,c,d) T(c,d,i,l)) both precisions stream their packed
-      // operands at the same HBM rate and split packs 11 bytes per element against 8, so the
-      // planner builds the plan in FP64 (before allocating anything).
-      constexpr double kMinSplitMN = 32;
-      c->sec = build_sector_plan(c->C, c->sa(), c->sb(), c->li, c->work, mode == TMX_EXEC_SPLIT_I8,
-                                 c->split_bits, c->parallel_split,
-                                 exec_mode == TMX_EXEC_AUTO_SPLIT ? kMinSplitMN : 0.0);
-      if (mode == TMX_EXEC_SPLIT_I8 && !sector_is_split(*c->sec)) mode = TMX_EXEC_SECTOR_F64;
+      mode = build_sector(*c, li, work, mode, exec_mode);
       // algorithmic flops: sum over triples of 2*M*N*K
       for (const CBlockWork& w : work) {
         std::vector<int64_t> rt0(li.red.size(), 0);
@@ -1082,6 +1119,7 @@ int tmx_contraction_set_constant(tmx_contraction c, int a_constant, int b_consta
                   "which operands are constant");
     c->const_a = a_constant != 0;
     c->const_b = b_constant != 0;
+    reconsider_small(*c);
     if (c->sec) forget_sector_packing(*c->sec);  // the next execution packs afresh
   });
 }

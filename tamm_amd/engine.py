@@ -387,10 +387,13 @@ class Contraction:
         check(lib().tmx_contraction_create(C.byref(self._ops[0].op), alpha, C.byref(self._ops[1].op),
                                            C.byref(self._ops[2].op), mode, C.byref(h)))
         self.h = h.value
+        self._read_info()
+        self.tensors = (Ct, At, Bt)
+
+    def _read_info(self) -> None:
         fl, npairs, ws, md = C.c_double(), C.c_int64(), C.c_int64(), C.c_int()
         check(lib().tmx_contraction_info(self.h, C.byref(fl), C.byref(npairs), C.byref(ws), C.byref(md)))
         self.flops, self.npairs, self.workspace, self.mode = fl.value, npairs.value, ws.value, md.value
-        self.tensors = (Ct, At, Bt)
 
     def split_info(self):
         a, b, n = C.c_int(), C.c_int(), C.c_int()
@@ -434,6 +437,7 @@ class Contraction:
         """Operands whose values never change at their address: packed once and kept
         (calling again drops the kept copies)."""
         check(lib().tmx_contraction_set_constant(self.h, int(a), int(b)))
+        self._read_info()  # an AUTO plan may have moved to the sector path
 
     def set_assign(self, on: bool) -> None:
         """C = alpha*A*B instead of C += alpha*A*B for later executions (TAMM's `C(..) = A*B`)."""
