@@ -129,7 +129,7 @@ int tmx_contraction_execute(tmx_contraction c, const double* A, const double* B,
 int tmx_contraction_info(tmx_contraction c, double* flops, int64_t* npairs,
                          int64_t* workspace_bytes, int* mode);
 /* Split-precision controls (TMX_EXEC_SPLIT_I8): bits kept per operand element and the
- * number of int8 moduli (0 = smallest count that keeps the product exact). */
+ * number of int8 moduli (enough to keep the product exact; 0 for FP64 plans). */
 int tmx_contraction_split_info(tmx_contraction c, int* bits_a, int* bits_b, int* nmoduli);
 int tmx_contraction_destroy(tmx_contraction c);
 /* Executes once with HIP events between the stages on `stream` and returns their durations

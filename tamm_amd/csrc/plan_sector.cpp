@@ -598,6 +598,10 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
     double have = 0;
     int n = 0;
     while (n < kMaxModuli && have < need) have += std::log2((double)kModuli[n++]);
+    // One more than ten, which short reductions make do with: the passes that combine kPairModuli
+    // residues save more than a GEMM plane costs (35 bits, K <= 280: dV += L T of 20 + 160 orbitals
+    // 3406 us with 10, 2478 with 11; hole-hole of 12 + 60 77 and 71).
+    if (n == kPairModuli - 1) have += std::log2((double)kModuli[n++]);
     return have < need ? -1 : n;
   };
   auto make_geoms = [&](const Parts& P, int nmod, bool trial) {
