@@ -1667,9 +1667,12 @@ constexpr int kXcds = 8, kCusPerXcd = 32;
 // panel that does not fit goes on to the next XCD, since one task too many on an XCD is a round
 // more of its CUs (FP64 ladder of 20 + 80 orbitals in 500 tasks of 256x80, 512 slots: 65 tasks of
 // whole panels on one XCD 807 us, 63 536).  bins (when given) receives each XCD's groups in that
-// order.  Returns the list schedule's makespan with `slots` tasks at once per CU.
+// order.  Returns the list schedule's makespan with `slots` tasks at once per CU.  paired: of the one
+// of tasks that share a CU in twos but run as fast there as alone (slots 1): the second 32 tasks of
+// an XCD start beside the first 32, in their order and not when one of them ends (304 tasks of
+// unequal K, ladder of 40 + 160 orbitals in 4 irreps: 417 us as a list, 616 so, 611 measured).
 static double deal_groups(std::vector<TaskGroup>& groups, int slots,
-                          std::vector<std::vector<TaskGroup>>* bins_out) {
+                          std::vector<std::vector<TaskGroup>>* bins_out, bool paired = false) {
   const auto longer = [](const TaskGroup& x, const TaskGroup& y) { return x.cost() > y.cost(); };
   if (!std::is_sorted(groups.begin(), groups.end(), longer)) std::stable_sort(groups.begin(), groups.end(), longer);
   std::vector<std::vector<TaskGroup>> bins(kXcds);
@@ -1691,6 +1694,17 @@ static double deal_groups(std::vector<TaskGroup>& groups, int slots,
   double makespan = 0;
   for (int x = 0; x < kXcds; ++x) {
     std::map<double, size_t> free_at{{0.0, (size_t)(kCusPerXcd * slots)}};  // time -> slots
+    if (paired) {
+      std::vector<double> cu(kCusPerXcd, 0.0);
+      size_t seen = 0;
+      for (TaskGroup& g : bins[x])
+        for (; g.b < g.e && seen < 2 * cu.size(); ++g.b) cu[seen++ % cu.size()] += g.each;
+      free_at.clear();
+      for (double t : cu) {
+        ++free_at[t];
+        makespan = std::max(makespan, t);
+      }
+    }
     for (size_t k = 0; k < bins[x].size();) {  // groups of equal tasks in a row as one
       const double each = bins[x][k].each;
       size_t left = 0;
@@ -1775,7 +1789,8 @@ static void tasks_by_shape(const std::vector<SectorGeom>& geoms, int planes,
 }
 
 // Duration of the launches of these sectors, one per tile shape, by the layout of their tasks.
-static double simulate_launches(bool split, int nmod, const std::vector<SectorGeom>& geoms, Model model) {
+static double simulate_launches(bool split, int nmod, const std::vector<SectorGeom>& geoms, Model model,
+                                bool paired = false) {
   std::map<std::pair<int, int>, std::vector<TaskGroup>> by;
   std::vector<std::pair<double, size_t>> order;  // sectors, their panels' cost
   for (size_t i = 0; i < geoms.size(); ++i) {
@@ -1799,7 +1814,7 @@ static double simulate_launches(bool split, int nmod, const std::vector<SectorGe
   for (auto& kv : by) {
     const int slots = model == Model::kShapes ? shape_of(split, kv.first.first, kv.first.second).slots
                                               : gemm_wg_per_cu(split, kv.first.first, kv.first.second);
-    t += deal_groups(kv.second, slots, nullptr) + (model == Model::kShapes ? 4e-6 : 0.0);
+    t += deal_groups(kv.second, slots, nullptr, paired) + (model == Model::kShapes ? 4e-6 : 0.0);
   }
   return t;
 }
@@ -1817,7 +1832,7 @@ int64_t sector_tasks(bool split, const std::vector<SectorGeom>& geoms) {
 double estimate_sector_seconds(bool split, int nmod, const std::vector<SectorGeom>& geoms, bool few) {
   if (!few) return simulate_launches(split, nmod, geoms, Model::kParts);
   // A CU's only task runs at 0.84 to 0.96 of the rate of two.
-  const double t = simulate_launches(split, nmod, geoms, Model::kShapes);
+  const double t = simulate_launches(split, nmod, geoms, Model::kShapes, true);
   return sector_tasks(split, geoms) <= kXcds * kCusPerXcd ? t / 0.87 : t;
 }
 
