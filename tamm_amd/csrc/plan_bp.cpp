@@ -429,12 +429,11 @@ static void build_bp_plan_as(BPPlan& plan, const LOperand& C, const LOperand& A,
 namespace {
 // Launch model of the fused block-pair kernels, one entry per C-tile shape: the launch takes the
 // longest of its padded work at the shape's full-chip rate (over whole rounds of one workgroup
-// per CU), its serial chains spread over the chip's workgroup slots, and its longest chain.  A
-// chain is a task's fixed time and, for each of its block pairs, a start and a time per `unit`
-// reduction indices.  Where waves share a reduction, the tasks' fixed time (the sum of the partial
-// tiles and the write) comes on top of the work.  Fitted to launches of 5 us to 5 ms (blocks of 1 to
-// 1600 rows, 1 to 50 pairs, K of 2 to 6400); over 324 of them the shapes taken are 2% above the
-// fastest in the mean.  E.g. a 12 + 24 orbital ladder in blocks of ~6x6, 64x64 112 us, 32x32
+// per CU) and the tasks' fixed time (tables, sums, the write) on top, its serial chains spread over
+// the chip's workgroup slots, and its longest chain.  A chain is a task's fixed time and, for each of
+// its block pairs, a start and a time per `unit` reduction indices.  Fitted to launches of 5 us to 5
+// ms (blocks of 1 to 1600 rows, 1 to 50 pairs, K of 2 to 6400); over 324 of them the shapes taken are
+// 2% above the fastest in the mean.  E.g. a 12 + 24 orbital ladder in blocks of ~6x6, 64x64 112 us, 32x32
 // 28, 16x16 16; a 20 + 80 orbital dense ladder 1250 / 1472 / 2517, split 64x64 1047; a Fock
 // term over blocks of 37 x 2600 with K = 37 340 / 421 / 495 / 610; the adjoint dV += L T of 25 +
 // 110 orbitals (K ~ 40 a pair) 908 / 1398 / 2474 / 1354, of 16 + 40 (2 pairs of K = 64) 24 / 34 /
@@ -461,8 +460,7 @@ struct BpLaunch {  // running sums of one launch
   double us(const BpShape& sh) const {
     if (tasks == 0) return 0;
     const double rounds = std::ceil(tasks / 256.0) * 256.0 / tasks;
-    const double work = flops / sh.rate * 1e6 * rounds + (sh.waves > 1 ? sh.fixed * tasks / sh.slots : 0.0);
-    return std::max({work, chains / sh.slots, longest});
+    return std::max({flops / sh.rate * 1e6 * rounds + sh.fixed * tasks / sh.slots, chains / sh.slots, longest});
   }
 };
 }  // namespace
