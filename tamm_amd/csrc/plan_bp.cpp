@@ -1462,11 +1462,9 @@ std::unique_ptr<AssignPlan> build_assign_plan(const LOperand& D, const LOperand&
     }
     if (d < 0) break;
   }
-  auto make_shapes = [&](int64_t elems) {
-    std::vector<AssignShape> v;
-    for (const std::vector<int64_t>& g : geoms)
-      v.push_back(make_assign_shape({g.begin(), g.begin() + r}, {g.begin() + r, g.end()}, elems));
-    return v;
+  auto shape_of_geom = [&](size_t i, int64_t elems) {
+    const std::vector<int64_t>& g = geoms[i];
+    return make_assign_shape({g.begin(), g.begin() + r}, {g.begin() + r, g.end()}, elems);
   };
   auto tiles_of = [](const AssignShape& sh) {
     int64_t n = 1;
@@ -1480,18 +1478,22 @@ std::unique_ptr<AssignPlan> build_assign_plan(const LOperand& D, const LOperand&
   // 17x40000 transposed: 4.7 and 7.1.
   struct Cut { int64_t elems; double start, each; };
   int64_t elems = 0;
-  std::vector<AssignShape> shapes;
   double best_us = -1;
+  const size_t step = (geoms.size() + 31) / 32;  // ragged blocks have thousands of shapes: 32 stand for all
   for (const Cut& c : {Cut{0, 3.0, 1.6e-3}, Cut{256, 3.5, 2e-3}, Cut{1024, 4.7, 4.5e-3}, Cut{kAssignElems, 6.3, 7.5e-3}}) {
-    std::vector<AssignShape> v = make_shapes(c.elems);
-    double n = 0;
-    for (size_t i = 0; i < v.size(); ++i) n += (double)tiles_of(v[i]) * (double)uses[i];
+    double n = 0, seen = 0;
+    for (size_t i = 0; i < geoms.size(); i += step) {
+      n += (double)tiles_of(shape_of_geom(i, c.elems)) * (double)uses[i];
+      seen += (double)uses[i];
+    }
+    if (seen > 0) n *= (double)jobs.size() / seen;
     const double us = c.start + n * c.each + (c.elems == 0 ? std::max(0.0, n - 2048) * 1.2e-3 : 0.0);
     if (best_us >= 0 && us >= best_us) continue;
     best_us = us;
     elems = c.elems;
-    shapes = std::move(v);
   }
+  std::vector<AssignShape> shapes;
+  for (size_t i = 0; i < geoms.size(); ++i) shapes.push_back(shape_of_geom(i, elems));
   std::vector<int64_t> tiles;
   for (const AssignShape& sh : shapes) {
     tiles.push_back(tiles_of(sh));
