@@ -593,10 +593,10 @@ struct tmx_contraction_s {
   bool const_a = false, const_b = false;
   // tmx_contraction_set_assign: C = alpha*A*B instead of C += alpha*A*B.
   bool assign = false;
-  // AUTO's estimates for a product that it took off the sector path as small (factor 0: none such):
-  // both paths, the packing of A and of B in the sector one, and how much faster grouped must be.
+  // AUTO's estimates for a product that it took off the sector path as small (0: none such): both
+  // paths, and the packing of A and of B in the sector one.
   struct Small {
-    double factor = 0, grouped_us = 0, sector_us = 0, pack_us[2] = {0, 0};
+    double grouped_us = 0, sector_us = 0, pack_us[2] = {0, 0};
     int exec_mode = 0;
   } small;
   // Holds of live graphs that captured an execution of the contraction (GraphHold).
@@ -781,13 +781,13 @@ static int build_sector(tmx_contraction_s& c, const LabelInfo& li, const std::ve
 }
 
 // A small product that AUTO put on the grouped path, once operands of it are constant: the sector
-// path then packs them once, and takes the product over where that is modelled fast enough (ladder of
-// 10 + 100 orbitals with constant V: 212 us grouped, 122 split; of 24 + 96 in tiles of 2 to 6: 587
-// and 206 in FP64).  For good: a level may have given the plan's product to other terms.
+// path then packs them once, and takes the product over unless grouped is modelled 1.25 times as
+// fast (ladder of 10 + 100 orbitals with constant V: 212 us grouped, 122 split; of 24 + 96 in tiles
+// of 2 to 6: 587 and 206 in FP64; rings of 10 + 100 stay at 20, split 37).  For good: a level may have given the plan's product to other terms.
 static void reconsider_small(tmx_contraction_s& c) {
-  if (c.small.factor == 0 || c.sec || !(c.const_a || c.const_b)) return;
+  if (c.small.grouped_us == 0 || c.sec || !(c.const_a || c.const_b)) return;
   const double us = c.small.sector_us - (c.const_a ? c.small.pack_us[0] : 0) - (c.const_b ? c.small.pack_us[1] : 0);
-  if (c.small.factor * c.small.grouped_us < us || stream_capturing(runtime().stream)) return;
+  if (1.25 * c.small.grouped_us < us || stream_capturing(runtime().stream)) return;
   const bool split = c.small.exec_mode == TMX_EXEC_AUTO_SPLIT;
   const LabelInfo li = analyse_labels(c.C, c.A, c.B);
   try {
@@ -882,11 +882,10 @@ int tmx_contraction_create(const tmx_operand* C, double alpha, const tmx_operand
         us += split ? std::max(fl / 120e6, avg_k / 64.0) : std::max(fl / 50e6, 0.9 * std::min(avg_k, 1024.0) / 8.0);
         double grouped_us = 0;
         bp_shape = grouped_bp_shape(c->C, c->A, c->B, li, work, &grouped_us);
-        const double factor = split ? 2.0 : 1.6;
-        if (factor * grouped_us < us) {
+        if ((split ? 2.0 : 1.6) * grouped_us < us) {
           sector = false;
           const double launches = 4.5 * (split ? 3 : 1);
-          c->small = {factor, grouped_us, us, {pass_us[0] + launches, pass_us[1] + launches}, exec_mode};
+          c->small = {grouped_us, us, {pass_us[0] + launches, pass_us[1] + launches}, exec_mode};
         }
       }
       mode = !sector ? TMX_EXEC_GROUPED_F64
