@@ -149,7 +149,8 @@ int tmx_contraction_execute_stages(tmx_contraction c, const double* A, const dou
 int tmx_contraction_execute_stages_n(tmx_contraction c, const double* A, const double* B, double* C,
                                      void* stream, float* stage_ms, int n);
 /* Executes once (C += alpha*A*B, as tmx_contraction_execute) and then autotunes the plan:
- * for each sector GEMM every tile shape is timed on the packed operands and the fastest kept,
+ * for each sector GEMM every tile shape is timed on the packed operands (where the plan reads A in
+ * place: every shape that can, reading it in place) and the fastest kept,
  * the plan's current shape unless another is more than 1% faster; for a plan of several
  * sectors the whole GEMM stage is also timed with every sector on one common shape (one
  * launch), which replaces the per-sector choice when more than 1% faster.  Each candidate's

@@ -1505,7 +1505,7 @@ static bool shape_allowed(const I8Shape& sh, int64_t mrows, int64_t nrows) {
 
 // Autotuner cache: sector geometry -> tile shape measured fastest.  Kept in memory and, when
 // TAMM_MI355X_TUNE_FILE names a file, loaded from and saved to that file (one entry per line:
-// "i8 nmod mrows_pad nrows_pad klen tm tn ms").
+// "i8|f64 nmod mrows_pad nrows_pad klen tm tn ms").
 namespace {
 struct TuneKey {
   int split, nmod;
@@ -1514,6 +1514,10 @@ struct TuneKey {
     return std::tie(split, nmod, m, n, k) < std::tie(o.split, o.nmod, o.m, o.n, o.k);
   }
 };
+// FP64 plans have no moduli: 1 there marks the choices of plans that read A in place.
+TuneKey tune_key(bool split, int nmod, int64_t m, int64_t n, int64_t k, bool inplace) {
+  return {split ? 1 : 0, split ? nmod : inplace ? 1 : 0, m, n, k};
+}
 struct TuneVal { int tm, tn; double ms; };
 std::mutex& tune_mu() { static std::mutex* m = new std::mutex; return *m; }
 std::map<TuneKey, TuneVal>& tune_map() {
@@ -1561,12 +1565,17 @@ static void cost_model_tile(const I8Shape (&shapes)[N], int64_t mrows, int64_t n
 
 // Tile shape of one sector: the autotuner's recorded choice for its geometry (returns true), else
 // the least padded area over efficiency.
-static bool choose_tile(bool split, int nmod, int64_t mrows, int64_t nrows, int64_t klen, int* tm, int* tn) {
+static bool choose_tile(bool split, int nmod, int64_t mrows, int64_t nrows, int64_t klen, TileRule rule,
+                        int* tm, int* tn) {
   {
     std::lock_guard<std::mutex> g(tune_mu());
     tune_load_locked();
-    auto it = tune_map().find(TuneKey{split ? 1 : 0, nmod, mrows, nrows, klen});
+    auto it = tune_map().find(tune_key(split, nmod, mrows, nrows, klen, rule.inplace));
     if (it != tune_map().end()) { *tm = it->second.tm; *tn = it->second.tn; return true; }
+  }
+  if (rule.narrow && nrows <= 32) {
+    *tm = *tn = 32;
+    return false;
   }
   if (split) cost_model_tile(kI8Shapes, mrows, nrows, tm, tn);
   else cost_model_tile(kF64Shapes, mrows, nrows, tm, tn);
@@ -1632,6 +1641,14 @@ static int gemm_wg_per_cu(bool split, int tm, int tn) {
   nb = std::max(nb, 1);
   cache[key] = nb;
   return nb;
+}
+
+bool reads_in_place(int tm, int tn) {
+#define TMX_F64_INP(TM_, TN_, WGM_, NS_, INP_) \
+  if (tm == TM_ && tn == TN_) return INP_;
+  TMX_F64_KERNELS(TMX_F64_INP)
+#undef TMX_F64_INP
+  return false;
 }
 
 static const I8Shape& shape_of(bool split, int tm, int tn) {
@@ -1841,14 +1858,14 @@ double estimate_sector_seconds(bool split, int nmod, const std::vector<SectorGeo
 // shape for all sectors at once (thin ones keep the narrow shapes made for them).  Ladder, ring
 // and hole-hole GEMMs of O = 30, V = 180 in split precision: 1774 -> 1543, 351 -> 292 and 128 ->
 // 97 us; FP64 ring 1155 -> 820.
-void choose_shapes(bool split, int nmod, std::vector<SectorGeom>& geoms, bool trial) {
+void choose_shapes(bool split, int nmod, std::vector<SectorGeom>& geoms, bool trial, TileRule rule) {
   const I8Shape* shapes = split ? kI8Shapes : kF64Shapes;
   const size_t n = split ? std::size(kI8Shapes) : std::size(kF64Shapes);
   std::vector<size_t> wide;
   bool tuned = false;
   for (size_t i = 0; i < geoms.size(); ++i) {
     SectorGeom& g = geoms[i];
-    tuned |= choose_tile(split, nmod, g.mrows_pad, g.nrows_pad, g.klen, &g.tm, &g.tn);
+    tuned |= choose_tile(split, nmod, g.mrows_pad, g.nrows_pad, g.klen, rule, &g.tm, &g.tn);
     for (size_t k = 0; k < n; ++k)
       if (shapes[k].tm == g.tm && shapes[k].tn == g.tn && shapes[k].small == 0) wide.push_back(i);
   }
@@ -1873,32 +1890,50 @@ void choose_shapes(bool split, int nmod, std::vector<SectorGeom>& geoms, bool tr
     geoms[wide[i]].tn = best[i].second;
   }
 }
-// XCD-aware task lists of a plan, one per tile shape.
-void build_sector_tasks(SectorPlan& sp) {
+
+std::vector<ShapeTasks> build_sector_tasks(bool split, int nmod, const std::vector<SectorGeom>& geoms,
+                                           double* exec_flops) {
   std::map<int, std::pair<std::vector<SecTask>, std::vector<int64_t>>> by;
-  double exec_flops = 0;
-  tasks_by_shape(sp.geoms, sp.split ? std::max(sp.nmod, 1) : 1, by, &exec_flops);
-  sp.exec_flops = exec_flops;
-  sp.shapes.clear();
+  const int planes = split ? std::max(nmod, 1) : 1;
+  tasks_by_shape(geoms, planes, by, exec_flops);
+  std::vector<ShapeTasks> out;
   for (auto& kv : by) {
     ShapeTasks st;
     st.tm = kv.first / 1000;
     st.tn = kv.first % 1000;
     std::vector<SecTask> laid;
-    layout_launch(sp.split, st.tm, st.tn, kv.second.first, kv.second.second, &laid);
+    layout_launch(split, st.tm, st.tn, kv.second.first, kv.second.second, &laid);
     st.ntasks = (int)laid.size();
-    st.nreal = (int)kv.second.first.size() / (sp.split ? std::max(sp.nmod, 1) : 1);
+    st.nreal = (int)kv.second.first.size() / planes;
     st.tasks = upload(laid);
-    sp.shapes.push_back(std::move(st));
+    out.push_back(std::move(st));
   }
+  return out;
 }
 
-void sector_schedule_info(const SectorPlan& sp, int* rounds, int* launches, int64_t* tasks) {
+// Whether an execution with this operand A reads it in place: not where it is constant (its packed
+// copy is made once and kept) or its address does not allow 16-byte loads.
+static bool runs_in_place(const SectorPlan& sp, const double* A) {
+  return sp.inplace && !sp.A.constant && reinterpret_cast<uintptr_t>(A) % 16 == 0;
+}
+static const std::vector<ShapeTasks>& launches_for(const SectorPlan& sp, const double* A) {
+  return sp.inplace && !runs_in_place(sp, A) ? sp.packed_shapes : sp.shapes;
+}
+
+void sector_schedule_info(const SectorPlan& sp, int* rounds, int* launches, int64_t* tasks, const double* A) {
+  const std::vector<ShapeTasks>& shapes = launches_for(sp, A);
   int64_t n = 0;
-  for (const ShapeTasks& st : sp.shapes) n += st.nreal;
+  for (const ShapeTasks& st : shapes) n += st.nreal;
   if (rounds) *rounds = sp.split_factor;
-  if (launches) *launches = (int)sp.shapes.size();
+  if (launches) *launches = (int)shapes.size();
   if (tasks) *tasks = n;
+}
+
+void sector_kernel_info(const SectorPlan& sp, int* rows, int* cols, bool* in_place) {
+  const std::vector<ShapeTasks>& shapes = launches_for(sp, nullptr);
+  if (rows) *rows = shapes.empty() ? 0 : shapes[0].tm;
+  if (cols) *cols = shapes.empty() ? 0 : shapes[0].tn;
+  if (in_place) *in_place = runs_in_place(sp, nullptr);
 }
 
 static int grid_units(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(n, 8192)); }
@@ -2039,7 +2074,11 @@ static void launch_gemm(SectorPlan& sp, const ShapeTasks& st, hipStream_t s, con
   TMX_HIP(hipGetLastError());
 }
 
-int autotune_sector_plan(SectorPlan& sp, hipStream_t s) {
+int autotune_sector_plan(SectorPlan& sp, const double* A, hipStream_t s) {
+  const bool inplace = runs_in_place(sp, A);
+  const double* const src = inplace ? A : nullptr;
+  const bool second = sp.inplace && !inplace;  // the plan's other launches
+  std::vector<SectorGeom>& geoms = second ? sp.packed_geoms : sp.geoms;
   hipEvent_t e0, e1;
   TMX_HIP(hipEventCreate(&e0));
   TMX_HIP(hipEventCreate(&e1));
@@ -2062,35 +2101,36 @@ int autotune_sector_plan(SectorPlan& sp, hipStream_t s) {
     }
     return best;
   };
+  const I8Shape* shapes = sp.split ? kI8Shapes : kF64Shapes;
+  const size_t nshapes = sp.split ? std::size(kI8Shapes) : std::size(kF64Shapes);
+  auto allowed = [&](const I8Shape& sh, const SectorGeom& g) {
+    return shape_allowed(sh, g.mrows_pad, g.nrows_pad) && (!inplace || reads_in_place(sh.tm, sh.tn));
+  };
+  auto record = [&](const SectorGeom& g) -> TuneVal& {  // tune_mu() held
+    return tune_map()[tune_key(sp.split, sp.nmod, g.mrows_pad, g.nrows_pad, g.klen, inplace)];
+  };
   int changed = 0;
-  for (SectorGeom& g : sp.geoms) {
+  for (SectorGeom& g : geoms) {
     int best_tm = g.tm, best_tn = g.tn;
     double best_ms = 0;
-    const I8Shape* shapes = sp.split ? kI8Shapes : kF64Shapes;
-    const size_t nshapes = sp.split ? sizeof(kI8Shapes) / sizeof(I8Shape) : sizeof(kF64Shapes) / sizeof(I8Shape);
     // The plan's current shape is timed first, and another replaces the best so far only when
     // it is more than 1% faster: shapes within timing noise of each other do not trade places
     // from one run to the next.
     int cur = -1;
     for (size_t si = 0; si < nshapes; ++si)
-      if (shapes[si].tm == g.tm && shapes[si].tn == g.tn && shape_allowed(shapes[si], g.mrows_pad, g.nrows_pad)) cur = (int)si;
+      if (shapes[si].tm == g.tm && shapes[si].tn == g.tn && allowed(shapes[si], g)) cur = (int)si;
     for (int oi = -1; oi < (int)nshapes; ++oi) {
       if (oi >= 0 && oi == cur) continue;
       if (oi < 0 && cur < 0) continue;
       const I8Shape& sh = shapes[oi < 0 ? cur : oi];
-      if (!shape_allowed(sh, g.mrows_pad, g.nrows_pad)) continue;
+      if (!allowed(sh, g)) continue;
       // this sector alone with this shape
       SectorGeom one = g;
       one.tm = sh.tm;
       one.tn = sh.tn;
-      SectorPlan probe_tasks;  // only its task list is used
-      probe_tasks.split = sp.split;
-      probe_tasks.nmod = sp.nmod;
-      probe_tasks.geoms.push_back(one);
-      build_sector_tasks(probe_tasks);
-      const ShapeTasks& st = probe_tasks.shapes.at(0);
-      launch_gemm(sp, st, s);  // warm-up
-      const double ms = min_time_ms(3, [&] { launch_gemm(sp, st, s); });
+      const std::vector<ShapeTasks> st = build_sector_tasks(sp.split, sp.nmod, {one});
+      launch_gemm(sp, st.at(0), s, src);  // warm-up
+      const double ms = min_time_ms(3, [&] { launch_gemm(sp, st[0], s, src); });
       if (best_ms == 0 || ms < best_ms * 0.99) { best_ms = ms; best_tm = sh.tm; best_tn = sh.tn; }
     }
     if (best_tm != g.tm || best_tn != g.tn) ++changed;
@@ -2098,8 +2138,7 @@ int autotune_sector_plan(SectorPlan& sp, hipStream_t s) {
     g.tn = best_tn;
     std::lock_guard<std::mutex> lk(tune_mu());
     tune_load_locked();
-    tune_map()[TuneKey{sp.split ? 1 : 0, sp.nmod, g.mrows_pad, g.nrows_pad, g.klen}] =
-        TuneVal{best_tm, best_tn, best_ms};
+    record(g) = TuneVal{best_tm, best_tn, best_ms};
   }
   // The shapes chosen sector by sector give one launch per distinct shape, run one after
   // another, and were timed with each sector alone.  Sectors side by side in one launch behave
@@ -2107,32 +2146,27 @@ int autotune_sector_plan(SectorPlan& sp, hipStream_t s) {
   // timed with every sector on one common shape, which replaces the per-sector choice when it
   // is more than 1% faster.
   std::vector<std::pair<int, int>> per_sector;
-  for (const SectorGeom& g : sp.geoms) per_sector.emplace_back(g.tm, g.tn);
-  if (sp.geoms.size() > 1) {
+  for (const SectorGeom& g : geoms) per_sector.emplace_back(g.tm, g.tn);
+  if (geoms.size() > 1) {
     auto stage_ms = [&](const std::vector<std::pair<int, int>>& shp) {
-      SectorPlan probe;  // only its task lists are used
-      probe.split = sp.split;
-      probe.nmod = sp.nmod;
-      probe.geoms = sp.geoms;
-      for (size_t i = 0; i < probe.geoms.size(); ++i) {
-        probe.geoms[i].tm = shp[i].first;
-        probe.geoms[i].tn = shp[i].second;
+      std::vector<SectorGeom> probe = geoms;
+      for (size_t i = 0; i < probe.size(); ++i) {
+        probe[i].tm = shp[i].first;
+        probe[i].tn = shp[i].second;
       }
-      build_sector_tasks(probe);
-      for (const ShapeTasks& st : probe.shapes) launch_gemm(sp, st, s);  // warm-up
+      const std::vector<ShapeTasks> launches = build_sector_tasks(sp.split, sp.nmod, probe);
+      for (const ShapeTasks& st : launches) launch_gemm(sp, st, s, src);  // warm-up
       return min_time_ms(3, [&] {
-        for (const ShapeTasks& st : probe.shapes) launch_gemm(sp, st, s);
+        for (const ShapeTasks& st : launches) launch_gemm(sp, st, s, src);
       });
     };
-    const I8Shape* shapes = sp.split ? kI8Shapes : kF64Shapes;
-    const size_t nshapes = sp.split ? sizeof(kI8Shapes) / sizeof(I8Shape) : sizeof(kF64Shapes) / sizeof(I8Shape);
     std::vector<std::pair<int, int>> best = per_sector;
     double best_ms = stage_ms(per_sector);
     for (size_t si = 0; si < nshapes; ++si) {
       bool ok = true;
-      for (const SectorGeom& g : sp.geoms) ok = ok && shape_allowed(shapes[si], g.mrows_pad, g.nrows_pad);
+      for (const SectorGeom& g : geoms) ok = ok && allowed(shapes[si], g);
       if (!ok) continue;
-      const std::vector<std::pair<int, int>> common(sp.geoms.size(), {shapes[si].tm, shapes[si].tn});
+      const std::vector<std::pair<int, int>> common(geoms.size(), {shapes[si].tm, shapes[si].tn});
       const double ms = stage_ms(common);
       if (ms < best_ms * 0.99) {
         best_ms = ms;
@@ -2142,16 +2176,18 @@ int autotune_sector_plan(SectorPlan& sp, hipStream_t s) {
     if (best != per_sector) {
       ++changed;
       std::lock_guard<std::mutex> lk(tune_mu());
-      for (size_t i = 0; i < sp.geoms.size(); ++i) {
-        SectorGeom& g = sp.geoms[i];
+      for (size_t i = 0; i < geoms.size(); ++i) {
+        SectorGeom& g = geoms[i];
         g.tm = best[i].first;
         g.tn = best[i].second;
-        tune_map()[TuneKey{sp.split ? 1 : 0, sp.nmod, g.mrows_pad, g.nrows_pad, g.klen}].tm = g.tm;
-        tune_map()[TuneKey{sp.split ? 1 : 0, sp.nmod, g.mrows_pad, g.nrows_pad, g.klen}].tn = g.tn;
+        record(g).tm = g.tm;
+        record(g).tn = g.tn;
       }
     }
   }
-  build_sector_tasks(sp);
+  double flops = 0;
+  (second ? sp.packed_shapes : sp.shapes) = build_sector_tasks(sp.split, sp.nmod, geoms, &flops);
+  if (!second) sp.exec_flops = flops;
   {
     std::lock_guard<std::mutex> lk(tune_mu());
     tune_save_locked();
@@ -2165,8 +2201,6 @@ void set_sector_constant(SectorPlan& sp, bool a, bool b) {
   sp.A.constant = a;
   sp.B.constant = b;
 }
-
-void set_sector_inplace(SectorPlan& sp, bool on) { sp.inplace_off = !on; }
 
 void forget_sector_packing(SectorPlan& sp) {
   sp.A.packed_src = sp.B.packed_src = nullptr;
@@ -2226,29 +2260,19 @@ static void scatter_stage(const SectorPlan& sp, const SectorPlan& src, double* C
   }
 }
 
-void sector_kernel_info(const SectorPlan& sp, int* rows, int* cols, bool* in_place) {
-  if (rows) *rows = sp.shapes.empty() ? 0 : sp.shapes[0].tm;
-  if (cols) *cols = sp.shapes.empty() ? 0 : sp.shapes[0].tn;
-  *in_place = sp.inplace;
-  for (const ShapeTasks& st : sp.shapes) *in_place = *in_place && st.tm >= 128;  // has such a kernel
-}
-
 void execute_sector_plan(SectorPlan& sp, const double* A, const double* B, double* C, double alpha,
                          hipStream_t s, hipEvent_t* ev, hipEvent_t* gemm_ev, hipEvent_t* pack_ev_a,
                          hipEvent_t* pack_ev_b) {
   if (ev) TMX_HIP(hipEventRecord(ev[0], s));
-  // In place unless the operand is constant (its packed copy is made once and kept) or the pointer
-  // does not allow 16-byte loads.
-  bool inplace = false;
-  sector_kernel_info(sp, nullptr, nullptr, &inplace);
-  inplace = inplace && !sp.inplace_off && !sp.A.constant && reinterpret_cast<uintptr_t>(A) % 16 == 0;
+  const bool inplace = runs_in_place(sp, A);
+  const std::vector<ShapeTasks>& launches = launches_for(sp, A);
   if (!inplace) pack_side(sp.A, A, sp.split, sp, s, pack_ev_a);
   if (ev) TMX_HIP(hipEventRecord(ev[1], s));
   pack_side(sp.B, B, sp.split, sp, s, pack_ev_b);
   if (ev) TMX_HIP(hipEventRecord(ev[2], s));
-  for (size_t i = 0; i < sp.shapes.size(); ++i) {
-    launch_gemm(sp, sp.shapes[i], s, inplace ? A : nullptr);
-    if (gemm_ev && i + 1 < sp.shapes.size()) TMX_HIP(hipEventRecord(gemm_ev[i], s));
+  for (size_t i = 0; i < launches.size(); ++i) {
+    launch_gemm(sp, launches[i], s, inplace ? A : nullptr);
+    if (gemm_ev && i + 1 < launches.size()) TMX_HIP(hipEventRecord(gemm_ev[i], s));
   }
   if (ev) TMX_HIP(hipEventRecord(ev[3], s));
   if (sp.split && sp.nfused == 0 && sp.crt_tiles > 0) {

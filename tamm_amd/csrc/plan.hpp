@@ -84,7 +84,9 @@ void destroy_sector_plan(SectorPlan* sp);
 // Split-K rounds (most parts of any sector), GEMM launches and GEMM tasks of a plan.
 // Row-scale reuse of split packing for executions after this call (process-wide).
 void set_scale_reuse(bool on);
-void sector_schedule_info(const SectorPlan& sp, int* rounds, int* launches, int64_t* tasks);
+// A: of the launches that an execution with this operand A takes (null: a 16-byte address).
+void sector_schedule_info(const SectorPlan& sp, int* rounds, int* launches, int64_t* tasks,
+                          const double* A = nullptr);
 struct SectorPlanDeleter {
   void operator()(SectorPlan* p) const { destroy_sector_plan(p); }
 };
@@ -115,15 +117,13 @@ bool sector_is_split(const SectorPlan& sp);
 void set_sector_assign(SectorPlan& sp, bool assign);
 // Marks the plan's operands constant (packed once per source address and kept) or not.
 void set_sector_constant(SectorPlan& sp, bool a, bool b);
-// Whether a plan that can read its A operand in place does (default) or packs it.
-void set_sector_inplace(SectorPlan& sp, bool on);
-// Tile of the plan's first GEMM launch, and whether the launches can read an operand A that is not
-// constant and lies at a 16-byte address in place.
+// Tile of the plan's first GEMM launch, and whether the launches read A in place, at a 16-byte address
+// and with the constant flags as they are.
 void sector_kernel_info(const SectorPlan& sp, int* rows, int* cols, bool* in_place);
 // Drops what the plan remembers of earlier packings (the next execution packs both operands).
 void forget_sector_packing(SectorPlan& sp);
-// Per-sector tile-shape autotuning on the plan's current packed operands (sector.hpp).
-int autotune_sector_plan(SectorPlan& sp, hipStream_t s);
+// Per-sector tile-shape autotuning (sector.hpp).
+int autotune_sector_plan(SectorPlan& sp, const double* A, hipStream_t s);
 void sector_split_info(const SectorPlan& sp, int* bits_a, int* bits_b, int* nmod);
 
 }  // namespace tmx

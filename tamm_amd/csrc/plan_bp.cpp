@@ -681,11 +681,15 @@ static void run_bp(const tmx_contraction_s* c, const double* A, const double* B,
   }
 }
 
+static void set_constant_flags(const tmx_contraction_s* c, SectorPlan& sp) {
+  set_sector_constant(sp, c->swapped ? c->const_b : c->const_a, c->swapped ? c->const_a : c->const_b);
+}
+
 // pack_ev: optional two events around the main packing pass of the call's A operand.
 static void run_sector(const tmx_contraction_s* c, SectorPlan& sp, const double* A, const double* B,
                        double* C, double alpha, hipStream_t s, hipEvent_t* ev = nullptr,
                        hipEvent_t* gemm_ev = nullptr, hipEvent_t* pack_ev = nullptr) {
-  set_sector_constant(sp, c->swapped ? c->const_b : c->const_a, c->swapped ? c->const_a : c->const_b);
+  set_constant_flags(c, sp);
   set_sector_assign(sp, c->assign);
   if (c->swapped) std::swap(A, B);
   execute_sector_plan(sp, A, B, C, alpha, s, ev, gemm_ev, c->swapped ? nullptr : pack_ev,
@@ -745,10 +749,8 @@ static int autotune_split_k(tmx_contraction_s* c, const double* A, const double*
     }
   }
   if (!best) return 0;
-  set_sector_inplace(*best, false);
   run_sector(c, *best, A, B, sc, 1.0, s);
-  autotune_sector_plan(*best, s);
-  set_sector_inplace(*best, true);
+  autotune_sector_plan(*best, c->swapped ? B : A, s);
   c->sec = std::move(best);
   return 1;
 }
@@ -951,10 +953,8 @@ int tmx_contraction_autotune(tmx_contraction c, const double* A, const double* B
                   "rebuilt under them): destroy them before autotuning");
     int n = 0;
     if (c->mode == TMX_EXEC_SECTOR_F64 || c->mode == TMX_EXEC_SPLIT_I8) {
-      set_sector_inplace(*c->sec, false);  // the shapes are timed on packed operands
       run_sector(c, *c->sec, A, B, C, c->alpha, s);
-      n = autotune_sector_plan(*c->sec, s);
-      set_sector_inplace(*c->sec, true);
+      n = autotune_sector_plan(*c->sec, c->swapped ? B : A, s);
       if (c->parallel_split == 0) n += autotune_split_k(c, A, B, s);
     } else {
       const int rc = tmx_contraction_execute(c, A, B, C, stream);
@@ -986,7 +986,8 @@ static void execute_stages(tmx_contraction c, const double* A, const double* B, 
   if (c->mode == TMX_EXEC_SECTOR_F64 || c->mode == TMX_EXEC_SPLIT_I8) {
     int64_t t = 0;
     int r = 0;
-    sector_schedule_info(*c->sec, &r, &launches, &t);
+    set_constant_flags(c, *c->sec);
+    sector_schedule_info(*c->sec, &r, &launches, &t, c->swapped ? B : A);
     const bool per_launch = launches > 1 && launches <= kMaxLaunchEvents + 1;
     run_sector(c, *c->sec, A, B, C, c->alpha, s, ev, per_launch ? ev + 5 : nullptr, pack_ev);
     if (!per_launch) launches = 1;
@@ -1079,7 +1080,6 @@ int tmx_contraction_kernel_info(tmx_contraction c, int* tile_rows, int* tile_col
     bool ks = false, inp = false;
     if (c->sec) {
       sector_kernel_info(*c->sec, &rows, &cols, &inp);
-      inp = inp && !(c->swapped ? c->const_b : c->const_a);
     } else {
       rows = bp_tile_rows(c->bp.tile);
       cols = bp_tile_cols(c->bp.tile);
@@ -1117,7 +1117,9 @@ int tmx_contraction_set_constant(tmx_contraction c, int a_constant, int b_consta
     c->const_a = a_constant != 0;
     c->const_b = b_constant != 0;
     reconsider_small(*c);
-    if (c->sec) forget_sector_packing(*c->sec);  // the next execution packs afresh
+    if (!c->sec) return;
+    set_constant_flags(c, *c->sec);
+    forget_sector_packing(*c->sec);  // the next execution packs afresh
   });
 }
 

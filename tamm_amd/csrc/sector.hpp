@@ -131,8 +131,12 @@ struct SectorPlan {
   std::vector<SectorGeom> geoms;
   std::vector<ShapeTasks> shapes;
   DevBuf ksegs;
-  bool inplace = false;      // A may be read in place (inplace_args)
-  bool inplace_off = false;  // switched off (the autotuner times GEMMs on packed operands)
+  // A is read in place (inplace_args) by the launches of `shapes`, which all have such kernels; an
+  // execution that packs it all the same (constant, or at an address without 16-byte alignment)
+  // takes packed_shapes, of packed_geoms.  Else `shapes` are the only ones.
+  bool inplace = false;
+  std::vector<SectorGeom> packed_geoms;
+  std::vector<ShapeTasks> packed_shapes;
   InPlaceA inplace_args{};
   DevBuf inplace_buf;
   DevBuf cdense;        // dense FP64 result, row-major per sector (ld = nrows_pad)
@@ -182,23 +186,32 @@ struct SectorPlan {
   double mn_intensity = 0;
 };
 
+// How the tiles of a plan's GEMMs are chosen.  inplace: A is read in place (the autotuner's choices
+// for such plans are kept apart).  narrow: sectors of at most 32 columns take 32x32 tiles.
+struct TileRule {
+  bool inplace = false, narrow = false;
+};
 // Tile shapes (rows of A x rows of B per workgroup) of a plan's sector GEMMs: the autotuner's
 // recorded choices for the geometries if there are any, else by the launch model.  trial: sector
 // by sector only (part counts that are costed, not built).
-void choose_shapes(bool split, int nmod, std::vector<SectorGeom>& geoms, bool trial);
-// Builds the GEMM task lists of all sectors from their geometry and tile shapes, one launch
-// per shape, each laid out for the XCD-aware workgroup mapping (balanced XCD ranges, longest
-// tasks first, padded with empty tasks), and the plan's executed-flop count.
-void build_sector_tasks(SectorPlan& sp);
+void choose_shapes(bool split, int nmod, std::vector<SectorGeom>& geoms, bool trial, TileRule rule);
+// True when a tile shape has a kernel that reads A in place.
+bool reads_in_place(int tm, int tn);
+// GEMM task lists of sectors from their geometry and tile shapes, one launch per shape, each laid out
+// for the XCD-aware workgroup mapping (balanced XCD ranges, longest tasks first, padded with empty
+// tasks).  exec_flops (may be null): executed flops, padding included.
+std::vector<ShapeTasks> build_sector_tasks(bool split, int nmod, const std::vector<SectorGeom>& geoms,
+                                           double* exec_flops = nullptr);
 // Simulated duration of the GEMM launches of these sectors (list schedule of the same layout
 // over the CU slots each kernel's occupancy allows), for choosing the split-K factor.
 // few: by the model for launches of few wide FP64 tasks.
 double estimate_sector_seconds(bool split, int nmod, const std::vector<SectorGeom>& geoms, bool few);
 int64_t sector_tasks(bool split, const std::vector<SectorGeom>& geoms);
-// Times every candidate tile shape of every sector on the plan's packed operands (which must
-// be current: run after an execution) and keeps the fastest; records the choices in the tune
-// cache.  Returns the number of sectors whose shape changed.
-int autotune_sector_plan(SectorPlan& sp, hipStream_t s);
+// Times every candidate tile shape of every sector as an execution with this A runs it: on the
+// operands packed by the last one, which must have been with the same A, or reading A in place (then
+// among the shapes that can).  Keeps the fastest and records the choices in the tune cache.  Returns
+// the number of sectors whose shape changed.
+int autotune_sector_plan(SectorPlan& sp, const double* A, hipStream_t s);
 // CRT constants for the first n moduli (host, exact 128-bit integer arithmetic).
 CrtConsts make_crt_consts(int n, const int* moduli);
 
