@@ -1939,8 +1939,11 @@ void sector_kernel_info(const SectorPlan& sp, int* rows, int* cols, bool* in_pla
 static int grid_units(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(n, 8192)); }
 // A packing or CRT scatter pass: a workgroup per unit (a workgroup that loops waits for its own stores before it
 // loads again: split V(a,b,c,d) of 50 + 320 orbitals 3871 us with 8192, 3654 so;
-// CRT scatter of 3.9e8 results 1865 and 1801), or at most `cap`.
-static int grid_full(int64_t n, int64_t cap = 1ll << 30) { return (int)std::min(xcd_rounds(n), cap); }
+// CRT scatter of 3.9e8 results 1865 and 1801), or at most `cap`, whose workgroups loop.  HIP takes fewer
+// than 2^32 work items a launch, which a tensor of 2^24 blocks of a few elements would exceed.
+constexpr int64_t kMaxGrid = 1ll << 23;
+static_assert(kMaxGrid % 8 == 0 && kMaxGrid * 256 < 1ll << 32);
+static int grid_full(int64_t n, int64_t cap = kMaxGrid) { return (int)std::min(xcd_rounds(n), cap); }
 
 static std::atomic<bool> g_scale_reuse{true};  // tmx_set_scale_reuse, read at execution
 constexpr int kScaleReuseBackoff = 8;
@@ -1979,7 +1982,7 @@ static void pack_side(PackSide& side, const double* src, bool split, const Secto
   // smaller (it returns at once unless enabled, and its blocks loop over the units);
   // zero_flag: cleared by the first block of the first launch.
   auto pack = [&](unsigned long long* maxout, const int* gate, int* zero_flag) {
-    const int64_t cap = gate ? 1024 : 1ll << 30;
+    const int64_t cap = gate ? 1024 : kMaxGrid;
     if (side.nunits > 0) {
       hipLaunchKernelGGL(k_pack<2>, dim3(grid_full(side.nunits, cap)), dim3(256), 0, s,
                          side.jobs.as<PackJob>(), side.units.as<TileUnit>(), side.nunits, src, nullptr,
