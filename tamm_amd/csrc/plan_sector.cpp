@@ -197,10 +197,11 @@ CrtConsts make_crt_consts(int n, const int* mod) {
   return c;
 }
 
-SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOperand& B,
+// lean: least memory instead of time.
+static SectorPlanPtr build_plan(const LOperand& C, const LOperand& A, const LOperand& B,
                                 const LabelInfo& li, const std::vector<CBlockWork>& work,
                                 bool split, int split_bits, int parallel_split,
-                                double min_split_mn) {
+                                double min_split_mn, bool lean) {
   SectorPlanPtr sp(new SectorPlan());
   sp->split = split;
   const std::vector<int>& ML = li.aouter;
@@ -601,7 +602,7 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
     // One more than ten, which short reductions make do with: the passes that combine kPairModuli
     // residues save more than a GEMM plane costs (35 bits, K <= 280: dV += L T of 20 + 160 orbitals
     // 3406 us with 10, 2478 with 11; hole-hole of 12 + 60 77 and 71).
-    if (n == kPairModuli - 1) have += std::log2((double)kModuli[n++]);
+    if (n == kPairModuli - 1 && !lean) have += std::log2((double)kModuli[n++]);
     return have < need ? -1 : n;
   };
   // 32x32 tiles for sectors of at most 32 columns whose A is packed, where there are enough of them:
@@ -648,7 +649,7 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
   // part's partial result (written by the GEMM, read back by the scatter, and for the split
   // path reduced from its residue planes).  A change must gain 3% to be taken.
   bool few = false;
-  if (!split && parallel_split <= 0 && !cpairs.empty()) {  // a fixed count keeps to parts of kMinPartK
+  if (!split && !lean && parallel_split <= 0 && !cpairs.empty()) {  // a fixed count keeps to parts of kMinPartK
     const int64_t tiles = sector_tasks(split, make_geoms(make_parts(min_parts), 0, true));
     few = tiles >= 0 && tiles <= kFewTiles &&
           sector_tasks(split, make_geoms(make_parts(max_parts), 0, true)) <= kFewTasks;
@@ -667,7 +668,7 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
   std::vector<int64_t> nparts(cpairs.size(), 1);
   if (parallel_split > 0) {
     std::fill(nparts.begin(), nparts.end(), (int64_t)parallel_split);
-  } else if (!cpairs.empty()) {
+  } else if (!cpairs.empty() && !lean) {  // lean: as few as there may be
     double cur = estimate(nparts);
     std::vector<int64_t> best = nparts;
     for (int64_t pfac : {2, 3, 4, 6, 8, 16, 32, 64}) {
@@ -980,6 +981,19 @@ SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOpe
                      sp->B.jobs.bytes + sp->A.rowmax.bytes * 3 +
                      sp->B.rowmax.bytes * 3);
   return sp;
+}
+
+SectorPlanPtr build_sector_plan(const LOperand& C, const LOperand& A, const LOperand& B,
+                                const LabelInfo& li, const std::vector<CBlockWork>& work,
+                                bool split, int split_bits, int parallel_split,
+                                double min_split_mn) {
+  try {
+    return build_plan(C, A, B, li, work, split, split_bits, parallel_split, min_split_mn, false);
+  } catch (const Error& e) {
+    if (e.code != TMX_ERR_OOM) throw;
+  }
+  // Scratch for parts or planes that only save time must not fail a plan that fits without it.
+  return build_plan(C, A, B, li, work, split, split_bits, parallel_split, min_split_mn, true);
 }
 
 int64_t sector_workspace_bytes(const SectorPlan& sp) { return sp.ws; }
