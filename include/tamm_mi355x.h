@@ -213,7 +213,8 @@ int tmx_set_split_bits(int bits);
  * model choose per sector, up to 256 parts (simulated XCD list schedule of the GEMM tasks
  * against the traffic of the extra partial results, which the scatter sums into C in one
  * pass); 1..16 fixes the count (still at least what the split path's
- * exact int32 accumulation needs, and parts of at least 1024 columns).  Results agree to the
+ * exact int32 accumulation needs, and parts of at least 1024 columns, every K block counted as a
+ * whole number of 32 (FP64) or 64 of them).  Results agree to the
  * mode's tolerance for every count (FP64 sums are reassociated).  A contraction keeps the
  * value it was created with; created with a fixed count, its autotuner keeps that count.
  * No counterpart in TAMM. */

@@ -1685,9 +1685,10 @@ constexpr int kXcds = 8, kCusPerXcd = 32;
 // more of its CUs (FP64 ladder of 20 + 80 orbitals in 500 tasks of 256x80, 512 slots: 65 tasks of
 // whole panels on one XCD 807 us, 63 536).  bins (when given) receives each XCD's groups in that
 // order.  Returns the list schedule's makespan with `slots` tasks at once per CU.  paired: of the one
-// of tasks that share a CU in twos but run as fast there as alone (slots 1): the second 32 tasks of
-// an XCD start beside the first 32, in their order and not when one of them ends (304 tasks of
-// unequal K, ladder of 40 + 160 orbitals in 4 irreps: 417 us as a list, 616 so, 611 measured).
+// of tasks that share a CU in twos, but run there hardly faster than alone (slots 1): the second 32
+// tasks of an XCD start beside the first 32, in their order and not when one of them ends (304 tasks
+// of unequal K, ladder of 40 + 160 orbitals in 4 irreps: 417 us as a list, 616 so, 611 measured).
+constexpr double kAloneRate = 0.87;  // of two tasks: 0.84 to 0.96
 static double deal_groups(std::vector<TaskGroup>& groups, int slots,
                           std::vector<std::vector<TaskGroup>>* bins_out, bool paired = false) {
   const auto longer = [](const TaskGroup& x, const TaskGroup& y) { return x.cost() > y.cost(); };
@@ -1712,12 +1713,14 @@ static double deal_groups(std::vector<TaskGroup>& groups, int slots,
   for (int x = 0; x < kXcds; ++x) {
     std::map<double, size_t> free_at{{0.0, (size_t)(kCusPerXcd * slots)}};  // time -> slots
     if (paired) {
-      std::vector<double> cu(kCusPerXcd, 0.0);
+      std::vector<double> cu[2] = {std::vector<double>(kCusPerXcd, 0.0), std::vector<double>(kCusPerXcd, 0.0)};
       size_t seen = 0;
       for (TaskGroup& g : bins[x])
-        for (; g.b < g.e && seen < 2 * cu.size(); ++g.b) cu[seen++ % cu.size()] += g.each;
+        for (; g.b < g.e && seen < 2 * kCusPerXcd; ++g.b, ++seen) cu[seen / kCusPerXcd][seen % kCusPerXcd] = g.each;
       free_at.clear();
-      for (double t : cu) {
+      for (int i = 0; i < kCusPerXcd; ++i) {
+        const double lo = std::min(cu[0][i], cu[1][i]), hi = std::max(cu[0][i], cu[1][i]);
+        const double t = 2 * lo + (hi - lo) / kAloneRate;
         ++free_at[t];
         makespan = std::max(makespan, t);
       }
@@ -1848,9 +1851,7 @@ int64_t sector_tasks(bool split, const std::vector<SectorGeom>& geoms) {
 
 double estimate_sector_seconds(bool split, int nmod, const std::vector<SectorGeom>& geoms, bool few) {
   if (!few) return simulate_launches(split, nmod, geoms, Model::kParts);
-  // A CU's only task runs at 0.84 to 0.96 of the rate of two.
-  const double t = simulate_launches(split, nmod, geoms, Model::kShapes, true);
-  return sector_tasks(split, geoms) <= kXcds * kCusPerXcd ? t / 0.87 : t;
+  return simulate_launches(split, nmod, geoms, Model::kShapes, true);
 }
 
 // Sectors of different shapes are launches of their own, each with a last partial round and the

@@ -45,14 +45,16 @@ constexpr int64_t kSplitKPart = 32768;
 // fused-scatter tiles are 32x32) and of 16 on the FP64 path (its MFMA and fragments are 16
 // rows): a class of 8 rows, e.g. one O tile, then streams 2x its bytes through the GEMM, not 4x.
 constexpr int RGRAN_SPLIT = 32, RGRAN_F64 = 16;
-// Shortest split-K part cut for parallelism (columns).  Where an FP64 product has at most two tiles
-// a CU, and such parts at most four, parts of 128 columns (16 us a task, besides 8 of fill and
+// Shortest split-K part cut for parallelism: kMinPartK counts every K block as a whole number of 64
+// (split) or 32 columns, so that blocks of a few columns, whose packing and scatter weigh more, may be
+// cut further; kMinPartKFew the columns that the GEMM runs.  Where an FP64 product has at most two tiles
+// a CU, and such parts at most four, parts of 64 columns (8 us a task, besides 8 of fill and
 // epilogue) fill the idle CUs, and the launch model is the one fitted to whole stages, which knows
 // that a CU's only task has nearly all of its rate: ring of 20 + 80 orbitals 223 -> 146 us in 3
 // parts of 533, ladder of 17 + 109 orbitals 400 -> 285 in 16 of 371.  Larger products gain less
 // than that model errs by: ring of O=30, V=180 (572 tiles) 801 us whole, 985 in the 2 parts that it
 // takes; L(a,b,i,j) V(a,b,c,d) of 19 + 133 orbitals 818 in 8 parts, 936 in its 4.
-constexpr int64_t kMinPartK = 1024, kMinPartKFew = 128, kFewTiles = 512, kFewTasks = 1024;
+constexpr int64_t kMinPartK = 1024, kMinPartKFew = 64, kFewTiles = 512, kFewTasks = 1024;
 // Most split-K parts of one sector.
 constexpr int64_t kMaxParts = 256;
 // Cost model of an extra split-K part: rate of its scratch traffic.
@@ -520,7 +522,7 @@ static SectorPlanPtr build_plan(const LOperand& C, const LOperand& A, const LOpe
   // region (rows_pad(A) x rows_pad(B), a whole number of 32x32 tiles) and is scattered into C in
   // its own round.
   struct Sector { int mc, nc; int64_t c_base; int seg_b, seg_e; int64_t klen; int round; };
-  // cutlen: the K blocks' columns, each padded to 64 (split) or 32: bounds the part count.
+  // cutlen: the K blocks' columns, each padded to 64 (split) or 32, for kMinPartK.
   struct Pair { int mc, nc; std::vector<KSeg> segs; int64_t klen, cutlen; };
   std::vector<Pair> cpairs;
   for (int a = 0; a < nMC; ++a)
@@ -655,7 +657,7 @@ static SectorPlanPtr build_plan(const LOperand& C, const LOperand& A, const LOpe
           sector_tasks(split, make_geoms(make_parts(max_parts), 0, true)) <= kFewTasks;
     if (few)
       for (size_t i = 0; i < cpairs.size(); ++i)
-        max_parts[i] = std::max(max_parts[i], std::min<int64_t>(kMaxParts, cpairs[i].cutlen / kMinPartKFew));
+        max_parts[i] = std::max(max_parts[i], std::min<int64_t>(kMaxParts, cpairs[i].klen / kMinPartKFew));
   }
   auto estimate = [&](const std::vector<int64_t>& np) {
     Parts E = make_parts(np);
