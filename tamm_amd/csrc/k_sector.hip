@@ -1918,7 +1918,7 @@ static bool runs_in_place(const SectorPlan& sp, const double* A) {
   return sp.inplace && !sp.A.constant && reinterpret_cast<uintptr_t>(A) % 16 == 0;
 }
 static const std::vector<ShapeTasks>& launches_for(const SectorPlan& sp, const double* A) {
-  return sp.inplace && !runs_in_place(sp, A) ? sp.packed_shapes : sp.shapes;
+  return sp.packed_shapes.empty() || runs_in_place(sp, A) ? sp.shapes : sp.packed_shapes;
 }
 
 void sector_schedule_info(const SectorPlan& sp, int* rounds, int* launches, int64_t* tasks, const double* A) {
@@ -2190,6 +2190,8 @@ int autotune_sector_plan(SectorPlan& sp, const double* A, hipStream_t s) {
     }
   }
   double flops = 0;
+  if (sp.inplace && sp.packed_shapes.empty())  // shared so far
+    (second ? sp.shapes : sp.packed_shapes) = build_sector_tasks(sp.split, sp.nmod, second ? sp.geoms : sp.packed_geoms);
   (second ? sp.packed_shapes : sp.shapes) = build_sector_tasks(sp.split, sp.nmod, geoms, &flops);
   if (!second) sp.exec_flops = flops;
   {

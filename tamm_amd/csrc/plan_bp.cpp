@@ -768,8 +768,13 @@ static int build_sector(tmx_contraction_s& c, const LabelInfo& li, const std::ve
   ab.insert(ab.end(), li.bouter.begin(), li.bouter.end());
   ba.insert(ba.end(), li.aouter.begin(), li.aouter.end());
   c.swapped = c.C.labels != ab && c.C.labels == ba;
-  c.li = c.swapped ? analyse_labels(c.C, c.B, c.A) : li;
-  c.work = c.swapped ? enumerate_pairs(c.C, c.B, c.A, c.li) : work;
+  if (c.swapped) {
+    c.li = analyse_labels(c.C, c.B, c.A);
+    c.work = enumerate_pairs(c.C, c.B, c.A, c.li);
+  } else {
+    c.li = li;
+    c.work = work;
+  }
   // AUTO_SPLIT: split precision pays only where the FP64 GEMM is MFMA-bound.  A sector GEMM
   // reads (mrows + nrows) K operand elements for 2 mrows nrows K flops; below
   // kMinSplitMN (flops-weighted mrows nrows / (mrows + nrows) of the sectors, e.g. the one-O-

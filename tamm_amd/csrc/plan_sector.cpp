@@ -963,7 +963,10 @@ static SectorPlanPtr build_plan(const LOperand& C, const LOperand& A, const LOpe
     sp->cdense = DevBuf(sizeof(double) * (size_t)cbase);
   }
   sp->shapes = build_sector_tasks(split, sp->nmod, sp->geoms, &sp->exec_flops);
-  if (sp->inplace) sp->packed_shapes = build_sector_tasks(split, sp->nmod, sp->packed_geoms);
+  bool differ = false;
+  for (size_t i = 0; i < sp->geoms.size() && sp->inplace; ++i)
+    differ = differ || sp->geoms[i].tm != sp->packed_geoms[i].tm || sp->geoms[i].tn != sp->packed_geoms[i].tn;
+  if (differ) sp->packed_shapes = build_sector_tasks(split, sp->nmod, sp->packed_geoms);
   // Padding (rows beyond a class's rows, columns beyond a block's columns) must read as zero;
   // pack kernels only ever write real elements, so clear once here.
   hipStream_t s = runtime().stream;

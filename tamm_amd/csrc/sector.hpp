@@ -133,7 +133,8 @@ struct SectorPlan {
   DevBuf ksegs;
   // A is read in place (inplace_args) by the launches of `shapes`, which all have such kernels; an
   // execution that packs it all the same (constant, or at an address without 16-byte alignment)
-  // takes packed_shapes, of packed_geoms.  Else `shapes` are the only ones.
+  // takes packed_shapes, of packed_geoms, unless that list is empty (the same tiles, or no plan in
+  // place at all).
   bool inplace = false;
   std::vector<SectorGeom> packed_geoms;
   std::vector<ShapeTasks> packed_shapes;
