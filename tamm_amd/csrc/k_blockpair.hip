@@ -445,14 +445,15 @@ void launch_bp_f64(const BPTask* tasks, int ntasks, const BPPair* pairs, const B
 // ---------------------------------------------------------------------------
 // Block assign / transpose-accumulate: HBM-bound (16 B per element, 24 when accumulating).
 //
-// A workgroup iteration takes one box of a (dst block, src block) pair (AssignShape).  The
+// A workgroup iteration of k_assign takes one box of a (dst block, src block) pair (AssignShape; blocks
+// that fill whole tiles take k_assign_tile below).  The
 // offsets of the box's X, Y and Z indices go to LDS tables once; elements are read with X
 // fastest, then Y, then Z (the source's contiguous mode along the lanes), pass through an LDS
 // tile and are written with Y fastest, then X, then Z.  Without X modes both orders are the same
 // and the tile is skipped.  Each thread has its PER source loads and, accumulating, its PER
 // destination loads in flight together: 1, 4 or 9 for boxes of 256, 1024 or 2304 elements.  Boxes
-// span as many modes as it takes to hold that many: with one workgroup per 32x32 tile or per run of the contiguous mode, amplitude blocks
-// of 48x48x16x16 gave each workgroup 256 or 16 elements: over 3.5e7 elements, R(a,b,i,j) -=
+// span as many modes as it takes to hold that many: in whole tiles or runs of the contiguous mode,
+// amplitude blocks of 48x48x16x16 gave each workgroup 256 or 16 elements: over 3.5e7 elements, R(a,b,i,j) -=
 // T(b,a,i,j) went from 9.49 to 0.17 ms (5.0 TB/s) and R(a,b,i,j) -= T(a,b,j,i) from 0.93 to 0.17.
 struct AssignTable {
   int s, d;

@@ -1477,11 +1477,13 @@ __global__ __launch_bounds__(256) void k_scatter(const ScatterJob* __restrict__ 
 // GEMM tile shapes and their relative MFMA efficiency (int8: measured on MI355X with the
 // ladder and square shapes; wider tiles need fewer LDS and L2 bytes per MFMA).
 // small > 0: offered only to sectors with at most `small` rows on one side.  64x64 serves
-// products with few rows or columns over a long K (e.g. Fo(k,i) = U(k,l,c,d) T(c,d,i,l) with
+// products with few rows and columns over a long K (e.g. Fo(k,i) = U(k,l,c,d) T(c,d,i,l) with
 // 60x60 outputs), where larger tiles would stream padding rows of A or B; on large sectors it
 // can time faster alone yet slow the plan down as a launch of its own.  FP64 32x32 serves
 // classes of one O tile (16 padded rows, e.g. that product's 8 x 8 sectors), which a 64-row
-// tile would load four times over.
+// tile would load four times over.  FP64 sectors of few columns and many rows have the least
+// padded area over eff in 256x80, which reads A in place: of 9 to 64 columns by 900 to 6400 rows
+// 0.45 times as long as packed and in the narrow tiles; with A packed, TileRule::narrow.
 // eff: MFMA efficiency for comparing shapes on one sector by padded area.  rate, fixed and
 // slots describe the shape in the launch model: multiply-adds per second of the full chip
 // (10^15 int8, 3.4 x 10^13 FP64), time per task outside its stages (pipeline fill and epilogue)
@@ -1856,7 +1858,7 @@ double estimate_sector_seconds(bool split, int nmod, const std::vector<SectorGeo
 
 // Sectors of different shapes are launches of their own, each with a last partial round and the
 // small sectors' launch too short to fill the chip; the launch model therefore also tries every
-// shape for all sectors at once (thin ones keep the narrow shapes made for them).  Ladder, ring
+// shape for all sectors at once (those that took 64x64 or 32x32 keep it).  Ladder, ring
 // and hole-hole GEMMs of O = 30, V = 180 in split precision: 1774 -> 1543, 351 -> 292 and 128 ->
 // 97 us; FP64 ring 1155 -> 820.
 void choose_shapes(bool split, int nmod, std::vector<SectorGeom>& geoms, bool trial, TileRule rule) {
