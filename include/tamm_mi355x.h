@@ -179,7 +179,8 @@ int tmx_contraction_autotune(tmx_contraction c, const double* A, const double* B
  * Refused (TMX_ERR_STATE) while a captured graph holds the contraction; a graph captured after
  * the packing replays without it.  Block-pair plans read operands in place and ignore the
  * flags, except that a small product which AUTO or AUTO_SPLIT had put on the grouped path moves to
- * the sector path here, for good, where packing the constant operands once makes that faster
+ * the sector path here, for good, where packing the constant operands once makes that faster and
+ * no graph capture is in progress
  * (tmx_contraction_info then reports the new mode and workspace).  No counterpart in TAMM, which
  * re-reads every block at every execution. */
 int tmx_contraction_set_constant(tmx_contraction c, int a_constant, int b_constant);

@@ -790,11 +790,12 @@ static int build_sector(tmx_contraction_s& c, const LabelInfo& li, const std::ve
 // A small product that AUTO put on the grouped path, once operands of it are constant: the sector
 // path then packs them once, and takes the product over unless grouped is modelled 1.25 times as
 // fast (ladder of 10 + 100 orbitals with constant V: 212 us grouped, 122 split; of 24 + 96 in tiles
-// of 2 to 6: 587 and 206 in FP64; rings of 10 + 100 stay at 20, split 37).  For good: a level may have given the plan's product to other terms.
+// of 2 to 6: 587 and 206 in FP64; rings of 10 + 100 stay at 20, split 37).  For good: a level may have given the plan's product to
+// other terms.  Not during a capture, whose executions stay grouped; the next call decides again.
 static void reconsider_small(tmx_contraction_s& c) {
   if (c.small.grouped_us == 0 || c.sec || !(c.const_a || c.const_b)) return;
   const double us = c.small.sector_us - (c.const_a ? c.small.pack_us[0] : 0) - (c.const_b ? c.small.pack_us[1] : 0);
-  if (1.25 * c.small.grouped_us < us || stream_capturing(runtime().stream)) return;
+  if (1.25 * c.small.grouped_us < us || capture_in_progress()) return;
   const bool split = c.small.exec_mode == TMX_EXEC_AUTO_SPLIT;
   const LabelInfo li = analyse_labels(c.C, c.A, c.B);
   try {

@@ -54,6 +54,12 @@ struct GraphObj {
 };
 }  // namespace
 
+bool capture_in_progress() {
+  if (stream_capturing(g_rt.stream)) return true;
+  std::lock_guard<std::mutex> g(capture_mu());
+  return !captures().empty();
+}
+
 void capture_hold(hipStream_t s, std::shared_ptr<void> obj) {
   if (!obj || !stream_capturing(s)) return;
   std::lock_guard<std::mutex> g(capture_mu());

@@ -72,6 +72,9 @@ void* pool_alloc(size_t bytes);
 void pool_free(void* p);
 // True while `s` is being captured into a graph.
 bool stream_capturing(hipStream_t s);
+// True while the engine stream, or any stream through tmx_graph_begin, is being captured: building a
+// plan allocates, copies and synchronises, which a capture on any stream of the thread does not survive.
+bool capture_in_progress();
 // Graph lifetime.  While a stream is captured through tmx_graph_begin / tmx_graph_end, every
 // plan object executed into it is recorded with that capture (capture_hold, a no-op when `s`
 // is not captured that way), and the graph made from the capture keeps a reference to each

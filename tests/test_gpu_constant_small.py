@@ -1,5 +1,7 @@
 """Small products that AUTO takes off the sector path: marking an operand constant moves them there
 where the kept packed copy makes it faster, with the same results; a tiny one stays."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -48,6 +50,36 @@ def test_constant_operand_moves_small_product(eng, mode):
     c.set_constant(False, False)
     got = _run(ew, c)
     assert np.linalg.norm(got - ref) <= TOL[mode] * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("mode", sorted(TOL))
+def test_no_move_during_a_capture(eng, mode):
+    # building a plan copies and synchronises, which another stream's capture may not survive
+    hip = eng.lib()  # its runtime
+    stream = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+    ew = _workload(eng, 10, 100, 5, 25)
+    C = ew.tensors["R"]
+    ref = _run(ew, ew.contraction(configs.LADDER, eng.EXEC_GROUPED_F64))
+    c = ew.contraction(configs.LADDER, getattr(eng, mode))
+
+    def record():
+        c.set_constant(True, False)
+        assert c.mode == eng.EXEC_GROUPED_F64
+        c.execute(stream=stream.value)
+
+    g = eng.Graph(record, stream=stream.value)
+    for rep in range(3):
+        C.fill(1.0)
+        eng.synchronize()
+        g.launch()
+        assert hip.hipStreamSynchronize(stream) == 0
+        assert np.array_equal(C.download(), ref)
+    del g
+    assert hip.hipStreamDestroy(stream) == 0
+    c.set_constant(True, False)
+    assert c.mode == (eng.EXEC_SECTOR_F64 if mode == "EXEC_AUTO" else eng.EXEC_SPLIT_I8)
+    assert np.linalg.norm(_run(ew, c) - ref) <= TOL[mode] * np.linalg.norm(ref)
 
 
 @pytest.mark.parametrize("mode", sorted(TOL))
